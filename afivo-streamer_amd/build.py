@@ -72,7 +72,7 @@ def build_ref():
     drivers that call them (oracle/ref/Makefile, outputs in oracle/_ref),
     where the reference checkout and amdflang are present; the tests that
     use them are skipped elsewhere."""
-    if not (os.path.isdir(REFERENCE) and os.path.exists(FLANG)):
+    if not (os.path.isdir(os.path.join(REFERENCE, "afivo", "src")) and os.path.exists(FLANG)):
         print("reference checkout or amdflang not present: oracle/_ref not built", flush=True)
         return None
     _run(["make", "-C", os.path.join(REPO_DIR, "oracle", "ref"), "REF=" + REFERENCE, "all"])
