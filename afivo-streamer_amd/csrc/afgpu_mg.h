@@ -183,24 +183,11 @@ __device__ inline CoarseVals<T> ghost_coarse_load(const DBox &bx, const T *var, 
   }
   return cv;
 }
-template <int D, int NC, typename T>
-__device__ inline GhostPart<T> ghost_coarse_form(const DBox &bx, const VarBc &m, int nb, int a, int b,
-                                                 const CoarseVals<T> &cv) {
-  const int d = nb / 2;
-  const bool low = (nb % 2) == 0;
+// The part of a refinement-boundary ghost formed from the coarse values.
+template <int D, typename T>
+__device__ inline GhostPart<T> coarse_part(const VarBc &m, int d, int a, int b, const CoarseVals<T> &cv) {
   GhostPart<T> g;
   g.c1 = T(0);
-  if (bx.nb[nb] < 0) {
-    T c0;
-    if (m.type[nb] == BC_DIRICHLET)
-      c0 = 2;
-    else if (m.type[nb] == BC_NEUMANN)
-      c0 = (T)bx.dr[d] * T(low ? -1 : 1);
-    else
-      c0 = 1;
-    g.p = c0 * (T)bc_value(m, nb, bx.run);
-    return g;
-  }
   if (m.rb == RB_MG) {
     if (D == 2) {
       const T grad = T(0.125) * (cv.v[0] - cv.v[1]);
@@ -225,6 +212,34 @@ __device__ inline GhostPart<T> ghost_coarse_form(const DBox &bx, const VarBc &m,
   g.c1 = cv.v[0];
   return g;
 }
+// ... and the terms of the box's cells x1, x2.
+template <typename T>
+__device__ inline T rb_finish(const VarBc &m, const GhostPart<T> &g, T x1, T x2) {
+  if (m.rb == RB_MG) return T(0.5) * g.p + T(0.75) * x1 - T(0.25) * x2;
+  T v = g.p + T(1 / 3.0) * x1;
+  if (m.rb == RB_INTERP_LIM && v > 2 * g.c1) v = 2 * g.c1;
+  return v;
+}
+template <int D, int NC, typename T>
+__device__ inline GhostPart<T> ghost_coarse_form(const DBox &bx, const VarBc &m, int nb, int a, int b,
+                                                 const CoarseVals<T> &cv) {
+  const int d = nb / 2;
+  const bool low = (nb % 2) == 0;
+  GhostPart<T> g;
+  g.c1 = T(0);
+  if (bx.nb[nb] < 0) {
+    T c0;
+    if (m.type[nb] == BC_DIRICHLET)
+      c0 = 2;
+    else if (m.type[nb] == BC_NEUMANN)
+      c0 = (T)bx.dr[d] * T(low ? -1 : 1);
+    else
+      c0 = 1;
+    g.p = c0 * (T)bc_value(m, nb, bx.run);
+    return g;
+  }
+  return coarse_part<D, T>(m, d, a, b, cv);
+}
 template <int D, int NC, typename T>
 __device__ inline GhostPart<T> ghost_coarse(const DBox &bx, const T *var, const VarBc &m, int nb, int a, int b,
                                             const T *coarse = nullptr) {
@@ -244,10 +259,7 @@ __device__ inline T ghost_finish(const DBox &bx, const VarBc &m, int nb, const G
     }
     return g.p + c1 * x1 + c2 * x2;
   }
-  if (m.rb == RB_MG) return T(0.5) * g.p + T(0.75) * x1 - T(0.25) * x2;
-  T v = g.p + T(1 / 3.0) * x1;
-  if (m.rb == RB_INTERP_LIM && v > 2 * g.c1) v = 2 * g.c1;
-  return v;
+  return rb_finish<T>(m, g, x1, x2);
 }
 
 template <int D, int NC, typename T>
@@ -994,137 +1006,259 @@ __device__ inline void lds_load_interior(T *s, const T *u) {
   }
 }
 
-// Staging of a box and its face ghosts into LDS in two memory rounds: the
-// interior and the same-level neighbour copies are loaded together (into
-// registers, then LDS); after a barrier, the ghosts that depend on the box's
-// own cells (physical boundary, refinement boundary) are formed from LDS.
-// colour >= 0: only the ghosts next to interior cells of that GSRB colour,
-// and in the colour-split FP32 layout only the interior cells of the other
-// colour, the only ones a half-sweep of that colour reads (the few cells of
-// the updated colour that those ghosts depend on are read from the pool).
+// v[n] for a small n that differs between lanes, without indexed registers
+// or a load per lane (v: kernel arguments, a box record's uniform fields).
+// (The values are selected, not their addresses: a selected address keeps
+// the whole array in scratch memory.)
+template <int N, typename V>
+__device__ inline V pick(const V *v, int n) {
+  if constexpr (N == 1) {
+    return V(v[0]);
+  } else {
+    const V lower = pick<N - 1>(v, n), last = V(v[N - 1]);
+    return (n == N - 1) ? V(last) : V(lower);
+  }
+}
+// Cell (i, j, k) at normal index pn and tangential (a, b) of face nb, for an
+// nb that may differ between lanes.
+template <int D>
+__device__ inline void face_cell(int nb, int a, int b, int pn, int &i, int &j, int &k) {
+  const int d = nb >> 1;
+  i = (d == 0) ? pn : a;
+  j = (d == 1) ? pn : (D == 2 || d == 0) ? a : b;
+  k = (D == 2) ? 0 : (d == 2) ? pn : b;
+}
+// The coarse cells the ghosts of a face at a refinement boundary are formed
+// from: the face layer of the coarse neighbour over the box's extent and one
+// cell around it.  Patch cell pa (+ PP pb) holds the coarse cell at
+// tangential (co[t0] + pa, co[t1] + pb), co the box's offset within its
+// parent.
+template <int D, int NC>
+struct CoarsePatch {
+  static constexpr int PP = NC / 2 + 2;
+  static constexpr int N = (D == 3) ? PP * PP : PP;
+};
+// The coarse values ghost_coarse_load reads for ghost (a, b)
+// (mg_sides_rb, afivo/src/m_af_multigrid.f90:294-461; af_gc_interp(_lim),
+// afivo/src/m_af_ghostcell.f90:394-605), in its order, from the patch.
+template <int D, int NC, typename T>
+__device__ inline CoarseVals<T> coarse_patch_vals(const T *cp, const VarBc &m, int a, int b) {
+  constexpr int PP = CoarsePatch<D, NC>::PP;
+  auto at = [&](int qa, int qb) { return cp[D == 3 ? qa + PP * qb : qa]; };
+  CoarseVals<T> cv = {{T(0), T(0), T(0), T(0), T(0)}};
+  if (m.rb == RB_MG) {
+    const int i = (a + 1) >> 1, j = (b + 1) >> 1;
+    cv.v[0] = at(i + 1, j);
+    cv.v[1] = at(i - 1, j);
+    if (D == 2) {
+      cv.v[2] = at(i, j);
+    } else {
+      cv.v[2] = at(i, j + 1);
+      cv.v[3] = at(i, j - 1);
+      cv.v[4] = at(i, j);
+    }
+    return cv;
+  }
+  const int a1 = (a + 1) >> 1, a2 = a1 + 1 - 2 * (a & 1);
+  const int b1 = (b + 1) >> 1, b2 = b1 + 1 - 2 * (b & 1);
+  cv.v[0] = at(a1, b1);
+  cv.v[1] = at(a2, b1);
+  if (D == 3) cv.v[2] = at(a1, b2);
+  return cv;
+}
+// Ghost (a, b) of a face without a same-level neighbour (nbv <= 0) from the
+// box's first and second cells x1, x2 and, at a refinement boundary, the
+// face's coarse patch cp: ghost_value's operations, for an nb that may
+// differ between lanes.  run_val: the run's value of face m.run_face.
+template <int D, int NC, typename T>
+__device__ inline T staged_ghost(const DBox &bx, const VarBc &m, double run_val, int nbv, int nb, int a, int b,
+                                 const T *cp, T x1, T x2) {
+  if (nbv < 0) {
+    const int type = pick<2 * D>(m.type, nb);
+    const double bv = (m.run_val && nb == m.run_face) ? run_val : pick<2 * D>(m.val, nb);
+    T c0, c1;
+    if (type == BC_DIRICHLET) {
+      c0 = 2;
+      c1 = -1;
+    } else if (type == BC_NEUMANN) {
+      c0 = (T)pick<D>(bx.dr, nb >> 1) * T((nb & 1) ? 1 : -1);
+      c1 = 1;
+    } else {
+      c0 = 1;
+      c1 = 0;
+    }
+    return c0 * (T)bv + c1 * x1 + T(0) * x2;
+  }
+  const CoarseVals<T> cv = coarse_patch_vals<D, NC, T>(cp, m, a, b);
+  const GhostPart<T> g = coarse_part<D, T>(m, nb >> 1, a, b, cv);
+  return rb_finish<T>(m, g, x1, x2);
+}
+
+// Staging of a box and its face ghosts into LDS in one memory round.  The
+// box record's fields are uniform; every lane issues its loads without
+// branches (the interior, and per face ghost one value: the same-level
+// neighbour's cell across the face, which is the ghost, or the box's own
+// first cell; then, in boxes at a refinement boundary, the coarse patches of
+// the faces there), so all of them are in flight together.  After a barrier
+// the ghosts of the faces without a neighbour are formed from LDS.  What
+// bounds it is that chain, record -> cells -> LDS, not the bytes, on all but
+// the largest levels.  A form with a branch per ghost and indexed face
+// fields waited for its loads branch by branch and kept the boundary methods
+// in scratch memory: per launch, the half-sweep of a refined mesh of 8^2
+// FP64 boxes then took 10.1 us (now 3.2), of 4000 8^3 FP32 boxes 21.7 us
+// (8.2), of 16^3 FP64 boxes 16.8 us (13.8); the FP64 residual of 1024 8^2
+// boxes 17.5 us (3.9), of 1856 16^3 boxes 45.1 us (41.6).
+// COL: only the ghosts next to interior cells of GSRB colour `colour`, and
+// in the colour-split FP32 layout only the interior cells of the other
+// colour, the only ones a half-sweep of that colour reads.
 // stored: the face ghosts are the box's own stored ghost layer (the
 // reference's smoother reads that layer as it stands before its first
 // half-sweep; FP64 layout only).
-// Ends with a barrier.
-template <int D, int NC, int BS, typename T, int BB = 1>
-__device__ inline void lds_stage(T *s, const DBox *__restrict__ boxes, const DBox &bx, int id, const T *var,
-                                 const VarBc &m, int colour, const T *coarse = nullptr, bool stored = false) {
+// issue() makes the loads, commit() the LDS copy s (afivo's order), with cp
+// (2 D CoarsePatch::N values) as scratch, and ends with a barrier; between
+// the two a kernel can do work that needs neither.
+template <int D, int NC, int BS, typename T, int BB, bool COL>
+struct Stage {
   using G = Geo<D, NC>;
   using L = Lay<D, NC, T>;
-  stored = stored && !L::SPLIT;
-  constexpr int NI = (G::NINT + BS - 1) / BS;
-  constexpr int NFC = 2 * D * G::NTAN;
-  constexpr int NF = (NFC + BS - 1) / BS;
-  const T *u = var + (size_t)(id - 1) * L::STRIDE;
-  const bool one = L::SPLIT && colour >= 0;
-  const int n_load = one ? G::NINT / 2 : G::NINT;
+  using P = CoarsePatch<D, NC>;
+  static constexpr bool ONE = L::SPLIT && COL;
+  static constexpr int NL = ONE ? G::NINT / 2 : G::NINT;  // interior cells loaded
+  static constexpr int NI = (NL + BS - 1) / BS;
+  static constexpr int NE = COL ? G::NTAN / 2 : G::NTAN;  // ghosts of a face
+  static constexpr int NGH = 2 * D * NE, NF = (NGH + BS - 1) / BS;
+  static constexpr int NPT = 2 * D * P::N, NP = (NPT + BS - 1) / BS;
+  T vi[NI], vf[NF], vp[NP];
+  int nbid[2 * D];
+  int colour;
+  bool any_rb, any_b, stored;
+  double run_val;
+
   // interior cell (i, j, k) of load q and its position in the pool: in the
   // split layout the loads run over the colour blocks in order
-  auto cell = [&](int q, int &i, int &j, int &k) {
+  __device__ int cell(int q, int &i, int &j, int &k) const {
     if constexpr (L::SPLIT) {
       constexpr int HALF = G::NINT / 2;
-      const int x = q + (one ? (1 - colour) * HALF : 0);
+      const int x = q + (ONE ? (1 - colour) * HALF : 0);
       colour_cell<D, NC>(x >= HALF, x >= HALF ? x - HALF : x, i, j, k);
       return x;
     } else {
       interior_ijk<D, NC>(q, i, j, k);
       return L::in_at(i, j, k);
     }
-  };
-  // with a colour, the physical and refinement-boundary ghosts' parts that
-  // do not depend on the box (the coarse values) are loaded in the first
-  // round too, and so are the updated colour's cells they need in the split
-  // layout: the second round then works in LDS only
-  const bool pre = colour >= 0;
-  T vi[NI], vf[NF], x1g[NF];
-  GhostPart<T> gp[NF];
-  int gi[NF];
-  for (int t = 0; t < NI; t++) {
-    const int q = ltid<BS>() + t * BS;
-    if (q < n_load) {
+  }
+  // ghost item q: its face and tangential position (COL: next to a cell
+  // with (i + j + k + colour) even)
+  __device__ void item(int q, int &nb, int &a, int &b) const {
+    nb = q / NE;
+    const int e = q % NE;
+    if constexpr (COL) {
+      const int pd = (nb & 1) ? NC : 1;
+      b = (D == 3) ? e / (NC / 2) + 1 : 0;
+      a = 2 * (e % (NC / 2)) + 1 + ((colour + pd + b + 1) & 1);
+    } else {
+      a = e % NC + 1;
+      b = (D == 3) ? e / NC + 1 : 0;
+    }
+  }
+
+  __device__ void issue(const DBox &bx, int id, const T *var, const VarBc &m, int colour_, const T *coarse = nullptr,
+                        bool stored_ = false) {
+    colour = colour_;
+    stored = stored_ && !L::SPLIT;
+    any_rb = any_b = false;
+#pragma unroll
+    for (int nb = 0; nb < 2 * D; nb++) {
+      nbid[nb] = __builtin_amdgcn_readfirstlane(bx.nb[nb]);
+      any_b = any_b || nbid[nb] <= 0;
+      any_rb = any_rb || nbid[nb] == 0;
+    }
+    any_b = any_b && !stored;
+    any_rb = any_rb && !stored;
+    const T *u = var + (size_t)(id - 1) * L::STRIDE;
+#pragma unroll
+    for (int t = 0; t < NI; t++) {
+      int q = ltid<BS>() + t * BS;
+      if (NL % BS) q = min(q, NL - 1);
       int i, j, k;
       vi[t] = u[cell(q, i, j, k)];
     }
-  }
-  for (int t = 0; t < NF; t++) {
-    gi[t] = -1;
-    const int q = ltid<BS>() + t * BS;
-    if (q >= NFC) continue;
-    const int nb = q / G::NTAN, r = q % G::NTAN;
-    const int nb_id = bx.nb[nb];
-    if (nb_id <= 0 && !pre && !stored) continue;
-    const int a = r % NC + 1, b = (D == 3) ? r / NC + 1 : 0;
-    const bool low = (nb % 2) == 0;
-    int p[3];
-    face_pos<D>(nb, a, b, low ? 1 : NC, p);
-    if (colour >= 0 && ((p[0] + p[1] + p[2] + colour) & 1)) continue;
-    if (stored) {
-      p[nb / 2] = low ? 0 : NC + 1;
-      gi[t] = G::idx(p[0], p[1], p[2]);
-      vf[t] = u[L::at(p[0], p[1], p[2])];
-      continue;
+#pragma unroll
+    for (int t = 0; t < NF; t++) {
+      int q = ltid<BS>() + t * BS;
+      if (NGH % BS) q = min(q, NGH - 1);
+      int nb, a, b, i, j, k;
+      item(q, nb, a, b);
+      const int nbv = pick<2 * D>(nbid, nb);
+      const bool low = (nb & 1) == 0, copy = nbv > 0 && !stored;
+      const int pn = stored ? (low ? 0 : NC + 1) : (copy == low) ? NC : 1;
+      face_cell<D>(nb, a, b, pn, i, j, k);
+      const T *from = var + (size_t)((copy ? nbv : id) - 1) * L::STRIDE;
+      vf[t] = from[L::SPLIT ? L::in_at(i, j, k) : L::at(i, j, k)];
     }
-    if (nb_id <= 0) {
-      gp[t] = ghost_coarse<D, NC, T>(bx, var, m, nb, a, b, coarse);
-      if (one) x1g[t] = u[L::in_at(p[0], p[1], p[2])];
-      continue;
+    if (any_rb) {
+      const T *cvar = coarse ? coarse : var;
+      int co[3];
+#pragma unroll
+      for (int d = 0; d < D; d++) co[d] = ((bx.ix[d] - 1) & 1) * (NC / 2);
+#pragma unroll
+      for (int t = 0; t < NP; t++) {
+        const int q = min(ltid<BS>() + t * BS, NPT - 1);
+        const int nb = q / P::N, e = q % P::N, d = nb >> 1;
+        const bool rb = pick<2 * D>(nbid, nb) == 0;
+        const int c0 = (d == 0) ? co[1] : co[0], c1 = (D == 2) ? 0 : (d == 2) ? co[1] : co[2];
+        int i, j, k;
+        face_cell<D>(nb, c0 + e % P::PP, (D == 3) ? c1 + e / P::PP : 0, (nb & 1) ? 1 : NC, i, j, k);
+        const T *from = rb ? cvar + (size_t)(pick<2 * D>(bx.pnb, nb) - 1) * L::STRIDE + L::at(i, j, k) : u;
+        vp[t] = *from;
+      }
     }
-    int d = nb / 2;
-    p[d] = low ? 0 : NC + 1;
-    gi[t] = G::idx(p[0], p[1], p[2]);
-    p[d] = low ? NC : 1;  // the neighbour's cell across the face
-    vf[t] = var[(size_t)(nb_id - 1) * L::STRIDE + L::in_at(p[0], p[1], p[2])];
+    run_val = (any_b && m.run_val) ? m.run_val[bx.run] : 0.0;
   }
-  for (int t = 0; t < NI; t++) {
-    const int q = ltid<BS>() + t * BS;
-    if (q < n_load) {
+
+  __device__ void commit(T *s, T *cp, const DBox &bx, const VarBc &m) {
+#pragma unroll
+    for (int t = 0; t < NI; t++) {
+      const int q = ltid<BS>() + t * BS;
       int i, j, k;
       cell(q, i, j, k);
-      s[G::idx(i, j, k)] = vi[t];
+      if (NL % BS == 0 || q < NL) s[G::idx(i, j, k)] = vi[t];
     }
-  }
-  for (int t = 0; t < NF; t++)
-    if (gi[t] >= 0) s[gi[t]] = vf[t];
-  gsync<BS, BB>();
-  bool any = false;
-  for (int nb = 0; nb < 2 * D; nb++) any = any || bx.nb[nb] <= 0;
-  if (any && !stored) {
-    if (pre) {
-      for (int t = 0; t < NF; t++) {
+#pragma unroll
+    for (int t = 0; t < NF; t++) {
+      const int q = ltid<BS>() + t * BS;
+      if (NGH % BS && q >= NGH) continue;
+      int nb, a, b, i, j, k;
+      item(q, nb, a, b);
+      face_cell<D>(nb, a, b, (nb & 1) ? NC + 1 : 0, i, j, k);
+      // (the ghosts of the other faces are written again below)
+      s[G::idx(i, j, k)] = vf[t];
+    }
+    if (any_rb) {
+#pragma unroll
+      for (int t = 0; t < NP; t++) {
         const int q = ltid<BS>() + t * BS;
-        if (q >= NFC) continue;
-        const int nb = q / G::NTAN, r = q % G::NTAN;
-        if (bx.nb[nb] > 0) continue;
-        const int a = r % NC + 1, b = (D == 3) ? r / NC + 1 : 0;
-        const bool low = (nb % 2) == 0;
-        int p[3];
-        face_pos<D>(nb, a, b, low ? 1 : NC, p);
-        if ((p[0] + p[1] + p[2] + colour) & 1) continue;
-        const T x1 = one ? x1g[t] : s[G::idx(p[0], p[1], p[2])];
-        face_pos<D>(nb, a, b, low ? 2 : NC - 1, p);
-        const T x2 = s[G::idx(p[0], p[1], p[2])];
-        face_pos<D>(nb, a, b, low ? 0 : NC + 1, p);
-        s[G::idx(p[0], p[1], p[2])] = ghost_finish<D, NC, T>(bx, m, nb, gp[t], x1, x2);
-      }
-    } else {
-      for (int q = ltid<BS>(); q < NFC; q += BS) {
-        const int nb = q / G::NTAN, r = q % G::NTAN;
-        if (bx.nb[nb] > 0) continue;
-        const int a = r % NC + 1, b = (D == 3) ? r / NC + 1 : 0;
-        const bool low = (nb % 2) == 0;
-        int p[3];
-        face_pos<D>(nb, a, b, low ? 1 : NC, p);
-        const T x1 = s[G::idx(p[0], p[1], p[2])];
-        face_pos<D>(nb, a, b, low ? 2 : NC - 1, p);
-        const T x2 = s[G::idx(p[0], p[1], p[2])];
-        const T g = ghost_value<D, NC, T>(boxes, bx, var, m, nb, a, b, x1, x2, coarse);
-        face_pos<D>(nb, a, b, low ? 0 : NC + 1, p);
-        s[G::idx(p[0], p[1], p[2])] = g;
+        if (q < NPT) cp[q] = vp[t];
       }
     }
     gsync<BS, BB>();
+    if (!any_b) return;
+#pragma unroll
+    for (int t = 0; t < NF; t++) {
+      const int q = ltid<BS>() + t * BS;
+      if (NGH % BS && q >= NGH) continue;
+      int nb, a, b, i, j, k;
+      item(q, nb, a, b);
+      const int nbv = pick<2 * D>(nbid, nb);
+      if (nbv > 0) continue;
+      face_cell<D>(nb, a, b, (nb & 1) ? NC - 1 : 2, i, j, k);
+      const T x2 = s[G::idx(i, j, k)];
+      face_cell<D>(nb, a, b, (nb & 1) ? NC + 1 : 0, i, j, k);
+      s[G::idx(i, j, k)] = staged_ghost<D, NC, T>(bx, m, run_val, nbv, nb, a, b, cp + nb * P::N, vf[t], x2);
+    }
+    gsync<BS, BB>();
   }
-}
+};
 
 // k_gsrb with the box staged in LDS (levels with one workgroup per box).
 template <int D, int NC, int BS, typename T, int BB = 1>
@@ -1134,12 +1268,12 @@ __global__ void __launch_bounds__(BS * BB) k_gsrb_lds(const int *__restrict__ id
   using G = Geo<D, NC>;
   using L = Lay<D, NC, T>;
   __shared__ T s_all[BB][G::NCELL];
-  T *s = s_all[lgrp<BS, BB>()];
+  __shared__ T cp_all[BB][2 * D * CoarsePatch<D, NC>::N];
+  T *s = s_all[lgrp<BS, BB>()], *cp = cp_all[lgrp<BS, BB>()];
   for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
-    const int id = ids[w];
+    const int id = __builtin_amdgcn_readfirstlane(ids[w]);
     if (id <= 0) continue;  // run masked out
     const DBox &bx = boxes[id - 1];
-    const Sten<D, T> st = lpl_stencil<D, T>(bx, lambda2);
     T *u = phi + (size_t)(id - 1) * L::STRIDE;
     const T *r = rhs + (size_t)(id - 1) * L::STRIDE;
     constexpr int HALF = G::NINT / 2;
@@ -1163,7 +1297,10 @@ __global__ void __launch_bounds__(BS * BB) k_gsrb_lds(const int *__restrict__ id
       }
     }
     // the updated cells satisfy (i + j + k + redblack) even
-    lds_stage<D, NC, BS, T, BB>(s, boxes, bx, id, phi, m, redblack & 1, nullptr, stored != 0);
+    Stage<D, NC, BS, T, BB, true> sg;
+    sg.issue(bx, id, phi, m, redblack & 1, nullptr, stored != 0);
+    const Sten<D, T> st = lpl_stencil<D, T>(bx, lambda2);
+    sg.commit(s, cp, bx, m);
     for (int t = 0; t < NH; t++) {
       const int q = ltid<BS>() + t * BS;
       if (q >= HALF) break;
@@ -1211,34 +1348,6 @@ __global__ void __launch_bounds__(BS * BB) k_gsrb_lds(const int *__restrict__ id
     }
     gsync<BS, BB>();  // (the group's LDS is reused by its next item)
   }
-}
-
-// The coarse values ghost_coarse_load reads for ghost (a, b) of a 3D face at
-// a refinement boundary (mg_sides_rb, afivo/src/m_af_multigrid.f90:294-461;
-// af_gc_interp(_lim), afivo/src/m_af_ghostcell.f90:394-605), in its order,
-// from a PP x PP patch of the coarse neighbour's face layer: patch cell
-// pa + PP pb holds the coarse cell at tangential (co[t0] + pa, co[t1] + pb),
-// co the box's offset within its parent.
-template <int NC>
-__device__ inline CoarseVals<float> coarse_patch_vals(const float *cp, const VarBc &m, int a, int b) {
-  constexpr int PP = NC / 2 + 2;
-  auto at = [&](int qa, int qb) { return cp[qa + PP * qb]; };
-  CoarseVals<float> cv = {{0.0f, 0.0f, 0.0f, 0.0f, 0.0f}};
-  if (m.rb == RB_MG) {
-    const int i = (a + 1) >> 1, j = (b + 1) >> 1;
-    cv.v[0] = at(i + 1, j);
-    cv.v[1] = at(i - 1, j);
-    cv.v[2] = at(i, j + 1);
-    cv.v[3] = at(i, j - 1);
-    cv.v[4] = at(i, j);
-    return cv;
-  }
-  const int a1 = (a + 1) >> 1, a2 = a1 + 1 - 2 * (a & 1);
-  const int b1 = (b + 1) >> 1, b2 = b1 + 1 - 2 * (b & 1);
-  cv.v[0] = at(a1, b1);
-  cv.v[1] = at(a2, b1);
-  cv.v[2] = at(a1, b2);
-  return cv;
 }
 
 // k_gsrb_lds for 3D boxes in the colour-split single-precision layout.  A
@@ -1353,7 +1462,7 @@ __global__ void __launch_bounds__(NT) k_gsrb_split(const int *__restrict__ ids, 
       face_pos<D>(nb, a, b, low ? 2 : NC - 1, p);
       const float x2 = s_other[L::in_at(p[0], p[1], p[2]) - oc * HALF];
       CoarseVals<float> cv = {{0.0f, 0.0f, 0.0f, 0.0f, 0.0f}};
-      if (nbv == 0) cv = coarse_patch_vals<NC>(s_cp[nb], m, a, b);
+      if (nbv == 0) cv = coarse_patch_vals<D, NC, float>(s_cp[nb], m, a, b);
       s_gh[nb][e] =
           ghost_finish<D, NC, float>(bx, m, nb, ghost_coarse_form<D, NC, float>(bx, m, nb, a, b, cv), s_x1[nb][e], x2);
     }
@@ -1588,13 +1697,13 @@ __global__ void __launch_bounds__(BS * BB) k_mp_residual_lds(const int *__restri
                                                              int cyl, VarBc m, unsigned long long *leafmax, int nw) {
   using G = Geo<D, NC>;
   __shared__ double s_all[BB][G::NCELL];
-  double *s = s_all[lgrp<BS, BB>()];
+  __shared__ double cp_all[BB][2 * D * CoarsePatch<D, NC>::N];
+  double *s = s_all[lgrp<BS, BB>()], *cp = cp_all[lgrp<BS, BB>()];
   __shared__ double sh[BS / 64];
   for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
-    const int id = ids[w];
+    const int id = __builtin_amdgcn_readfirstlane(ids[w]);
     if (id <= 0) continue;  // run masked out
     const DBox &bx = boxes[id - 1];
-    const Sten<D, double> st = lpl_stencil<D, double>(bx, lambda2);
     const size_t base = (size_t)(id - 1) * G::NCELL;
     constexpr int NI = (G::NINT + BS - 1) / BS;
     double rr[NI];
@@ -1606,7 +1715,10 @@ __global__ void __launch_bounds__(BS * BB) k_mp_residual_lds(const int *__restri
         rr[t] = rhs[base + G::idx(i, j, k)];
       }
     }
-    lds_stage<D, NC, BS, double, BB>(s, boxes, bx, id, phi, m, -1);
+    Stage<D, NC, BS, double, BB, false> sg;
+    sg.issue(bx, id, phi, m, 0);
+    const Sten<D, double> st = lpl_stencil<D, double>(bx, lambda2);
+    sg.commit(s, cp, bx, m);
     double mx = 0;
     for (int t = 0; t < NI; t++) {
       const int q = ltid<BS>() + t * BS;
@@ -1638,15 +1750,18 @@ __global__ void __launch_bounds__(BS * BB) k_restrict_residual_lds(const int *__
   constexpr int H = NC / 2;
   constexpr int NQ = (D == 3) ? H * H * H : H * H;
   __shared__ T s_all[BB][G::NCELL];
-  T *s = s_all[lgrp<BS, BB>()];
+  __shared__ T cp_all[BB][2 * D * CoarsePatch<D, NC>::N];
+  T *s = s_all[lgrp<BS, BB>()], *cp = cp_all[lgrp<BS, BB>()];
   for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
-    const int id = ids[w];
+    const int id = __builtin_amdgcn_readfirstlane(ids[w]);
     if (id <= 0) continue;  // run masked out
     const DBox &bc = boxes[id - 1];
     const DBox &bp = boxes[bc.parent - 1];
-    const Sten<D, T> st = lpl_stencil<D, T>(bc, lambda2);
     const size_t cb = (size_t)(id - 1) * L::STRIDE, pb = (size_t)(bc.parent - 1) * L::STRIDE;
-    lds_stage<D, NC, BS, T, BB>(s, boxes, bc, id, child, m, -1, (const T *)phi);
+    Stage<D, NC, BS, T, BB, false> sg;
+    sg.issue(bc, id, child, m, 0, (const T *)phi);
+    const Sten<D, T> st = lpl_stencil<D, T>(bc, lambda2);
+    sg.commit(s, cp, bc, m);
     int off[3] = {0, 0, 0};
     for (int d = 0; d < D; d++) off[d] = ((bc.ix[d] - 1) & 1) * H;
     for (int q = ltid<BS>(); q < NQ; q += BS) {
@@ -1810,18 +1925,20 @@ __global__ void __launch_bounds__(BS * BB) k_mp_correct_leaves(const int *__rest
   }
 }
 
-// af_gc_box with the box staged in LDS: face ghosts as lds_stage forms them,
+// af_gc_box with the box staged in LDS: face ghosts as Stage forms them,
 // then (with corners) the edge and corner ghosts of gc_edge_cell /
 // gc_corner_cell from the LDS values, then only the ghost layer is written.
 // One workgroup per box.
 template <int D, int NC, int BS, typename T, int BB>
-__device__ inline void gc_lds_box(T *s, const DBox *__restrict__ boxes, int id, T *var, const VarBc &m,
+__device__ inline void gc_lds_box(T *s, T *cp, const DBox *__restrict__ boxes, int id, T *var, const VarBc &m,
                                   int corners) {
   using G = Geo<D, NC>;
   using L = Lay<D, NC, T>;
   const DBox &bx = boxes[id - 1];
   T *u = var + (size_t)(id - 1) * L::STRIDE;
-  lds_stage<D, NC, BS, T, BB>(s, boxes, bx, id, var, m, -1);
+  Stage<D, NC, BS, T, BB, false> sg;
+  sg.issue(bx, id, var, m, 0);
+  sg.commit(s, cp, bx, m);
   if (corners) {
     if (D == 3) {
       for (int q = ltid<BS>(); q < 12 * NC; q += BS) {
@@ -1885,11 +2002,12 @@ template <int D, int NC, int BS, typename T, int BB = 1>
 __global__ void __launch_bounds__(BS * BB) k_gc_lds(const int *__restrict__ ids, const DBox *__restrict__ boxes, T *var,
                                                     VarBc m, int corners, int nw) {
   __shared__ T s_all[BB][Geo<D, NC>::NCELL];
-  T *s = s_all[lgrp<BS, BB>()];
+  __shared__ T cp_all[BB][2 * D * CoarsePatch<D, NC>::N];
+  T *s = s_all[lgrp<BS, BB>()], *cp = cp_all[lgrp<BS, BB>()];
   for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
-    const int id = ids[w];
+    const int id = __builtin_amdgcn_readfirstlane(ids[w]);
     if (id <= 0) continue;  // run masked out
-    gc_lds_box<D, NC, BS, T, BB>(s, boxes, id, var, m, corners);
+    gc_lds_box<D, NC, BS, T, BB>(s, cp, boxes, id, var, m, corners);
   }
 }
 
@@ -1905,10 +2023,11 @@ template <int D, int NC, int BS>
 __global__ void __launch_bounds__(BS) k_gc_lds_vars(const int *__restrict__ ids, const DBox *__restrict__ boxes,
                                                     GcVars vars, int corners, int nw) {
   __shared__ double s[Geo<D, NC>::NCELL];
+  __shared__ double cp[2 * D * CoarsePatch<D, NC>::N];
   for (int w = blockIdx.x; w < nw; w += gridDim.x) {
     const int id = ids[w / vars.n];
     if (id <= 0) continue;
-    gc_lds_box<D, NC, BS, double, 1>(s, boxes, id, vars.v[w % vars.n], vars.m[w % vars.n], corners);
+    gc_lds_box<D, NC, BS, double, 1>(s, cp, boxes, id, vars.v[w % vars.n], vars.m[w % vars.n], corners);
   }
 }
 
