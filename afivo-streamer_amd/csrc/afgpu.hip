@@ -30,6 +30,7 @@
 #include "afgpu_chem.h"
 #include "afgpu_diag.h"
 #include "afgpu_refine.h"
+#include "afgpu_tail.h"
 
 using namespace afg;
 
@@ -296,6 +297,18 @@ struct afgpu_ctx {
       double *mf = nullptr, *bf = nullptr, *eigf = nullptr;
     } f[1 + AFGPU_MAX_MODES];
   } dir;
+  // the coarse levels of the FP64 multigrid in one workgroup per run
+  // (k_tail): levels 1..lt, the box id of every slot, and the operations
+  // recorded for the next launch while a cycle is being enqueued
+  struct Tail {
+    bool set = false;  // lt and the map are current for the tree
+    int lt = 0;
+    int *d_map = nullptr;
+    size_t n_map = 0;
+    unsigned *d_tab = nullptr;  // the geometry's index tables (tail_tables)
+    int op = -1;  // the operator whose cycle is being enqueued (-1: none)
+    std::vector<TailOp> ops;
+  } tail;
   // reductions
   unsigned long long *d_red = nullptr, *h_red = nullptr;  // [run][stripe][slot], host: [run][slot]
   unsigned long long *d_red_out = nullptr;                // stripes folded, [run][slot]
@@ -543,6 +556,7 @@ struct Impl : ImplBase {
   template <typename K, typename... Args>
   int launch(K kernel, int nblocks, Args... args) {
     if (nblocks <= 0) return AFGPU_OK;
+    RCHK(tail_flush());
     hipLaunchKernelGGL(kernel, dim3(nblocks), dim3(BS), 0, c.cur, args...);
     HIPCHK(hipGetLastError());
     return AFGPU_OK;
@@ -586,6 +600,7 @@ struct Impl : ImplBase {
   int items(int cls, K kernel, int nw, Args... args) {
     if (c.class_timing && c.timing && !c.capture_pairs) return items_timed<BB>(3 + cls, 0.0, cls, kernel, nw, args...);
     if (nw <= 0) return AFGPU_OK;
+    RCHK(tail_flush());
     hipLaunchKernelGGL(kernel, dim3(grid_for(cls, nw, BB)), dim3(BS * BB), 0, c.cur, args..., nw);
     HIPCHK(hipGetLastError());
     return AFGPU_OK;
@@ -600,6 +615,7 @@ struct Impl : ImplBase {
   // items_timed() of a kernel with NT threads per workgroup
   template <int NT, int BB, typename K, typename... Args>
   int items_nt(int kind, double bytes, int cls, K kernel, int nw, Args... args) {
+    RCHK(tail_flush());
     if (!c.timing || c.capture_pairs) {
       if (nw <= 0) return AFGPU_OK;
       hipLaunchKernelGGL(kernel, dim3(grid_for(cls, nw, BB)), dim3(NT), 0, c.cur, args..., nw);
@@ -611,6 +627,153 @@ struct Impl : ImplBase {
     hipEvent_t a, b;
     RCHK(timer_events(c, kind, bytes, &a, &b));
     hipExtLaunchKernelGGL(kernel, dim3(grid_for(cls, nw, BB)), dim3(NT), 0, c.cur, a, b, 0, args..., nw);
+    HIPCHK(hipGetLastError());
+    return AFGPU_OK;
+  }
+
+  // --- coarse levels of the FP64 cycles (k_tail) ------------------------------
+  using TG = TailGeo<D, NC>;
+  // The levels held by k_tail: levels 1..lt cover the domain of every run,
+  // with the neighbours that a box's position implies (allocation and
+  // upload, so this runs before any capture).
+  int ensure_tail() {
+    afgpu_ctx::Tail &tl = c.tail;
+    if (tl.set) return AFGPU_OK;
+    constexpr int S = TG::SLOTS;
+    std::vector<int> map((size_t)c.n_runs * S, 0);
+    int lt = 0;
+    for (int l = 1; l <= std::min((int)TG::LT, c.highest_lvl); l++) {
+      const int n1 = 1 << (l - 1), per = 1 << (D * (l - 1)), off = TG::off(l);
+      bool ok = (long long)c.l_ids[l].n == (long long)c.n_runs * per;
+      auto pos_of = [&](const int *x) { return x[0] + n1 * (x[1] + (D == 3 ? n1 * x[2] : 0)); };
+      for (int q = 0; ok && q < c.l_ids[l].n; q++) {
+        const int id = std::abs(c.h_lists[c.l_ids[l].off + q]);
+        const DBox &b = c.hboxes[id - 1];
+        int x[3] = {0, 0, 0};
+        for (int d = 0; d < D; d++) {
+          x[d] = b.ix[d] - 1;
+          ok = ok && x[d] >= 0 && x[d] < n1;
+        }
+        ok = ok && b.run >= 0 && b.run < c.n_runs;
+        if (!ok) break;
+        int &m = map[(size_t)b.run * S + off + pos_of(x)];
+        ok = m == 0;
+        m = id;
+      }
+      for (int r = 0; ok && r < c.n_runs; r++) {
+        const int *m = &map[(size_t)r * S + off];
+        for (int p = 0; ok && p < per; p++) {
+          const DBox &b = c.hboxes[m[p] - 1], &b0 = c.hboxes[m[0] - 1];
+          const int x[3] = {p % n1, (p / n1) % n1, p / (n1 * n1)};
+          // same-level neighbours where the domain goes on, the physical
+          // boundary where it ends; diagonals alike
+          auto id_at = [&](int dx, int dy, int dz) {
+            const int y[3] = {x[0] + dx, x[1] + dy, x[2] + dz};
+            for (int d = 0; d < D; d++)
+              if (y[d] < 0 || y[d] >= n1) return 0;
+            return m[pos_of(y)];
+          };
+          for (int nb = 0; nb < 2 * D; nb++) {
+            const int o = (nb & 1) ? 1 : -1, d = nb / 2;
+            const int want = id_at(d == 0 ? o : 0, d == 1 ? o : 0, d == 2 ? o : 0);
+            ok = ok && (want > 0 ? b.nb[nb] == want : b.nb[nb] < 0);
+          }
+          for (int dz = (D == 3 ? -1 : 0); dz <= (D == 3 ? 1 : 0); dz++)
+            for (int dy = -1; dy <= 1; dy++)
+              for (int dx = -1; dx <= 1; dx++) {
+                if (!dx && !dy && !dz) continue;
+                const int want = id_at(dx, dy, dz), have = b.nbmat[nbmat_at<D>(dx, dy, dz)];
+                ok = ok && (want > 0 ? have == want : have <= 0);
+              }
+          for (int d = 0; d < D; d++) ok = ok && b.dr[d] == b0.dr[d];
+          ok = ok && b.r_min[0] == c.hboxes[m[x[0]] - 1].r_min[0];  // (of the same column)
+          if (l > 1) {
+            int y[3] = {x[0] >> 1, x[1] >> 1, x[2] >> 1};
+            const int h = n1 / 2;
+            ok = ok && b.parent == map[(size_t)r * S + TG::off(l - 1) + y[0] + h * (y[1] + (D == 3 ? h * y[2] : 0))];
+          }
+        }
+      }
+      if (!ok) break;
+      lt = l;
+    }
+    if (lt > 0) {
+      if (!tl.d_tab) {
+        std::vector<unsigned> tab(TG::N_GH + TG::N_CR);
+        tail_tables<D, NC>(tab.data(), tab.data() + TG::N_GH);
+        HIPCHK(hipMalloc(&tl.d_tab, tab.size() * sizeof(unsigned)));
+        HIPCHK(hipMemcpy(tl.d_tab, tab.data(), tab.size() * sizeof(unsigned), hipMemcpyHostToDevice));
+      }
+      if (map.size() > tl.n_map) {
+        (void)hipFree(tl.d_map);
+        tl.d_map = nullptr;
+        tl.n_map = 0;
+        HIPCHK(hipMalloc(&tl.d_map, map.size() * sizeof(int)));
+        tl.n_map = map.size();
+      }
+      // (slots above level lt, which a failed check may have left half
+      // filled, are read by nothing)
+      HIPCHK(hipMemcpy(tl.d_map, map.data(), map.size() * sizeof(int), hipMemcpyHostToDevice));
+    }
+    tl.lt = lt;
+    tl.set = true;
+    if (lt > 0 && c.masked) RCHK(mask_tail());
+    return AFGPU_OK;
+  }
+  int mask_tail() {
+    const int n = c.n_runs * TG::SLOTS;
+    hipLaunchKernelGGL(k_mask_ids, dim3((n + 255) / 256), dim3(256), 0, c.cur, c.tail.d_map, n,
+                       (const int *)c.d_run_of, (const int *)c.d_run_active);
+    HIPCHK(hipGetLastError());
+    return AFGPU_OK;
+  }
+  // Enqueue an FP64 cycle of operator op (body), its operations on levels
+  // 1..lt recorded and run by k_tail; not while launches are timed, class by
+  // class.
+  template <typename F>
+  int with_tail(int op, F body) {
+    c.tail.ops.clear();
+    c.tail.op = (c.tail.set && c.tail.lt > 0 && !c.timing) ? op : -1;
+    int rc = body();
+    if (rc == AFGPU_OK) rc = tail_flush();
+    c.tail.op = -1;
+    c.tail.ops.clear();
+    return rc;
+  }
+  template <typename T>
+  bool in_tail(int lvl) const {
+    return std::is_same<T, double>::value && c.tail.op >= 0 && lvl <= c.tail.lt;
+  }
+  int tail_push(int code, int lvl, int a = 0, int b = 0) {
+    c.tail.ops.push_back(TailOp{(unsigned char)code, (unsigned char)lvl, (unsigned char)a, (unsigned char)b});
+    return (int)c.tail.ops.size() == TAIL_MAX_OPS ? tail_flush() : AFGPU_OK;
+  }
+  // Every other launch of a cycle comes after the recorded operations.
+  int tail_flush() {
+    afgpu_ctx::Tail &tl = c.tail;
+    if (tl.op < 0 || tl.ops.empty()) return AFGPU_OK;
+    const Mg<double> v = mg64(tl.op);
+    const afgpu_ctx::Op &o = c.ops[tl.op];
+    TailArgs A{};
+    A.map = tl.d_map;
+    A.gh = tl.d_tab;
+    A.cr = tl.d_tab + TG::N_GH;
+    A.boxes = c.d_boxes;
+    A.phi = v.phi;
+    A.rhs = v.rhs;
+    A.tmp = v.tmp;
+    A.m = v.m;
+    A.lambda2 = v.lambda2;
+    A.vinv = o.d_vinv;
+    A.v = o.d_v;
+    A.eig = o.d_eig;
+    A.red = c.d_red;
+    A.cyl = c.coord == AFGPU_CYL;
+    A.lt = tl.lt;
+    A.n_ops = (int)tl.ops.size();
+    std::copy(tl.ops.begin(), tl.ops.end(), A.ops);
+    tl.ops.clear();
+    hipLaunchKernelGGL((k_tail<D, NC>), dim3(c.n_runs), dim3(TAIL_NT), 0, c.cur, A);
     HIPCHK(hipGetLastError());
     return AFGPU_OK;
   }
@@ -636,6 +799,7 @@ struct Impl : ImplBase {
 
   template <typename T>
   int gc_var(int lvl, T *var, const VarBc &m, bool corners) {
+    if (in_tail<T>(lvl)) return tail_push(TL_GC, lvl, corners);
     return gc_list(c.l_ids[lvl], var, m, corners);
   }
   // the ghost layer of the boxes of list l (all of one level)
@@ -704,6 +868,10 @@ struct Impl : ImplBase {
   int gsrb_boxes(const Mg<T> &v, int lvl, bool down, bool final_gc = true, bool stored_first = false) {
     int n_cycle = down ? c.p.mg_n_cycle_down : c.p.mg_n_cycle_up;
     if (std::is_same<T, float>::value && c.mixed_smooth > 0) n_cycle = c.mixed_smooth;
+    if (in_tail<T>(lvl) && n_cycle <= 127) {
+      return tail_push(TL_SWEEP, lvl, 2 * n_cycle,
+                       (stored_first ? TS_STORED : 0) | (final_gc ? TS_GC : 0) | (final_gc && !down ? TS_CORNERS : 0));
+    }
     const List &l = c.l_ids[lvl];
     // algorithmic bytes of a half-sweep: the other colour and the rhs of
     // the updated colour are read, the updated colour is written
@@ -780,6 +948,9 @@ struct Impl : ImplBase {
       // run's own finest level needs it, and for the other runs the fill
       // repeats the one the level above has just made, with the same values)
       if (!v_cycle && (lvl == c.highest_lvl || c.uneven)) RCHK(gc_var(lvl, v.phi, v.m, true));
+      if (in_tail<T>(lvl))
+        RCHK(tail_push(TL_RESTRICT, lvl, !v_cycle));
+      else
       RCHK(with_bb(KC_RESTRICT, [&](auto B) {
         constexpr int bb = decltype(B)::value;
         return items<bb>(KC_RESTRICT, k_restrict_residual<D, NC, BS, T, bb>, l.n * k, c.list(l),
@@ -787,6 +958,7 @@ struct Impl : ImplBase {
       }));
     }
     RCHK(gc_var(lvl - 1, v.phi, v.m, true));
+    if (in_tail<T>(lvl - 1)) return tail_push(TL_RHS, lvl - 1, v_cycle);
     const List &pl = c.l_parents[lvl - 1];
     const int k2 = bpb(pl.n, G::NCELL);
     return with_bb(KC_PROLONG, [&](auto B) {
@@ -799,7 +971,11 @@ struct Impl : ImplBase {
   // (target: the buffer holding the children's level, see use_block)
   template <typename T>
   int correct_children(const Mg<T> &v, int lvl_p, T *target = nullptr) {
-    RCHK(boxop<T>(c.l_parents[lvl_p], v.phi, v.tmp, OP_SUB_FROM));
+    if (in_tail<T>(lvl_p))
+      RCHK(tail_push(TL_SUB, lvl_p));
+    else
+      RCHK(boxop<T>(c.l_parents[lvl_p], v.phi, v.tmp, OP_SUB_FROM));
+    if (in_tail<T>(lvl_p + 1)) return tail_push(TL_PROLONG, lvl_p + 1);
     const List &l = c.l_ids[lvl_p + 1];
     const int k = bpb(l.n, G::NINT);
     return with_bb(KC_PROLONG, [&](auto B) {
@@ -839,6 +1015,10 @@ struct Impl : ImplBase {
   // widened on load and rounded on store).
   template <typename T>
   int solve_coarse(const Mg<T> &v) {
+    if (in_tail<T>(1)) {
+      RCHK(tail_push(TL_SOLVE, 1));
+      return gc_var(1, v.phi, v.m, true);
+    }
     const List &l1 = c.l_ids[1];  // one box per run
     const afgpu_ctx::Op &o = c.ops[v.op];
     hipLaunchKernelGGL((k_coarse_solve<D, NC, 1024, T>), dim3(l1.n), dim3(1024), 0, c.cur, c.list(l1),
@@ -851,8 +1031,10 @@ struct Impl : ImplBase {
 
   int vcycle(int op, bool set_residual, int max_lvl) override {
     RCHK(ensure_factors(op));  // allocation and upload happen outside any capture
-    return run_graph(c, {G_VCYCLE, op, (int)set_residual, max_lvl},
-                     [&] { return vcycle_body(mg64(op), set_residual, max_lvl, 1, true); });
+    RCHK(ensure_tail());
+    return run_graph(c, {G_VCYCLE, op, (int)set_residual, max_lvl}, [&] {
+      return with_tail(op, [&] { return vcycle_body(mg64(op), set_residual, max_lvl, 1, true); });
+    });
   }
 
   // FAS V-cycle from max_lvl down to the coarsest level lc (1: the level-1
@@ -873,24 +1055,36 @@ struct Impl : ImplBase {
     // (no ghost fill between the correction and the smoother: the fused
     // half-sweeps form every out-of-box neighbour themselves, and the
     // stored layer is rewritten after the last half-sweep)
+    int res_lo = 1;  // levels below have their residual already
     for (int lvl = lc + 1; lvl <= max_lvl; lvl++) {
+      if (set_residual && lvl > 2 && in_tail<T>(lvl - 1) && !in_tail<T>(lvl)) {
+        // the last operations of this cycle in k_tail: the residuals of its
+        // levels but the finest, whose tmp the prolongation still reads
+        RCHK(tail_push(TL_RESET, 1));
+        for (int l = 1; l < lvl - 1; l++) RCHK(tail_push(TL_RESID, l));
+        res_lo = lvl - 1;
+      }
       RCHK(correct_children(v, lvl - 1, level_buf(v, lvl, true)));
       // the single-precision correction's ghost layer on the finest level
       // is read by nothing after the cycle
       const bool final_gc = !(std::is_same<T, float>::value && lvl == c.highest_lvl);
       RCHK(gsrb_boxes(v, lvl, false, final_gc));
     }
-    if (set_residual) RCHK(residual_pass(v, max_lvl, true));
+    if (set_residual) RCHK(residual_pass(v, max_lvl, res_lo == 1, res_lo));
     return AFGPU_OK;
   }
   // residual on every box of levels 1..max_lvl; the max |residual| over
   // leaves is reduced on the fly into slot 0 of each run (read back with
   // leaf_residual_max), cleared first with `reset`
   template <typename T>
-  int residual_pass(const Mg<T> &v, int max_lvl, bool reset) {
+  int residual_pass(const Mg<T> &v, int max_lvl, bool reset, int min_lvl = 1) {
     const int cyl = c.coord == AFGPU_CYL;
-    if (reset) RCHK(set_red(0, 0ull));
-    for (int lvl = 1; lvl <= max_lvl; lvl++) {
+    if (reset) RCHK(in_tail<T>(1) ? tail_push(TL_RESET, 1) : set_red(0, 0ull));
+    for (int lvl = min_lvl; lvl <= max_lvl; lvl++) {
+      if (in_tail<T>(lvl) && (lvl == max_lvl || min_lvl == 1)) {
+        RCHK(tail_push(TL_RESID, lvl));
+        continue;
+      }
       const List &l = c.l_ids[lvl];
       const int k = bpb(l.n, G::NINT);
       RCHK(with_bb(KC_RESID, [&](auto B) {
@@ -941,6 +1135,7 @@ struct Impl : ImplBase {
   // Device side of the masks (capturable): the list kernels work on the
   // runs made active by the host whose highest level lies in [lo, hi].
   int mask_levels(int lo, int hi) {
+    RCHK(tail_flush());
     hipLaunchKernelGGL(k_runs_in_levels, dim3((c.n_runs + 63) / 64), dim3(64), 0, c.cur, (const int *)c.d_run_host,
                        (const int *)c.d_run_maxlvl, c.d_run_active, lo, hi, c.n_runs);
     HIPCHK(hipGetLastError());
@@ -954,7 +1149,7 @@ struct Impl : ImplBase {
                          (const int *)c.d_run_of, (const int *)c.d_run_active);
       HIPCHK(hipGetLastError());
     }
-    return AFGPU_OK;
+    return (c.tail.set && c.tail.lt > 0) ? mask_tail() : AFGPU_OK;
   }
 
   // Device side of the masks of a mode's close in a forest (capturable):
@@ -973,10 +1168,18 @@ struct Impl : ImplBase {
 
   int fmg(int op, bool set_residual, bool have_guess) override {
     RCHK(ensure_factors(op));
-    return run_graph(c, {G_FMG, op, (int)set_residual, (int)have_guess},
-                     [&] { return fmg_body(mg64(op), set_residual, have_guess); });
+    RCHK(ensure_tail());
+    return run_graph(c, {G_FMG, op, (int)set_residual, (int)have_guess}, [&] {
+      return with_tail(op, [&] { return fmg_body(mg64(op), set_residual, have_guess); });
+    });
   }
 
+  // tmp = phi on a level
+  template <typename T>
+  int copy_phi(const Mg<T> &v, int lvl) {
+    if (in_tail<T>(lvl)) return tail_push(TL_COPY, lvl);
+    return boxop<T>(c.l_ids[lvl], v.phi, v.tmp, OP_COPY);
+  }
   template <typename T>
   int fmg_body(const Mg<T> &v, bool set_residual, bool have_guess, int lc = 1) {
     if (have_guess) {
@@ -996,11 +1199,11 @@ struct Impl : ImplBase {
     // the single-precision correction starts from zero on its coarsest level
     // too (refined boxes there keep the last cycle's values otherwise)
     if (std::is_same<T, float>::value && !have_guess) RCHK(boxop<T>(c.l_ids[lc], v.phi, v.phi, OP_CLEAR));
-    RCHK(boxop<T>(c.l_ids[lc], v.phi, v.tmp, OP_COPY));
+    RCHK(copy_phi(v, lc));
     if (c.uneven) return fmg_up_uneven(v, set_residual, lc);
     RCHK(vcycle_body(v, set_residual && c.highest_lvl == lc, lc, lc));
     for (int lvl = lc + 1; lvl <= c.highest_lvl; lvl++) {
-      RCHK(boxop<T>(c.l_ids[lvl], v.phi, v.tmp, OP_COPY));
+      RCHK(copy_phi(v, lvl));
       RCHK(correct_children(v, lvl - 1));
       RCHK(vcycle_body(v, set_residual && lvl == c.highest_lvl, lvl, lc));
     }
@@ -1022,7 +1225,7 @@ struct Impl : ImplBase {
     }
     for (int lvl = lc + 1; lvl <= c.highest_lvl; lvl++) {
       RCHK(mask_levels(lvl, top));
-      RCHK(boxop<T>(c.l_ids[lvl], v.phi, v.tmp, OP_COPY));
+      RCHK(copy_phi(v, lvl));
       RCHK(correct_children(v, lvl - 1));
       RCHK(vcycle_body(v, false, lvl, lc));
       if (set_residual) {
@@ -1541,6 +1744,7 @@ struct Impl : ImplBase {
   // reduction slot i of every run := value (a kernel, so that it can live
   // in a graph)
   int set_red(int i, unsigned long long value) {
+    RCHK(tail_flush());
     hipLaunchKernelGGL(k_set_run_slots, dim3((c.n_runs * RED_STRIPES + 63) / 64), dim3(64), 0, c.cur, c.d_red + i,
                        value, c.n_runs);
     HIPCHK(hipGetLastError());
@@ -2617,6 +2821,8 @@ int afgpu_destroy(afgpu_t *h) {
   for (int i = 0; i < AFGPU_N_CC; i++) (void)hipFree(h->cc[i]);
   for (int i = 0; i < AFGPU_N_FC; i++) (void)hipFree(h->fc[i]);
   for (int i = 0; i < 4; i++) (void)hipFree(h->cc32[i]);
+  (void)hipFree(h->tail.d_map);
+  (void)hipFree(h->tail.d_tab);
   (void)hipFree(h->dir.d_map);
   (void)hipFree(h->d_ref_ids);
   (void)hipFree(h->d_ref_flags);
@@ -2981,6 +3187,7 @@ int afgpu_sync_tree(afgpu_t *h, int n_boxes, const int *lvl, const int *ix, cons
   for (auto &o : h->ops) o.ok = false;  // level-1 box may have changed
   h->dir.set = false;
   for (auto &f : h->dir.f) f.ok = false;
+  h->tail.set = false;
   drop_graphs(*h);
   return AFGPU_OK;
 }

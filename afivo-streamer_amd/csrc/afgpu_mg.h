@@ -537,6 +537,24 @@ __device__ inline T restrict_cell(const T *f, int i_f, int jf, int kf, bool cyl_
   }
 }
 
+// The same from the children's 2^D values (i fastest, then j, then k).
+template <typename T>
+__device__ inline T restrict_weight(const DBox &bp, int ic) {
+  const T r = (T)bp.r_min[0] + (T(ic) - T(0.5)) * (T)bp.dr[0];
+  return T(0.25) * (T)bp.dr[0] / r;
+}
+template <int D, typename T>
+__device__ inline T restrict_children(const T *rs, bool cyl_geom, const DBox &bp, int ic) {
+  if (D == 2 && cyl_geom) {
+    const T t = restrict_weight<T>(bp, ic);
+    T w1 = T(1) - t, w2 = T(1) + t;
+    return T(0.25) * (w1 * (rs[0] + rs[2]) + w2 * (rs[1] + rs[3]));
+  }
+  T sm = rs[0];
+  for (int c = 1; c < (1 << D); c++) sm = sm + rs[c];
+  return T(1.0 / (1 << D)) * sm;
+}
+
 // Restrict variable `src` of child boxes into `dst` of their parents.
 template <int D, int NC, int BS, typename T, int BB = 1>
 __global__ void __launch_bounds__(BS * BB) k_restrict(const int *__restrict__ ids, const DBox *__restrict__ boxes,
@@ -604,25 +622,7 @@ __global__ void __launch_bounds__(BS * BB) k_restrict_residual(const int *__rest
         if (store_residual) tmp[cb + cp[c]] = rs[c];
       }
       const int ic = off[0] + i, jc = off[1] + j, kc = (D == 3) ? off[2] + k : 0;
-      T rv;
-      if (D == 2) {
-        if (cyl) {
-          T r = (T)bp.r_min[0] + (T(ic) - T(0.5)) * (T)bp.dr[0];
-          T t = T(0.25) * (T)bp.dr[0] / r;
-          T w1 = T(1) - t, w2 = T(1) + t;
-          rv = T(0.25) * (w1 * (rs[0] + rs[2]) + w2 * (rs[1] + rs[3]));
-        } else {
-          T sm = rs[0];
-          sm = sm + rs[1];
-          sm = sm + rs[2];
-          sm = sm + rs[3];
-          rv = T(0.25) * sm;
-        }
-      } else {
-        T sm = rs[0];
-        for (int c = 1; c < 8; c++) sm = sm + rs[c];
-        rv = T(0.125) * sm;
-      }
+      const T rv = restrict_children<D, T>(rs, cyl != 0, bp, ic);
       tmp[pb + L::in_at(ic, jc, kc)] = rv;
       phi[pb + L::in_at(ic, jc, kc)] = restrict_cell<D, NC, T, L>(phi + cb, i_f, jf, kf, false, bp, ic);
     }
@@ -706,9 +706,28 @@ __global__ void __launch_bounds__(BS * BB) k_boxop(const int *__restrict__ ids, 
   }
 }
 
-// phi(child) += P(tmp(parent)): stencil_prolong_248 with add
-// (afivo/src/m_af_stencil.f90:695-815), weights of
+// v + P(tmp) at cell (i, j, k) of a child box at offset off within its
+// parent, whose values P are: stencil_prolong_248
+// (afivo/src/m_af_stencil.f90:695-815) with the weights of
 // mg_box_prolong_linear_stencil (m_af_multigrid.f90:1267-1284).
+template <int D, int NC, typename T>
+__device__ inline T prolong_value(T v, const T *P, const int *off, int i, int j, int k) {
+  using L = Lay<D, NC, T>;
+  const int i1 = off[0] + ((i + 1) >> 1), i2 = i1 + 1 - 2 * (i & 1);
+  const int j1 = off[1] + ((j + 1) >> 1), j2 = j1 + 1 - 2 * (j & 1);
+  if (D == 2) {
+    const T w0 = T(9 / 16.0), w1 = T(3 / 16.0), w2 = T(3 / 16.0), w3 = T(1 / 16.0);
+    return v + w0 * P[L::at(i1, j1, 0)] + w1 * P[L::at(i2, j1, 0)] + w2 * P[L::at(i1, j2, 0)] +
+           w3 * P[L::at(i2, j2, 0)];
+  }
+  const int k1 = off[2] + ((k + 1) >> 1), k2 = k1 + 1 - 2 * (k & 1);
+  const T w0 = T(27 / 64.0), w1 = T(9 / 64.0), w3 = T(3 / 64.0), w7 = T(1 / 64.0);
+  return v + w0 * P[L::at(i1, j1, k1)] + w1 * P[L::at(i2, j1, k1)] + w1 * P[L::at(i1, j2, k1)] +
+         w3 * P[L::at(i2, j2, k1)] + w1 * P[L::at(i1, j1, k2)] + w3 * P[L::at(i2, j1, k2)] +
+         w3 * P[L::at(i1, j2, k2)] + w7 * P[L::at(i2, j2, k2)];
+}
+
+// phi(child) += P(tmp(parent)), with add.
 template <int D, int NC, int BS, typename T, int BB = 1>
 __global__ void __launch_bounds__(BS * BB) k_prolong_add(const int *__restrict__ ids, const DBox *__restrict__ boxes,
                                                          const T *__restrict__ src, T *dst, int bpb, int nw) {
@@ -727,20 +746,8 @@ __global__ void __launch_bounds__(BS * BB) k_prolong_add(const int *__restrict__
     for (int q = pt.q0; q < G::NINT; q += pt.stride) {
       int i, j, k;
       interior_ijk<D, NC>(q, i, j, k);
-      const int i1 = off[0] + ((i + 1) >> 1), i2 = i1 + 1 - 2 * (i & 1);
-      const int j1 = off[1] + ((j + 1) >> 1), j2 = j1 + 1 - 2 * (j & 1);
-      const int x = L::at(i, j, k);
-      if (D == 2) {
-        const T w0 = T(9 / 16.0), w1 = T(3 / 16.0), w2 = T(3 / 16.0), w3 = T(1 / 16.0);
-        u[x] = u[x] + w0 * P[L::at(i1, j1, 0)] + w1 * P[L::at(i2, j1, 0)] + w2 * P[L::at(i1, j2, 0)] +
-               w3 * P[L::at(i2, j2, 0)];
-      } else {
-        const int k1 = off[2] + ((k + 1) >> 1), k2 = k1 + 1 - 2 * (k & 1);
-        const T w0 = T(27 / 64.0), w1 = T(9 / 64.0), w3 = T(3 / 64.0), w7 = T(1 / 64.0);
-        u[x] = u[x] + w0 * P[L::at(i1, j1, k1)] + w1 * P[L::at(i2, j1, k1)] + w1 * P[L::at(i1, j2, k1)] +
-               w3 * P[L::at(i2, j2, k1)] + w1 * P[L::at(i1, j1, k2)] + w3 * P[L::at(i2, j1, k2)] +
-               w3 * P[L::at(i1, j2, k2)] + w7 * P[L::at(i2, j2, k2)];
-      }
+      T &v = u[L::at(i, j, k)];
+      v = prolong_value<D, NC, T>(v, P, off, i, j, k);
     }
   }
 }
@@ -817,12 +824,104 @@ __global__ void __launch_bounds__(BS * BB) k_maxabs(const int *__restrict__ ids,
   }
 }
 
+// Level-1 rhs b at cell (i, j, k) with the boundary values folded in, as
+// coarse_solver_set_rhs_phi does (afivo/src/m_coarse_solver.f90:286-338).
+template <int D, int NC>
+__device__ inline double coarse_rhs_value(const DBox &bx, const VarBc &m, const Sten<D, double> &s, bool cyl, double b,
+                                          int i, int j, int k) {
+  const int p[3] = {i, j, (D == 3) ? k : 1};
+#pragma unroll
+  for (int nb = 0; nb < 2 * D; nb++) {
+    if (bx.nb[nb] >= 0) continue;
+    const int d = nb / 2;
+    const bool low = (nb % 2) == 0;
+    if (p[d] != (low ? 1 : NC)) continue;
+    double cnb = s.c[1 + nb];
+    if (cyl && d == 0) {
+      double dr = bx.dr[0];
+      double rr = bx.r_min[0] + (i - 0.5) * dr;
+      double inv_r = 1 / rr;
+      double rf = low ? (rr - 0.5 * dr) * inv_r : (rr + 0.5 * dr) * inv_r;
+      cnb = rf * s.c[1 + nb];
+    }
+    double f;
+    if (m.type[nb] == BC_DIRICHLET)
+      f = -2 * cnb;
+    else
+      f = -(cnb * bx.dr[d]) * (double)(low ? -1 : 1);
+    b = b + f * bc_value(m, nb, bx.run);
+  }
+  return b;
+}
+// One axis of the level-1 transforms: out = M buf along axis AX, with M's
+// rows padded to NC + 1 (rows of different lanes then lie in different LDS
+// banks).  A thread's cells differ along the last axis, so along the other
+// axes they share the matrix row and along the last axis the line.
+template <int D, int NC, int NT, int AX>
+__device__ inline void coarse_axis(double *buf, const double *M) {
+  constexpr int N = Geo<D, NC>::NINT, PER = (N + NT - 1) / NT;
+  constexpr int st = (AX == 0) ? 1 : (AX == 1) ? NC : NC * NC;
+  static_assert(N % NT == 0 || N < NT, "whole strides of cells");
+  const int tid = threadIdx.x;
+  double out[PER];
+  if (tid < N) {
+    int row[PER], line[PER];
+#pragma unroll
+    for (int t = 0; t < PER; t++) {
+      const int q = tid + t * NT;
+      row[t] = (q / st) % NC;
+      line[t] = q - row[t] * st;
+      out[t] = 0.0;
+    }
+    if constexpr (AX < D - 1 && N > NT) row[PER - 1] = row[0];  // (equal; so the compiler reads the row once)
+#pragma unroll 4
+    for (int mm = 0; mm < NC; mm++) {
+      const double m0 = M[row[0] * (NC + 1) + mm], b0 = buf[line[0] + mm * st];
+#pragma unroll
+      for (int t = 0; t < PER; t++) {
+        const double mt = (AX < D - 1) ? m0 : M[row[t] * (NC + 1) + mm];
+        const double bt = (AX == D - 1 && N > NT) ? b0 : buf[line[t] + mm * st];
+        out[t] = out[t] + mt * bt;
+      }
+    }
+  }
+  __syncthreads();
+  if (tid < N)
+#pragma unroll
+    for (int t = 0; t < PER; t++) buf[tid + t * NT] = out[t];
+  __syncthreads();
+}
+// The level-1 solve on buf (interior cells, x fastest): V^-1 along each
+// axis, division by the eigenvalue sums, V along each axis.  mat: the 2 D
+// matrices, V^-1 first, rows padded to NC + 1.
+template <int D, int NC, int NT>
+__device__ inline void coarse_transforms(double *buf, const double *mat, const double *__restrict__ eig,
+                                         double lambda2) {
+  constexpr int MS = NC * (NC + 1);
+  coarse_axis<D, NC, NT, 0>(buf, mat);
+  coarse_axis<D, NC, NT, 1>(buf, mat + MS);
+  if constexpr (D == 3) coarse_axis<D, NC, NT, 2>(buf, mat + 2 * MS);
+  for (int q = threadIdx.x; q < Geo<D, NC>::NINT; q += NT) {
+    int i, j, k;
+    interior_ijk<D, NC>(q, i, j, k);
+    double den = eig[i - 1] + eig[NC + j - 1];
+    if (D == 3) den = den + eig[2 * NC + k - 1];
+    den = den - lambda2;
+    buf[q] = buf[q] / den;
+  }
+  __syncthreads();
+  coarse_axis<D, NC, NT, 0>(buf, mat + D * MS);
+  coarse_axis<D, NC, NT, 1>(buf, mat + (D + 1) * MS);
+  if constexpr (D == 3) coarse_axis<D, NC, NT, 2>(buf, mat + (D + 2) * MS);
+}
+
 // Exact level-1 solve by fast diagonalisation (replaces hypre PFMG,
-// afivo/src/m_coarse_solver.f90:421): fold boundary values into the rhs as
-// coarse_solver_set_rhs_phi (:286-338) does, transform with V^-1 along each
-// axis, divide by the eigenvalue sums, transform back with V.  One
-// workgroup of CBS threads per level-1 box (one per run of a forest); the
-// box lives in LDS.
+// afivo/src/m_coarse_solver.f90:421): fold boundary values into the rhs,
+// transform with V^-1 along each axis, divide by the eigenvalue sums,
+// transform back with V.  One workgroup of CBS threads per level-1 box (one
+// per run of a forest); the box and the matrices live in LDS.  Bound by the
+// 2 D dependent products of one workgroup: 17 us for a 16^3 box, and 52 us
+// with the matrices read from memory by every cell.
 // TS is the storage type of rhs and phi; the transforms always run in FP64.
 template <int D, int NC, int CBS, typename TS>
 __global__ void __launch_bounds__(CBS) k_coarse_solve(const int *__restrict__ ids, const DBox *__restrict__ boxes,
@@ -834,79 +933,22 @@ __global__ void __launch_bounds__(CBS) k_coarse_solve(const int *__restrict__ id
   using G = Geo<D, NC>;
   using L = Lay<D, NC, TS>;
   constexpr int N = G::NINT;
-  constexpr int PER = (N + CBS - 1) / CBS;
   __shared__ double buf[N];
+  __shared__ double mat[2 * D * NC * (NC + 1)];
   const int id = ids[blockIdx.x];
   if (id <= 0) return;  // run masked out
   const DBox &bx = boxes[id - 1];
   const Sten<D, double> s = lpl_stencil<D, double>(bx, lambda2);
   const TS *r = rhs + (size_t)(id - 1) * L::STRIDE;
-  auto lin = [](int i, int j, int k) { return (i - 1) + NC * ((j - 1) + NC * (D == 3 ? k - 1 : 0)); };
+  for (int q = threadIdx.x; q < 2 * D * NC * NC; q += CBS)
+    mat[(q / NC) * (NC + 1) + q % NC] = (q < D * NC * NC) ? vinv[q] : v[q - D * NC * NC];
   for (int q = threadIdx.x; q < N; q += CBS) {
     int i, j, k;
     interior_ijk<D, NC>(q, i, j, k);
-    double bval = (double)r[L::in_at(i, j, k)];
-    int p[3] = {i, j, (D == 3) ? k : 1};
-    for (int nb = 0; nb < 2 * D; nb++) {
-      if (bx.nb[nb] >= 0) continue;
-      const int d = nb / 2;
-      const bool low = (nb % 2) == 0;
-      if (p[d] != (low ? 1 : NC)) continue;
-      double cnb = s.c[1 + nb];
-      if (cyl && d == 0) {
-        double dr = bx.dr[0];
-        double rr = bx.r_min[0] + (i - 0.5) * dr;
-        double inv_r = 1 / rr;
-        double rf = low ? (rr - 0.5 * dr) * inv_r : (rr + 0.5 * dr) * inv_r;
-        cnb = rf * s.c[1 + nb];
-      }
-      double f;
-      if (m.type[nb] == BC_DIRICHLET)
-        f = -2 * cnb;
-      else
-        f = -(cnb * bx.dr[d]) * (double)(low ? -1 : 1);
-      bval = bval + f * bc_value(m, nb, bx.run);
-    }
-    buf[lin(i, j, k)] = bval;
+    buf[q] = coarse_rhs_value<D, NC>(bx, m, s, cyl != 0, (double)r[L::in_at(i, j, k)], i, j, k);
   }
   __syncthreads();
-  for (int pass = 0; pass < 2 * D; pass++) {
-    const int d = pass % D;
-    const double *M = ((pass < D) ? vinv : v) + (size_t)d * NC * NC;
-    if (pass == D) {
-      for (int q = threadIdx.x; q < N; q += CBS) {
-        int i, j, k;
-        interior_ijk<D, NC>(q, i, j, k);
-        double den = eig[i - 1] + eig[NC + j - 1];
-        if (D == 3) den = den + eig[2 * NC + k - 1];
-        den = den - lambda2;
-        buf[q] = buf[q] / den;
-      }
-      __syncthreads();
-    }
-    double out[PER];
-    for (int t = 0; t < PER; t++) {
-      const int q = threadIdx.x + t * CBS;
-      if (q >= N) break;
-      int i, j, k;
-      interior_ijk<D, NC>(q, i, j, k);
-      int p[3] = {i, j, (D == 3) ? k : 1};
-      const int row = p[d];
-      double sum = 0.0;
-      for (int mm = 1; mm <= NC; mm++) {
-        int qq[3] = {p[0], p[1], p[2]};
-        qq[d] = mm;
-        sum = sum + M[(row - 1) * NC + (mm - 1)] * buf[lin(qq[0], qq[1], qq[2])];
-      }
-      out[t] = sum;
-    }
-    __syncthreads();
-    for (int t = 0; t < PER; t++) {
-      const int q = threadIdx.x + t * CBS;
-      if (q < N) buf[q] = out[t];
-    }
-    __syncthreads();
-  }
+  coarse_transforms<D, NC, CBS>(buf, mat, eig, lambda2);
   TS *u = phi + (size_t)(id - 1) * L::STRIDE;
   for (int q = threadIdx.x; q < N; q += CBS) {
     int i, j, k;
@@ -1066,29 +1108,40 @@ __device__ inline CoarseVals<T> coarse_patch_vals(const T *cp, const VarBc &m, i
   if (D == 3) cv.v[2] = at(a1, b2);
   return cv;
 }
+// Ghost of a face on the physical boundary from the box's first and second
+// cells x1, x2: p + c1 x1 + 0 x2 (ghost_value's operations, for an nb that
+// may differ between lanes).  dr: the box's spacing; run_val: the run's value
+// of face m.run_face.
+template <int D, typename T>
+__device__ inline void phys_coeffs(const double *dr, const VarBc &m, double run_val, int nb, T &p, T &c1) {
+  const int type = pick<2 * D>(m.type, nb);
+  const double bv = (m.run_val && nb == m.run_face) ? run_val : pick<2 * D>(m.val, nb);
+  T c0;
+  if (type == BC_DIRICHLET) {
+    c0 = 2;
+    c1 = -1;
+  } else if (type == BC_NEUMANN) {
+    c0 = (T)pick<D>(dr, nb >> 1) * T((nb & 1) ? 1 : -1);
+    c1 = 1;
+  } else {
+    c0 = 1;
+    c1 = 0;
+  }
+  p = c0 * (T)bv;
+}
+template <int D, typename T>
+__device__ inline T phys_ghost(const DBox &bx, const VarBc &m, double run_val, int nb, T x1, T x2) {
+  T p, c1;
+  phys_coeffs<D, T>(bx.dr, m, run_val, nb, p, c1);
+  return p + c1 * x1 + T(0) * x2;
+}
 // Ghost (a, b) of a face without a same-level neighbour (nbv <= 0) from the
 // box's first and second cells x1, x2 and, at a refinement boundary, the
-// face's coarse patch cp: ghost_value's operations, for an nb that may
-// differ between lanes.  run_val: the run's value of face m.run_face.
+// face's coarse patch cp.
 template <int D, int NC, typename T>
 __device__ inline T staged_ghost(const DBox &bx, const VarBc &m, double run_val, int nbv, int nb, int a, int b,
                                  const T *cp, T x1, T x2) {
-  if (nbv < 0) {
-    const int type = pick<2 * D>(m.type, nb);
-    const double bv = (m.run_val && nb == m.run_face) ? run_val : pick<2 * D>(m.val, nb);
-    T c0, c1;
-    if (type == BC_DIRICHLET) {
-      c0 = 2;
-      c1 = -1;
-    } else if (type == BC_NEUMANN) {
-      c0 = (T)pick<D>(bx.dr, nb >> 1) * T((nb & 1) ? 1 : -1);
-      c1 = 1;
-    } else {
-      c0 = 1;
-      c1 = 0;
-    }
-    return c0 * (T)bv + c1 * x1 + T(0) * x2;
-  }
+  if (nbv < 0) return phys_ghost<D, T>(bx, m, run_val, nb, x1, x2);
   const CoarseVals<T> cv = coarse_patch_vals<D, NC, T>(cp, m, a, b);
   const GhostPart<T> g = coarse_part<D, T>(m, nb >> 1, a, b, cv);
   return rb_finish<T>(m, g, x1, x2);
@@ -1778,25 +1831,7 @@ __global__ void __launch_bounds__(BS * BB) k_restrict_residual_lds(const int *__
         if (store_residual) tmp[cb + cp[c]] = rs[c];
       }
       const int ic = off[0] + i, jc = off[1] + j, kc = (D == 3) ? off[2] + k : 0;
-      T rv;
-      if (D == 2) {
-        if (cyl) {
-          T r = (T)bp.r_min[0] + (T(ic) - T(0.5)) * (T)bp.dr[0];
-          T t = T(0.25) * (T)bp.dr[0] / r;
-          T w1 = T(1) - t, w2 = T(1) + t;
-          rv = T(0.25) * (w1 * (rs[0] + rs[2]) + w2 * (rs[1] + rs[3]));
-        } else {
-          T sm = rs[0];
-          sm = sm + rs[1];
-          sm = sm + rs[2];
-          sm = sm + rs[3];
-          rv = T(0.25) * sm;
-        }
-      } else {
-        T sm = rs[0];
-        for (int c = 1; c < 8; c++) sm = sm + rs[c];
-        rv = T(0.125) * sm;
-      }
+      const T rv = restrict_children<D, T>(rs, cyl != 0, bp, ic);
       tmp[pb + L::in_at(ic, jc, kc)] = rv;
       phi[pb + L::in_at(ic, jc, kc)] = restrict_cell<D, NC, T>(s, i_f, jf, kf, false, bp, ic);
     }
