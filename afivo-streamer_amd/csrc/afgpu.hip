@@ -805,14 +805,10 @@ struct Impl : ImplBase {
   // the ghost layer of the boxes of list l (all of one level)
   template <typename T>
   int gc_list(const List &l, T *var, const VarBc &m, bool corners) {
-    const int k = corners ? 1 : bpb(l.n, 2 * D * G::NTAN);
-    if (k == 1)
-      return with_bb(KC_GC, [&](auto B) {
-        constexpr int bb = decltype(B)::value;
-        return items<bb>(KC_GC, k_gc_lds<D, NC, BS, T, bb>, l.n, c.list(l), (const DBox *)c.d_boxes, var, m,
-                         (int)corners);
-      });
-    return items<1>(KC_GC, k_gc<D, NC, BS, T, 1>, l.n * k, c.list(l), (const DBox *)c.d_boxes, var, m, (int)corners, k);
+    return with_bb(KC_GC, [&](auto B) {
+      constexpr int bb = decltype(B)::value;
+      return items<bb>(KC_GC, k_gc<D, NC, BS, T, bb>, l.n, c.list(l), (const DBox *)c.d_boxes, var, m, (int)corners);
+    });
   }
   int gc_lvl(int lvl, int iv, bool corners) override { return gc_var(lvl, c.cc[iv], var_methods(c, iv), corners); }
   int gc_tree(int iv) {
@@ -876,7 +872,6 @@ struct Impl : ImplBase {
     // algorithmic bytes of a half-sweep: the other colour and the rhs of
     // the updated colour are read, the updated colour is written
     const double bytes = 1.5 * sizeof(T) * l.n * G::NINT;
-    const int k = bpb(l.n, G::NINT / 2);
     const int cyl = c.coord == AFGPU_CYL;
     if (use_block<T>(lvl)) {
       T *in = down ? v.phi : v.alt, *out = down ? v.alt : v.phi;
@@ -889,32 +884,36 @@ struct Impl : ImplBase {
     for (int n = 1; n <= 2 * n_cycle; n++) {
       const int stored = (stored_first && n == 1 && !Lay<D, NC, T>::SPLIT) ? 1 : 0;
       if constexpr (D == 2 && Lay<D, NC, T>::SPLIT && NC == 8) {
-        if (k == 1 && !c.box_lds) {  // (a wavefront per eight boxes, four wavefronts per workgroup)
+        // A wavefront per eight boxes, four wavefronts per workgroup: on
+        // large levels, where the bytes count.  On small ones its chain of
+        // loads is the longer one: 4.7 us against 3.2 us for 1024 boxes,
+        // 5.2 against 4.5 for 6144, 5.2 against 6.1 for 8192.
+        if (l.n >= 7168 && !c.box_lds) {
           RCHK((items_nt<256, 1>(0, bytes, KC_GSRB, k_gsrb_split2d<NC>, (l.n + 31) / 32, c.list(l),
                                  (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, n, v.lambda2, cyl, v.m, l.n)));
           continue;
         }
       }
       if constexpr (D == 3 && Lay<D, NC, T>::SPLIT && BS == NC * NC) {
-        if (k == 1 && !c.box_lds) {
+        if (!c.box_lds) {
           RCHK((items_nt<GSRB_SPLIT_NT, 1>(0, bytes, KC_GSRB, k_gsrb_split<D, NC, GSRB_SPLIT_NT>, l.n, c.list(l),
                                            (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, n, v.lambda2, v.m)));
           continue;
         }
       }
-      if (k == 1)
-        RCHK(with_bb(KC_GSRB, [&](auto B) {
-          constexpr int bb = decltype(B)::value;
-          return items_timed<bb>(0, bytes, KC_GSRB, k_gsrb_lds<D, NC, BS, T, bb>, l.n, c.list(l),
-                                 (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, n, v.lambda2, cyl, v.m, stored);
-        }));
-      else
-        RCHK(with_bb(KC_GSRB, [&](auto B) {
-          constexpr int bb = decltype(B)::value;
-          return items_timed<bb>(0, bytes, KC_GSRB, k_gsrb<D, NC, BS, T, bb>, l.n * k, c.list(l),
-                                 (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, n, v.lambda2, cyl, v.m, stored,
-                                 k);
-        }));
+      if constexpr (D == 3 && NC == 16) {
+        // up to one box per CU: four times the threads on each
+        if (l.n <= c.n_cu) {
+          RCHK((items_nt<1024, 1>(0, bytes, KC_GSRB, k_gsrb_lds<D, NC, 1024, T, 1>, l.n, c.list(l),
+                                  (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, n, v.lambda2, cyl, v.m, stored)));
+          continue;
+        }
+      }
+      RCHK(with_bb(KC_GSRB, [&](auto B) {
+        constexpr int bb = decltype(B)::value;
+        return items_timed<bb>(0, bytes, KC_GSRB, k_gsrb_lds<D, NC, BS, T, bb>, l.n, c.list(l),
+                               (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, n, v.lambda2, cyl, v.m, stored);
+      }));
     }
     // ghost layer after the last half-sweep (corners on the final up-sweep)
     return final_gc ? gc_var(lvl, v.phi, v.m, !down) : AFGPU_OK;
@@ -2291,7 +2290,7 @@ struct Impl : ImplBase {
       gv.m[k] = var_methods(c, vars[k].methods);
     }
     const int nw = n * n_vars;
-    hipLaunchKernelGGL((k_gc_lds_vars<D, NC, BS>), dim3(std::min(nw, 8 * c.n_cu)), dim3(BS), 0, c.cur, ids,
+    hipLaunchKernelGGL((k_gc_vars<D, NC, BS>), dim3(std::min(nw, 8 * c.n_cu)), dim3(BS), 0, c.cur, ids,
                        (const DBox *)c.d_boxes, gv, 1, nw);
     HIPCHK(hipGetLastError());
     return AFGPU_OK;

@@ -294,169 +294,6 @@ __device__ inline void face_pos(int nb, int a, int b, int pn, int *p) {
   p[d] = pn;
 }
 
-// Corner (2D) / edge + corner (3D) ghost cells (af_gc_box_corner :125-170,
-// af_edge_gc_extrap :885-924, af_corner_gc_extrap :860-879).
-__constant__ int c_edge_dim3[12] = {0, 0, 0, 0, 1, 1, 1, 1, 2, 2, 2, 2};
-__constant__ int c_edge_dir3[12][3] = {{0, -1, -1}, {0, 1, -1}, {0, -1, 1}, {0, 1, 1},
-                                       {-1, 0, -1}, {1, 0, -1}, {-1, 0, 1}, {1, 0, 1},
-                                       {-1, -1, 0}, {1, -1, 0}, {-1, 1, 0}, {1, 1, 0}};
-
-template <int D, int NC, typename T>
-__device__ inline void gc_edge_cell(const DBox &bx, T *var, int id, int n, int qq) {
-  using G = Geo<D, NC>;
-  using L = Lay<D, NC, T>;
-  T *u = var + (size_t)(id - 1) * L::STRIDE;
-  const int dim = c_edge_dim3[n];
-  const int *dir = c_edge_dir3[n];
-  int lo[3];
-  for (int dd = 0; dd < 3; dd++) lo[dd] = (dir[dd] > 0) ? NC + 1 : 0;
-  lo[dim] = qq;
-  const int nb_id = bx.nbmat[nbmat_at<D>(dir[0], dir[1], dir[2])];
-  if (nb_id > 0) {
-    const T *w = var + (size_t)(nb_id - 1) * L::STRIDE;
-    u[L::at(lo[0], lo[1], lo[2])] = w[L::at(lo[0] - dir[0] * NC, lo[1] - dir[1] * NC, lo[2] - dir[2] * NC)];
-  } else {
-    const int o0 = (dim + 1) % 3, o1 = (dim + 2) % 3;
-    int di[3];
-    for (int dd = 0; dd < 3; dd++) di[dd] = 1 - 2 * (lo[dd] & 1);
-    di[dim] = 0;
-    int ia[3] = {lo[0], lo[1], lo[2]}, ib[3] = {lo[0], lo[1], lo[2]};
-    ia[o0] += di[o0];
-    ib[o1] += di[o1];
-    u[L::at(lo[0], lo[1], lo[2])] = u[L::at(ia[0], ia[1], ia[2])] + u[L::at(ib[0], ib[1], ib[2])] -
-                                     u[L::at(lo[0] + di[0], lo[1] + di[1], lo[2] + di[2])];
-  }
-}
-
-template <int D, int NC, typename T>
-__device__ inline void gc_corner_cell(const DBox &bx, T *var, int id, int n) {
-  using G = Geo<D, NC>;
-  using L = Lay<D, NC, T>;
-  T *u = var + (size_t)(id - 1) * L::STRIDE;
-  const int cx = n & 1, cy = (n >> 1) & 1, cz = (n >> 2) & 1;
-  const int dnb[3] = {2 * cx - 1, 2 * cy - 1, (D == 3) ? 2 * cz - 1 : 0};
-  const int lo[3] = {cx * (NC + 1), cy * (NC + 1), (D == 3) ? cz * (NC + 1) : 0};
-  const int nb_id = bx.nbmat[nbmat_at<D>(dnb[0], dnb[1], dnb[2])];
-  if (nb_id > 0) {
-    const T *w = var + (size_t)(nb_id - 1) * L::STRIDE;
-    u[L::at(lo[0], lo[1], lo[2])] = w[L::at(lo[0] - dnb[0] * NC, lo[1] - dnb[1] * NC, lo[2] - dnb[2] * NC)];
-  } else if (D == 2) {
-    const int di = 1 - 2 * (lo[0] & 1), dj = 1 - 2 * (lo[1] & 1);
-    u[L::at(lo[0], lo[1], 0)] =
-        u[L::at(lo[0] + di, lo[1], 0)] + u[L::at(lo[0], lo[1] + dj, 0)] - u[L::at(lo[0] + di, lo[1] + dj, 0)];
-  } else {
-    const int di = 1 - 2 * (lo[0] & 1), dj = 1 - 2 * (lo[1] & 1), dk = 1 - 2 * (lo[2] & 1);
-    const int x = lo[0], y = lo[1], z = lo[2];
-    u[L::at(x, y, z)] = u[L::at(x, y + dj, z + dk)] + u[L::at(x + di, y, z + dk)] +
-                         u[L::at(x + di, y + dj, z)] - 2 * u[L::at(x + di, y + dj, z + dk)];
-  }
-}
-
-// af_gc_box for all boxes of a list.  Corners need the face ghosts of the
-// same box, so with corners the box must be handled by one workgroup
-// (bpb = 1); face-only fills may be split over several workgroups.
-template <int D, int NC, int BS, typename T, int BB = 1>
-__global__ void __launch_bounds__(BS * BB) k_gc(const int *__restrict__ ids, const DBox *__restrict__ boxes, T *var,
-                                                VarBc m, int corners, int bpb, int nw) {
-  using G = Geo<D, NC>;
-  using L = Lay<D, NC, T>;
-  for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
-    const Part pt = part_of<BS>(ids, bpb, w);
-    if (pt.id <= 0) continue;  // run masked out
-    const int id = pt.id;
-    const DBox &bx = boxes[id - 1];
-    T *u = var + (size_t)(id - 1) * L::STRIDE;
-    constexpr int NFC = 2 * D * G::NTAN;
-    for (int q = pt.q0; q < NFC; q += pt.stride) {
-      const int nb = q / G::NTAN, r = q % G::NTAN;
-      const int a = r % NC + 1, b = (D == 3) ? r / NC + 1 : 0;
-      const bool low = (nb % 2) == 0;
-      int p[3];
-      face_pos<D>(nb, a, b, low ? 1 : NC, p);
-      const T x1 = u[L::at(p[0], p[1], p[2])];
-      face_pos<D>(nb, a, b, low ? 2 : NC - 1, p);
-      const T x2 = u[L::at(p[0], p[1], p[2])];
-      const T g = ghost_value<D, NC, T>(boxes, bx, var, m, nb, a, b, x1, x2);
-      face_pos<D>(nb, a, b, low ? 0 : NC + 1, p);
-      u[L::at(p[0], p[1], p[2])] = g;
-    }
-    if (!corners) continue;
-    gsync<BS, BB>();
-    if (D == 3) {
-      for (int q = ltid<BS>(); q < 12 * NC; q += BS) gc_edge_cell<D, NC, T>(bx, var, id, q / NC, q % NC + 1);
-      gsync<BS, BB>();
-    }
-    for (int q = ltid<BS>(); q < (1 << D); q += BS) gc_corner_cell<D, NC, T>(bx, var, id, q);
-  }
-}
-
-// Red-black Gauss-Seidel half-sweep (stencil_gsrb_357,
-// m_af_stencil.f90:838-998) fused with the ghost-cell fill that the
-// reference performs before it (gsrb_boxes, m_af_multigrid.f90:648-687):
-// a neighbour outside the box is taken from ghost_value() with the same
-// inputs af_gc_box would use, so the updated cells are bit-identical while
-// no separate ghost-fill pass is needed between half-sweeps.  (The stored
-// ghost layer is refreshed once after the last half-sweep.)  stored: the
-// first half-sweep of a V-cycle's finest level reads the stored layer as
-// the reference does, also where it is out of date (the neighbours of boxes
-// just added or removed by refinement).
-template <int D, int NC, int BS, typename T, int BB = 1>
-__global__ void __launch_bounds__(BS * BB) k_gsrb(const int *__restrict__ ids, const DBox *__restrict__ boxes, T *phi,
-                                                  const T *__restrict__ rhs, int redblack, T lambda2, int cyl, VarBc m,
-                                                  int stored, int bpb, int nw) {
-  using G = Geo<D, NC>;
-  using L = Lay<D, NC, T>;
-  for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
-    const Part pt = part_of<BS>(ids, bpb, w);
-    if (pt.id <= 0) continue;  // run masked out
-    const int id = pt.id;
-    const DBox &bx = boxes[id - 1];
-    const Sten<D, T> s = lpl_stencil<D, T>(bx, lambda2);
-    T *u = phi + (size_t)(id - 1) * L::STRIDE;
-    const T *r = rhs + (size_t)(id - 1) * L::STRIDE;
-    constexpr int HALF = G::NINT / 2;
-    for (int q = pt.q0; q < HALF; q += pt.stride) {
-      const int mm = q % (NC / 2);
-      const int j = (q / (NC / 2)) % NC + 1;
-      const int k = (D == 3) ? q / ((NC / 2) * NC) + 1 : 0;
-      const int i0 = 2 - ((redblack ^ (D == 3 ? k + j : j)) & 1);
-      const int i = i0 + 2 * mm;
-      const int x = L::in_at(i, j, k);
-      const int pos[3] = {i, j, k};
-      T nbv[6];
-      for (int nb = 0; nb < 2 * D; nb++) {
-        const int d = nb / 2;
-        const bool low = (nb % 2) == 0;
-        const bool edge = low ? pos[d] == 1 : pos[d] == NC;
-        if (!edge || (stored && !L::SPLIT)) {
-          nbv[nb] = u[L::nb_at(i, j, k, d, low ? -1 : 1)];
-        } else {
-          int t0, t1;
-          tangential(D, d, t0, t1);
-          const T x2 = u[L::nb_at(i, j, k, d, low ? 1 : -1)];
-          nbv[nb] = ghost_value<D, NC, T>(boxes, bx, phi, m, nb, pos[t0], (D == 3) ? pos[t1] : 0, u[x], x2);
-        }
-      }
-      if (D == 2) {
-        if (cyl) {
-          T c1, c2, c3;
-          cyl_coeffs<T>(bx, i, s.c, c1, c2, c3);
-          T inv1 = T(1) / c1;
-          u[x] = (r[x] - c2 * nbv[0] - c3 * nbv[1] - s.c[3] * nbv[2] - s.c[4] * nbv[3]) * inv1;
-        } else {
-          T inv_c1 = T(1) / s.c[0];
-          u[x] = (r[x] - s.c[1] * nbv[0] - s.c[2] * nbv[1] - s.c[3] * nbv[2] - s.c[4] * nbv[3]) * inv_c1;
-        }
-      } else {
-        T inv_c1 = T(1) / s.c[0];
-        u[x] = (r[x] - s.c[1] * nbv[0] - s.c[2] * nbv[1] - s.c[3] * nbv[2] - s.c[4] * nbv[3] - s.c[5] * nbv[4] -
-                s.c[6] * nbv[5]) *
-               inv_c1;
-      }
-    }
-  }
-}
-
 // tmp = rhs - L phi on interior cells (residual_box, m_af_multigrid.f90:801-810);
 // for leaf boxes the max |tmp| is also reduced into *leafmax
 // (af_tree_maxabs_cc, afivo/src/m_af_utils.f90:773).
@@ -1313,7 +1150,17 @@ struct Stage {
   }
 };
 
-// k_gsrb with the box staged in LDS (levels with one workgroup per box).
+// Red-black Gauss-Seidel half-sweep (stencil_gsrb_357,
+// m_af_stencil.f90:838-998) fused with the ghost-cell fill that the
+// reference performs before it (gsrb_boxes, m_af_multigrid.f90:648-687):
+// a neighbour outside the box is taken from ghost_value() with the same
+// inputs af_gc_box would use, so the updated cells are bit-identical while
+// no separate ghost-fill pass is needed between half-sweeps.  (The stored
+// ghost layer is refreshed once after the last half-sweep.)  stored: the
+// first half-sweep of a V-cycle's finest level reads the stored layer as
+// the reference does, also where it is out of date (the neighbours of boxes
+// just added or removed by refinement).
+// One workgroup (or, for 8^2 boxes, wavefront) per box, the box in LDS.
 template <int D, int NC, int BS, typename T, int BB = 1>
 __global__ void __launch_bounds__(BS * BB) k_gsrb_lds(const int *__restrict__ ids, const DBox *__restrict__ boxes,
                                                       T *phi, const T *__restrict__ rhs, int redblack, T lambda2,
@@ -1846,7 +1693,7 @@ __global__ void __launch_bounds__(BS * BB) k_restrict_residual_lds(const int *__
 // block-Jacobi sweep), which lets every workgroup read `in` while writing
 // `out`; physical and refinement-boundary ghosts depend on the box's own
 // cells and are formed again before every half-sweep.  Inside the box the
-// half-sweeps are exactly those of k_gsrb.
+// half-sweeps are exactly those of k_gsrb_lds.
 template <int D, int NC, int BS, typename T>
 __global__ void __launch_bounds__(BS) k_smooth_block(const int *__restrict__ ids, const DBox *__restrict__ boxes,
                                                      const T *in, T *out, const T *__restrict__ rhs,
@@ -1960,89 +1807,178 @@ __global__ void __launch_bounds__(BS * BB) k_mp_correct_leaves(const int *__rest
   }
 }
 
-// af_gc_box with the box staged in LDS: face ghosts as Stage forms them,
-// then (with corners) the edge and corner ghosts of gc_edge_cell /
-// gc_corner_cell from the LDS values, then only the ghost layer is written.
-// One workgroup per box.
+// af_gc_box (afivo/src/m_af_ghostcell.f90:49-170): the face ghosts of a box
+// and, with corners, its edge (3D) and corner ghosts (af_gc_box_corner
+// :125-170, af_edge_gc_extrap :885-924, af_corner_gc_extrap :860-879), by one
+// group of BS threads.  Only what the ghosts need is read: one value per face
+// ghost (the neighbour's cell, or the box's own first one), on boxes at a
+// boundary the second cells and the coarse patches too, and one value per
+// edge or corner cell (the diagonal neighbour's, or the box's own cell next
+// to it); all loads are in flight together.  Bound by that chain (record ->
+// cells -> store), and on large levels by the scattered words of the faces
+// along x.  Staging the whole box first took 9.5 us for 8 FP64 boxes of 16^3
+// (now 5.2), 16.4 us for 768 (14.2), 5.2 us for 64 boxes of 8^3 (4.1), and
+// 37 us a launch over the FP32 levels of 21 million 2D cells (31).
+template <int D, int NC>
+struct GcGeo {
+  static constexpr int NTAN = Geo<D, NC>::NTAN;
+  static constexpr int NFC = 2 * D * NTAN;                    // face ghosts
+  static constexpr int NED = (D == 3) ? 12 * NC : 0;          // edge cells
+  static constexpr int NX = NED + (1 << D);                   // and corners
+};
 template <int D, int NC, int BS, typename T, int BB>
-__device__ inline void gc_lds_box(T *s, T *cp, const DBox *__restrict__ boxes, int id, T *var, const VarBc &m,
-                                  int corners) {
+__device__ inline void gc_box(T *sf, T *cp, const DBox *__restrict__ boxes, int id, T *var, const VarBc &m,
+                              int corners) {
   using G = Geo<D, NC>;
   using L = Lay<D, NC, T>;
+  using GG = GcGeo<D, NC>;
+  using P = CoarsePatch<D, NC>;
+  constexpr int NTAN = G::NTAN, NF = (GG::NFC + BS - 1) / BS, NPT = 2 * D * P::N, NP = (NPT + BS - 1) / BS;
+  static_assert(GG::NX <= BS, "an edge or corner cell per thread");
   const DBox &bx = boxes[id - 1];
   T *u = var + (size_t)(id - 1) * L::STRIDE;
-  Stage<D, NC, BS, T, BB, false> sg;
-  sg.issue(bx, id, var, m, 0);
-  sg.commit(s, cp, bx, m);
+  const int tid = ltid<BS>();
+  // the thread's edge or corner cell: its direction and position
+  int dir[3] = {0, 0, 0}, lo[3] = {0, 0, 0}, dim = -1, nbe = 0;
   if (corners) {
-    if (D == 3) {
-      for (int q = ltid<BS>(); q < 12 * NC; q += BS) {
-        const int n = q / NC, qq = q % NC + 1;
-        const int dim = c_edge_dim3[n];
-        const int *dir = c_edge_dir3[n];
-        int lo[3];
-        for (int dd = 0; dd < 3; dd++) lo[dd] = (dir[dd] > 0) ? NC + 1 : 0;
-        lo[dim] = qq;
-        const int nb_id = bx.nbmat[nbmat_at<D>(dir[0], dir[1], dir[2])];
-        T v;
-        if (nb_id > 0) {
-          const T *w = var + (size_t)(nb_id - 1) * L::STRIDE;
-          v = w[L::in_at(lo[0] - dir[0] * NC, lo[1] - dir[1] * NC, lo[2] - dir[2] * NC)];
-        } else {
-          const int o0 = (dim + 1) % 3, o1 = (dim + 2) % 3;
-          int di[3];
-          for (int dd = 0; dd < 3; dd++) di[dd] = 1 - 2 * (lo[dd] & 1);
-          di[dim] = 0;
-          int ia[3] = {lo[0], lo[1], lo[2]}, ib[3] = {lo[0], lo[1], lo[2]};
-          ia[o0] += di[o0];
-          ib[o1] += di[o1];
-          v = s[G::idx(ia[0], ia[1], ia[2])] + s[G::idx(ib[0], ib[1], ib[2])] -
-              s[G::idx(lo[0] + di[0], lo[1] + di[1], lo[2] + di[2])];
-        }
-        s[G::idx(lo[0], lo[1], lo[2])] = v;
+    const int e = min(tid, GG::NX - 1);
+    const bool edge = e < GG::NED;
+    const int n = edge ? e / NC : e - GG::NED;
+    if (edge) dim = n >> 2;
+    int bit = 0;
+#pragma unroll
+    for (int d = 0; d < D; d++) {
+      const bool along = d == dim;
+      const int up = (n >> bit) & 1;
+      dir[d] = along ? 0 : 2 * up - 1;
+      lo[d] = along ? e % NC + 1 : up ? NC + 1 : 0;
+      if (!along) bit++;
+    }
+    nbe = bx.nbmat[nbmat_at<D>(dir[0], dir[1], dir[2])];
+  }
+  int nbid[2 * D];
+  bool any_rb = false, any_b = false;
+#pragma unroll
+  for (int nb = 0; nb < 2 * D; nb++) {
+    nbid[nb] = __builtin_amdgcn_readfirstlane(bx.nb[nb]);
+    any_b = any_b || nbid[nb] <= 0;
+    any_rb = any_rb || nbid[nb] == 0;
+  }
+  auto item = [&](int t, int &nb, int &a, int &b) {
+    int q = tid + t * BS;
+    if (GG::NFC % BS) q = min(q, GG::NFC - 1);
+    nb = q / NTAN;
+    a = q % NC + 1;
+    b = (D == 3) ? (q % NTAN) / NC + 1 : 0;
+  };
+  T vf[NF], v2[NF], vp[NP];
+#pragma unroll
+  for (int t = 0; t < NF; t++) {
+    int nb, a, b, i, j, k;
+    item(t, nb, a, b);
+    const int nbv = pick<2 * D>(nbid, nb);
+    const bool low = (nb & 1) == 0, copy = nbv > 0;
+    face_cell<D>(nb, a, b, (copy == low) ? NC : 1, i, j, k);
+    vf[t] = (var + (size_t)((copy ? nbv : id) - 1) * L::STRIDE)[L::in_at(i, j, k)];
+  }
+  T ve = T(0);
+  if (corners) {
+    const int w = nbe > 0 ? NC : 1;
+    ve = (var + (size_t)((nbe > 0 ? nbe : id) - 1) * L::STRIDE)[L::in_at(lo[0] - dir[0] * w, lo[1] - dir[1] * w,
+                                                                         lo[2] - dir[2] * w)];
+  }
+  double run_val = 0.0;
+  if (any_b) {
+#pragma unroll
+    for (int t = 0; t < NF; t++) {
+      int nb, a, b, i, j, k;
+      item(t, nb, a, b);
+      face_cell<D>(nb, a, b, (nb & 1) ? NC - 1 : 2, i, j, k);
+      v2[t] = u[L::in_at(i, j, k)];
+    }
+    if (any_rb) {
+      int co[3];
+#pragma unroll
+      for (int d = 0; d < D; d++) co[d] = ((bx.ix[d] - 1) & 1) * (NC / 2);
+#pragma unroll
+      for (int t = 0; t < NP; t++) {
+        const int q = min(tid + t * BS, NPT - 1);
+        const int nb = q / P::N, e = q % P::N, d = nb >> 1;
+        const bool rb = pick<2 * D>(nbid, nb) == 0;
+        const int c0 = (d == 0) ? co[1] : co[0], c1 = (D == 2) ? 0 : (d == 2) ? co[1] : co[2];
+        int i, j, k;
+        face_cell<D>(nb, c0 + e % P::PP, (D == 3) ? c1 + e / P::PP : 0, (nb & 1) ? 1 : NC, i, j, k);
+        const T *from = rb ? var + (size_t)(pick<2 * D>(bx.pnb, nb) - 1) * L::STRIDE + L::at(i, j, k) : u;
+        vp[t] = *from;
+      }
+#pragma unroll
+      for (int t = 0; t < NP; t++) {
+        const int q = tid + t * BS;
+        if (q < NPT) cp[q] = vp[t];
       }
       gsync<BS, BB>();
     }
-    for (int n = ltid<BS>(); n < (1 << D); n += BS) {
-      const int cx = n & 1, cy = (n >> 1) & 1, cz = (n >> 2) & 1;
-      const int dnb[3] = {2 * cx - 1, 2 * cy - 1, (D == 3) ? 2 * cz - 1 : 0};
-      const int lo[3] = {cx * (NC + 1), cy * (NC + 1), (D == 3) ? cz * (NC + 1) : 0};
-      const int nb_id = bx.nbmat[nbmat_at<D>(dnb[0], dnb[1], dnb[2])];
-      T v;
-      if (nb_id > 0) {
-        const T *w = var + (size_t)(nb_id - 1) * L::STRIDE;
-        v = w[L::in_at(lo[0] - dnb[0] * NC, lo[1] - dnb[1] * NC, lo[2] - dnb[2] * NC)];
-      } else if (D == 2) {
-        const int di = 1 - 2 * (lo[0] & 1), dj = 1 - 2 * (lo[1] & 1);
-        v = s[G::idx(lo[0] + di, lo[1], 0)] + s[G::idx(lo[0], lo[1] + dj, 0)] - s[G::idx(lo[0] + di, lo[1] + dj, 0)];
-      } else {
-        const int di = 1 - 2 * (lo[0] & 1), dj = 1 - 2 * (lo[1] & 1), dk = 1 - 2 * (lo[2] & 1);
-        const int x = lo[0], y = lo[1], z = lo[2];
-        v = s[G::idx(x, y + dj, z + dk)] + s[G::idx(x + di, y, z + dk)] + s[G::idx(x + di, y + dj, z)] -
-            2 * s[G::idx(x + di, y + dj, z + dk)];
-      }
-      s[G::idx(lo[0], lo[1], lo[2])] = v;
+    run_val = m.run_val ? m.run_val[bx.run] : 0.0;
+#pragma unroll
+    for (int t = 0; t < NF; t++) {
+      int nb, a, b;
+      item(t, nb, a, b);
+      const int nbv = pick<2 * D>(nbid, nb);
+      if (nbv <= 0) vf[t] = staged_ghost<D, NC, T>(bx, m, run_val, nbv, nb, a, b, cp + nb * P::N, vf[t], v2[t]);
     }
-    gsync<BS, BB>();
   }
-  // the ghost layer back: faces, and with corners the edges and corners
-  for (int x = ltid<BS>(); x < G::NCELL; x += BS) {
-    const int i = x % G::NG, j = (x / G::NG) % G::NG, k = (D == 3) ? x / (G::NG * G::NG) : 0;
-    const int out = (i == 0 || i == NC + 1) + (j == 0 || j == NC + 1) + (D == 3 && (k == 0 || k == NC + 1));
-    if (out == 1 || (corners && out > 1)) u[L::at(i, j, k)] = s[x];
+#pragma unroll
+  for (int t = 0; t < NF; t++) {
+    const int q = tid + t * BS;
+    if (GG::NFC % BS && q >= GG::NFC) continue;
+    int nb, a, b, i, j, k;
+    item(t, nb, a, b);
+    face_cell<D>(nb, a, b, (nb & 1) ? NC + 1 : 0, i, j, k);
+    u[L::at(i, j, k)] = vf[t];
+    if (corners) sf[q] = vf[t];
+  }
+  if (!corners) {
+    if (any_rb) gsync<BS, BB>();  // (cp is reused by the group's next item)
+    return;
+  }
+  gsync<BS, BB>();
+  if (tid < GG::NX) {
+    // the face ghost next to the cell along axis d: at p, behind the face of
+    // axis f
+    auto ghost = [&](int f, int p0, int p1, int p2) {
+      const int df = (f == 0) ? dir[0] : (f == 1) ? dir[1] : dir[2];
+      const int a = (f == 0) ? p1 : p0, b = (D == 2) ? 1 : (f == 2) ? p1 : p2;
+      return sf[(2 * f + (df > 0)) * NTAN + (a - 1) + NC * (b - 1)];
+    };
+    const int x = lo[0], y = lo[1], z = lo[2], xi = x - dir[0], yi = y - dir[1], zi = z - dir[2];
+    if (nbe <= 0) {
+      if (D == 2) {
+        ve = ghost(1, xi, y, 0) + ghost(0, x, yi, 0) - ve;
+      } else if (dim >= 0) {
+        // moved inwards along axis dim + 1 (behind the face of axis
+        // dim + 2), then along axis dim + 2
+        const int o0 = (dim == 2) ? 0 : dim + 1, o1 = (dim == 0) ? 2 : dim - 1;
+        const T g0 = ghost(o1, o0 == 0 ? xi : x, o0 == 1 ? yi : y, o0 == 2 ? zi : z);
+        const T g1 = ghost(o0, o1 == 0 ? xi : x, o1 == 1 ? yi : y, o1 == 2 ? zi : z);
+        ve = g0 + g1 - ve;
+      } else {
+        ve = ghost(0, x, yi, zi) + ghost(1, xi, y, zi) + ghost(2, xi, yi, z) - 2 * ve;
+      }
+    }
+    u[L::at(x, y, z)] = ve;
   }
   gsync<BS, BB>();  // (the group's LDS is reused by its next item)
 }
 template <int D, int NC, int BS, typename T, int BB = 1>
-__global__ void __launch_bounds__(BS * BB) k_gc_lds(const int *__restrict__ ids, const DBox *__restrict__ boxes, T *var,
+__global__ void __launch_bounds__(BS * BB) k_gc(const int *__restrict__ ids, const DBox *__restrict__ boxes, T *var,
                                                     VarBc m, int corners, int nw) {
-  __shared__ T s_all[BB][Geo<D, NC>::NCELL];
+  __shared__ T s_all[BB][GcGeo<D, NC>::NFC];
   __shared__ T cp_all[BB][2 * D * CoarsePatch<D, NC>::N];
   T *s = s_all[lgrp<BS, BB>()], *cp = cp_all[lgrp<BS, BB>()];
   for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
     const int id = __builtin_amdgcn_readfirstlane(ids[w]);
     if (id <= 0) continue;  // run masked out
-    gc_lds_box<D, NC, BS, T, BB>(s, cp, boxes, id, var, m, corners);
+    gc_box<D, NC, BS, T, BB>(s, cp, boxes, id, var, m, corners);
   }
 }
 
@@ -2055,14 +1991,14 @@ struct GcVars {
   int n;
 };
 template <int D, int NC, int BS>
-__global__ void __launch_bounds__(BS) k_gc_lds_vars(const int *__restrict__ ids, const DBox *__restrict__ boxes,
+__global__ void __launch_bounds__(BS) k_gc_vars(const int *__restrict__ ids, const DBox *__restrict__ boxes,
                                                     GcVars vars, int corners, int nw) {
-  __shared__ double s[Geo<D, NC>::NCELL];
+  __shared__ double s[GcGeo<D, NC>::NFC];
   __shared__ double cp[2 * D * CoarsePatch<D, NC>::N];
   for (int w = blockIdx.x; w < nw; w += gridDim.x) {
     const int id = ids[w / vars.n];
     if (id <= 0) continue;
-    gc_lds_box<D, NC, BS, double, 1>(s, cp, boxes, id, vars.v[w % vars.n], vars.m[w % vars.n], corners);
+    gc_box<D, NC, BS, double, 1>(s, cp, boxes, id, vars.v[w % vars.n], vars.m[w % vars.n], corners);
   }
 }
 

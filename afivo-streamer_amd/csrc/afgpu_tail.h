@@ -228,7 +228,7 @@ __global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs A) {
 
   // Edges (3D) and corners of a level's boxes, the faces being filled: the
   // diagonal neighbour's cell, or extrapolated from the face ghosts and the
-  // box's own cells (gc_edge_cell, gc_corner_cell).
+  // box's own cells (as gc_box forms them).
   auto corners = [&](int o, int n_box) {
     for (int q = tid; q < n_box * NX; q += TAIL_NT) {
       const unsigned w = s_cr[o * NX + q];
