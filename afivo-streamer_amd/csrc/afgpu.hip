@@ -250,7 +250,7 @@ struct afgpu_ctx {
   bool photoi_inner_vcycle = false;  // photoionization inner cycle: V-cycle instead of FMG
   bool flux32 = true;  // mixed precision: FP32 flux stencil (FP64 accumulation)
   bool box_lds = false;  // mixed precision, 3D 16^3 boxes: whole boxes staged in LDS by the half-sweeps
-  bool fuse_direct = false;  // uniform-level solve: last-axis transforms fused into one pass
+  bool fuse_direct = false;  // AFGPU_OPT_FUSE_DIRECT (the last axis runs as one pass either way)
   bool direct_f32 = false;   // uniform-level solve of the FP32 inner cycle in FP32 (else FP64; matrix cores)
   bool direct_fold = true;   // uniform-level solve: reflection-symmetric axes transformed by parity (half the products)
   // refinement flags: the boxes evaluated and their flags (device)
@@ -291,8 +291,10 @@ struct afgpu_ctx {
       bool ok = false;
       double *vinv = nullptr, *v = nullptr, *vinvT = nullptr, *vT = nullptr, *eig = nullptr;
       float *vinv32 = nullptr, *v32 = nullptr, *eig32 = nullptr;  // (rounded copies)
-      // parity-folded factors (k_lc_mfma FOLD): per axis N x N/2 forward,
-      // N/2 x N backward, the eigenvalues in the folded modes' order
+      // matrix-core operands (lc_pack): V^-1 and V per axis; parity-folded
+      // ones (k_lc_x, k_lc_line FOLD): N x N/2 forward, N/2 x N backward, the
+      // eigenvalues in the folded modes' order
+      double *vinv_p = nullptr, *v_p = nullptr;
       bool fold[3] = {false, false, false};
       double *mf = nullptr, *bf = nullptr, *eigf = nullptr;
     } f[1 + AFGPU_MAX_MODES];
@@ -1369,11 +1371,28 @@ struct Impl : ImplBase {
         }
       f.fold[dd] = true;
     }
-    double **dst[8] = {&f.vinv, &f.v, &f.vinvT, &f.vT, &f.eig, &f.mf, &f.bf, &f.eigf};
-    const std::vector<double> *srcs[8] = {&vinv, &v, &vinvT, &vT, &eig, &mf, &bf, &eigf};
-    for (int q = 0; q < 8; q++) {
+    // the matrix-core transforms' operands, packed axis by axis
+    std::vector<double> vinv_p, v_p, mf_p, bf_p;
+    if (lc_mfma_size(N)) {
+      auto pack = [&](std::vector<double> &to, const std::vector<double> &m, int rows, int cols) {
+        for (int dd = 0; dd < D; dd++) {
+          const std::vector<double> p = lc_pack(m.data() + (size_t)dd * rows * cols, rows, cols);
+          to.insert(to.end(), p.begin(), p.end());
+        }
+      };
+      pack(vinv_p, vinv, N, N);
+      pack(v_p, v, N, N);
+      if (N == 128) {
+        pack(mf_p, mf, N, H);
+        pack(bf_p, bf, H, N);
+      }
+    }
+    double **dst[10] = {&f.vinv, &f.v, &f.vinvT, &f.vT, &f.eig, &f.mf, &f.bf, &f.eigf, &f.vinv_p, &f.v_p};
+    const std::vector<double> *srcs[10] = {&vinv, &v, &vinvT, &vT, &eig, &mf_p, &bf_p, &eigf, &vinv_p, &v_p};
+    for (int q = 0; q < 10; q++) {
       (void)hipFree(*dst[q]);
       *dst[q] = nullptr;
+      if (srcs[q]->empty()) continue;
       HIPCHK(hipMalloc(dst[q], srcs[q]->size() * sizeof(double)));
       HIPCHK(hipMemcpy(*dst[q], srcs[q]->data(), srcs[q]->size() * sizeof(double), hipMemcpyHostToDevice));
     }
@@ -1390,18 +1409,83 @@ struct Impl : ImplBase {
     return AFGPU_OK;
   }
 
-  // The transforms of the uniform-level solve on the grids A0 / A1 (the
-  // level gathered into A0; *result: the grid holding the result).  On the matrix cores
-  // with a box pool given (rhs_pool, phi_pool), the first x transform reads
-  // the level's rhs from the pool and the last writes phi to it (gather and
-  // scatter fused), and the last forward transform, the division and the
-  // first backward one run as one pass when that pass has a workgroup per
-  // CU at least.
-  // wavefronts per 64 x 64 tile of the matrix-core transforms
-  static constexpr int LC_WAVES = 8;
+  // The transforms of the uniform-level solve on the matrix cores (32, 64 or
+  // 128 cells per axis): the first x transform reads the level's rhs from
+  // the pool, the last writes phi to it; the last axis' two transforms and
+  // the division run as one pass, in place.  The grids of all runs are
+  // transformed together: the x rows of every run, and the y lines with the
+  // run as the remaining coordinate.
+  static bool lc_mfma_size(int n) { return n == 32 || n == 64 || n == 128; }
   template <int N, typename T>
+  int direct_mfma(const afgpu_ctx::Direct::F &f, double lambda2, double *A0, double *A1, const T *rhs_pool,
+                  T *phi_pool) {
+    const int batch = (D == 3) ? N : c.n_runs;
+    const int rows = (D == 3) ? N * N : N * c.n_runs;
+    const int nb = N / NC, *map = c.dir.d_map;
+    const T *noin = nullptr;
+    T *noout = nullptr;
+    const double *nogrid = nullptr;
+    double *nog = nullptr;
+    // the eigenvalues in the order of the (folded) modes
+    const bool folding = c.direct_fold && (f.fold[0] || f.fold[1] || (D == 3 && f.fold[2]));
+    const double *eig = folding ? f.eigf : f.eig;
+    auto mats = [&](int axis, bool fold, const double **mf, const double **mb) {
+      const size_t o = (size_t)axis * N * N;
+      *mf = fold ? f.mf + o / 2 : f.vinv_p + o;
+      *mb = fold ? f.bf + o / 2 : f.v_p + o;
+    };
+    auto with_fold = [&](int axis, auto go) {
+      if constexpr (N == 128)
+        if (c.direct_fold && f.fold[axis]) return go(std::true_type());
+      return go(std::false_type());
+    };
+    auto x = [&](auto IO) {
+      return with_fold(0, [&](auto F) {
+        constexpr bool fold = decltype(F)::value;
+        constexpr int io = decltype(IO)::value;
+        constexpr int BT = LcGeo<N, fold>::BT;
+        const int row_blocks = rows / LcGeo<N, fold>::C;
+        const double *mf, *mb;
+        mats(0, fold, &mf, &mb);
+        if constexpr (io == 1)
+          hipLaunchKernelGGL((k_lc_x<D, N, 1, NC, T, fold>), dim3(row_blocks), dim3(BT), 0, c.cur, nogrid, A0, mf, map,
+                             nb, rhs_pool, noout);
+        else
+          hipLaunchKernelGGL((k_lc_x<D, N, 2, NC, T, fold>), dim3(row_blocks), dim3(BT), 0, c.cur,
+                             (const double *)A0, nog, mb, map, nb, noin, phi_pool);
+        return hipGetLastError();
+      });
+    };
+    auto line = [&](auto DIR, const double *in, double *out, int axis) {
+      return with_fold(axis, [&](auto F) {
+        constexpr bool fold = decltype(F)::value;
+        constexpr int BT = LcGeo<N, fold>::BT;
+        const int line_blocks = N / LcGeo<N, fold>::C * batch;
+        const double *mf, *mb;
+        mats(axis, fold, &mf, &mb);
+        hipLaunchKernelGGL((k_lc_line<D, N, decltype(DIR)::value, fold>), dim3(line_blocks), dim3(BT), 0, c.cur, in,
+                           out, mf, mb, axis, eig, lambda2);
+        return hipGetLastError();
+      });
+    };
+    using std::integral_constant;
+    HIPCHK(x(integral_constant<int, 1>()));
+    if constexpr (D == 3) {
+      HIPCHK(line(integral_constant<int, 1>(), A0, A1, 1));
+      HIPCHK(line(integral_constant<int, 3>(), A1, A1, 2));
+      HIPCHK(line(integral_constant<int, 2>(), A1, A0, 1));
+    } else {
+      HIPCHK(line(integral_constant<int, 3>(), A0, A0, 1));
+    }
+    HIPCHK(x(integral_constant<int, 2>()));
+    return AFGPU_OK;
+  }
+
+  // The same as vector FMA tiles on the level gathered into A0 (other sizes,
+  // or AFGPU_OPT_DIRECT_MFMA 0); *result: the grid holding the result.
+  template <int N>
   int direct_transforms(const afgpu_ctx::Direct::F &f, double lambda2, double *A0, double *A1,
-                        const double **result, const T *rhs_pool = nullptr, T *phi_pool = nullptr) {
+                        const double **result) {
     const size_t NN = (size_t)N * N;
     // the grids of all runs are transformed together: the x rows of every
     // run, and the y lines with the run as the remaining coordinate
@@ -1418,63 +1502,9 @@ struct Impl : ImplBase {
     constexpr int NM = TILED ? N : 64;
     const int gemm_row_blocks = (N / 64) * (nrows / 64);
     const int gemm_line_blocks = (N / 64) * (N / 64) * batch;
-    const bool MC = TILED && c.direct_mfma;
-    const int mfma_row_blocks = (N / 64) * (nrows / 64);
-    const int mfma_line_blocks = (N / 64) * (N / 64) * batch;
-    const bool pool = MC && rhs_pool && phi_pool;
-    const int nb = N / NC;
-    const int *map = c.dir.d_map;
-    const int *nomap = nullptr;
-    const T *noin = nullptr;
-    T *noout = nullptr;
-    // parity-folded transforms (FOLD 1 forward, 2 backward) of the axes
-    // that allow them; the eigenvalue sums then follow the folded order
-    const bool folding = MC && NM == 128 && c.direct_fold && (f.fold[0] || f.fold[1] || (D == 3 && f.fold[2]));
-    const double *eigs = folding ? (const double *)f.eigf : (const double *)f.eig;
-    auto rows_fold = [&](const double *in, double *out, int io, int fold) {
-      if constexpr (NM == 128) {
-        const double *Mx = (fold == 1) ? f.mf : f.bf;
-        const int blocks = (fold == 2) ? nrows / 64 : mfma_row_blocks;
-        if (io == 1)
-          hipLaunchKernelGGL((k_lc_mfma<D, NM, true, 1, NC, T, LC_WAVES, 1>), dim3(blocks), dim3(64 * LC_WAVES), 0,
-                             c.cur, in, out, Mx, 0, 0, eigs, lambda2, map, nb, rhs_pool, noout);
-        else if (io == 2)
-          hipLaunchKernelGGL((k_lc_mfma<D, NM, true, 2, NC, T, LC_WAVES, 2>), dim3(blocks), dim3(64 * LC_WAVES), 0,
-                             c.cur, in, out, Mx, 0, 0, eigs, lambda2, map, nb, noin, phi_pool);
-        else if (fold == 1)
-          hipLaunchKernelGGL((k_lc_mfma<D, NM, true, 0, NC, T, LC_WAVES, 1>), dim3(blocks), dim3(64 * LC_WAVES), 0,
-                             c.cur, in, out, Mx, 0, 0, eigs, lambda2, nomap, 0, noin, noout);
-        else
-          hipLaunchKernelGGL((k_lc_mfma<D, NM, true, 0, NC, T, LC_WAVES, 2>), dim3(blocks), dim3(64 * LC_WAVES), 0,
-                             c.cur, in, out, Mx, 0, 0, eigs, lambda2, nomap, 0, noin, noout);
-      }
-      return hipGetLastError();
-    };
-    auto lines_fold = [&](const double *in, double *out, int axis, int div, int fold) {
-      if constexpr (NM == 128) {
-        const double *Mx = ((fold == 1) ? f.mf : f.bf) + (size_t)axis * N * N / 2;
-        const int blocks = (fold == 2) ? mfma_line_blocks / (N / 64) : mfma_line_blocks;
-        if (fold == 1)
-          hipLaunchKernelGGL((k_lc_mfma<D, NM, false, 0, NC, T, LC_WAVES, 1>), dim3(blocks), dim3(64 * LC_WAVES),
-                             0, c.cur, in, out, Mx, axis, div, eigs, lambda2, nomap, 0, noin, noout);
-        else
-          hipLaunchKernelGGL((k_lc_mfma<D, NM, false, 0, NC, T, LC_WAVES, 2>), dim3(blocks), dim3(64 * LC_WAVES),
-                             0, c.cur, in, out, Mx, axis, div, eigs, lambda2, nomap, 0, noin, noout);
-      }
-      return hipGetLastError();
-    };
-    auto rows = [&](const double *in, double *out, const double *Mx, const double *MTx, int io) {
-      if (folding && f.fold[0]) return rows_fold(in, out, io, Mx == f.vinv ? 1 : 2);
-      if (MC && io == 1)
-        hipLaunchKernelGGL((k_lc_mfma<D, NM, true, 1, NC, T, LC_WAVES>), dim3(mfma_row_blocks), dim3(64 * LC_WAVES), 0, c.cur, in, out,
-                           Mx, 0, 0, eigs, lambda2, map, nb, rhs_pool, noout);
-      else if (MC && io == 2)
-        hipLaunchKernelGGL((k_lc_mfma<D, NM, true, 2, NC, T, LC_WAVES>), dim3(mfma_row_blocks), dim3(64 * LC_WAVES), 0, c.cur, in, out,
-                           Mx, 0, 0, eigs, lambda2, map, nb, noin, phi_pool);
-      else if (MC)
-        hipLaunchKernelGGL((k_lc_mfma<D, NM, true, 0, NC, T, LC_WAVES>), dim3(mfma_row_blocks), dim3(64 * LC_WAVES), 0, c.cur, in, out,
-                           Mx, 0, 0, eigs, lambda2, nomap, 0, noin, noout);
-      else if (TILED)
+    const double *eigs = f.eig;
+    auto rows = [&](const double *in, double *out, const double *Mx, const double *MTx) {
+      if (TILED)
         hipLaunchKernelGGL((k_lc_gemm<D, NM, true>), dim3(gemm_row_blocks), dim3(256), 0, c.cur, in, out, Mx, 0, 0,
                            eigs, lambda2);
       else
@@ -1482,11 +1512,7 @@ struct Impl : ImplBase {
       return hipGetLastError();
     };
     auto lines = [&](const double *in, double *out, const double *M, int axis, int div) {
-      if (folding && f.fold[axis]) return lines_fold(in, out, axis, div, M == f.vinv + (size_t)axis * NN ? 1 : 2);
-      if (MC)
-        hipLaunchKernelGGL((k_lc_mfma<D, NM, false, 0, NC, T, LC_WAVES>), dim3(mfma_line_blocks), dim3(64 * LC_WAVES), 0, c.cur, in,
-                           out, M, axis, div, eigs, lambda2, nomap, 0, noin, noout);
-      else if (TILED)
+      if (TILED)
         hipLaunchKernelGGL((k_lc_gemm<D, NM, false>), dim3(gemm_line_blocks), dim3(256), 0, c.cur, in, out, M, axis,
                            div, eigs, lambda2);
       else
@@ -1494,10 +1520,6 @@ struct Impl : ImplBase {
                            eigs, lambda2);
       return hipGetLastError();
     };
-    // the last forward, the division and the first backward transform
-    // along the last axis: one pass, or two
-    const int fused_blocks = (N / 64) * batch;
-    const bool fuse = MC && c.fuse_direct && !folding && fused_blocks >= c.n_cu;
     const int last = D - 1;
     const double *vinv_l = f.vinv + (size_t)last * NN, *v_l = f.v + (size_t)last * NN;
     // ping-pong between the grids: `cur` holds the latest result
@@ -1506,32 +1528,15 @@ struct Impl : ImplBase {
       std::swap(cur, nxt);
       return e;
     };
-    if (pool) {
-      nxt = A1;
-      HIPCHK(step(rows(nullptr, nxt, f.vinv, f.vinvT, 1)));
-    } else {
-      HIPCHK(step(rows(cur, nxt, f.vinv, f.vinvT, 0)));
-    }
+    HIPCHK(step(rows(cur, nxt, f.vinv, f.vinvT)));
     if (D == 3) HIPCHK(step(lines(cur, nxt, f.vinv + NN, 1, 0)));
-    if (fuse) {
-      hipLaunchKernelGGL((k_lc_mfma_fused<D, NM>), dim3(fused_blocks), dim3(4 * NM), 0, c.cur, cur, nxt, vinv_l,
-                         v_l, (const double *)f.eig, lambda2);
-      HIPCHK(step(hipGetLastError()));
-    } else {
-      HIPCHK(step(lines(cur, nxt, vinv_l, last, 1)));
-      HIPCHK(step(lines(cur, nxt, v_l, last, 0)));
-    }
+    HIPCHK(step(lines(cur, nxt, vinv_l, last, 1)));
+    HIPCHK(step(lines(cur, nxt, v_l, last, 0)));
     if (D == 3) HIPCHK(step(lines(cur, nxt, f.v + NN, 1, 0)));
-    if (pool) {
-      HIPCHK(rows(cur, nullptr, f.v, f.vT, 2));
-      *result = nullptr;
-    } else {
-      HIPCHK(step(rows(cur, nxt, f.v, f.vT, 0)));
-      *result = cur;
-    }
+    HIPCHK(step(rows(cur, nxt, f.v, f.vT)));
+    *result = cur;
     return AFGPU_OK;
   }
-
 
   // The transforms of the uniform-level solve in FP32 on the matrix cores
   // (64 or 128 cells per axis): the first x transform reads the rhs from the
@@ -1588,9 +1593,9 @@ struct Impl : ImplBase {
       set_err("uniform-level solve: grids not allocated");
       return AFGPU_ERR_STATE;
     }
-    // on the matrix cores (64 or 128 cells per axis) the transforms read
+    // on the matrix cores (32, 64 or 128 cells per axis) the transforms read
     // the rhs from the pool and write phi to it themselves
-    const bool pool = c.direct_mfma && (d.N == 64 || d.N == 128);
+    const bool pool = c.direct_mfma && lc_mfma_size(d.N);
     if (!pool) {
       hipLaunchKernelGGL((k_lc_gather<D, NC, BS, T>), dim3(nbox), dim3(BS), 0, c.cur, (const int *)d.d_map, nb,
                          (const T *)v.rhs, A0);
@@ -1600,7 +1605,7 @@ struct Impl : ImplBase {
     T *pp = pool ? v.phi : nullptr;
     const double l2 = c.ops[v.op].lambda2;
     if constexpr (std::is_same<T, float>::value) {
-      if (pool && c.direct_f32 && !c.fuse_direct) {
+      if (pool && d.N >= 64 && c.direct_f32 && !c.fuse_direct) {
         float *F0 = (float *)A0, *F1 = (float *)A1;
         if (d.N == 64)
           RCHK(direct_transforms32<64>(f, (float)l2, F0, F1, rp, pp));
@@ -1610,12 +1615,20 @@ struct Impl : ImplBase {
       }
     }
     const double *res = nullptr;
-    switch (d.N) {
-      case 16: RCHK((direct_transforms<16, T>(f, l2, A0, A1, &res))); break;
-      case 32: RCHK((direct_transforms<32, T>(f, l2, A0, A1, &res))); break;
-      case 64: RCHK((direct_transforms<64, T>(f, l2, A0, A1, &res, rp, pp))); break;
-      case 128: RCHK((direct_transforms<128, T>(f, l2, A0, A1, &res, rp, pp))); break;
-      default: set_err("uniform-level solve: unsupported size"); return AFGPU_ERR_UNSUPPORTED;
+    if (pool) {
+      switch (d.N) {
+        case 32: RCHK((direct_mfma<32, T>(f, l2, A0, A1, rp, pp))); break;
+        case 64: RCHK((direct_mfma<64, T>(f, l2, A0, A1, rp, pp))); break;
+        default: RCHK((direct_mfma<128, T>(f, l2, A0, A1, rp, pp))); break;
+      }
+    } else {
+      switch (d.N) {
+        case 16: RCHK((direct_transforms<16>(f, l2, A0, A1, &res))); break;
+        case 32: RCHK((direct_transforms<32>(f, l2, A0, A1, &res))); break;
+        case 64: RCHK((direct_transforms<64>(f, l2, A0, A1, &res))); break;
+        case 128: RCHK((direct_transforms<128>(f, l2, A0, A1, &res))); break;
+        default: set_err("uniform-level solve: unsupported size"); return AFGPU_ERR_UNSUPPORTED;
+      }
     }
     if (!pool) {
       hipLaunchKernelGGL((k_lc_scatter<D, NC, BS, T>), dim3(nbox), dim3(BS), 0, c.cur, (const int *)d.d_map, nb,
@@ -2841,6 +2854,8 @@ int afgpu_destroy(afgpu_t *h) {
     (void)hipFree(f.eig32);
     (void)hipFree(f.mf);
     (void)hipFree(f.bf);
+    (void)hipFree(f.vinv_p);
+    (void)hipFree(f.v_p);
     (void)hipFree(f.eigf);
   }
   (void)hipFree(h->d_boxes);

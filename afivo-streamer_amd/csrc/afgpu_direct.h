@@ -13,6 +13,8 @@
 // transformed back.  All transforms run in FP64.
 #pragma once
 
+#include <vector>
+
 #include "afgpu_common.h"
 
 namespace afg {
@@ -159,7 +161,7 @@ __global__ void __launch_bounds__(256) k_lc_rows(const double *__restrict__ in, 
   }
 }
 
-// The same transforms for N = 64 and 128 as a tiled product
+// The same transforms for N = 64 and 128 as a tiled product (vector FMA)
 //   out(i, col) = sum_m M[i][m] X(m, col)
 // over 64 x 64 output tiles (i0.., col0..): chunks of 16 m are staged in LDS
 // for both M and X (the next chunk is prefetched into registers while the
@@ -267,14 +269,6 @@ __global__ void __launch_bounds__(256) k_lc_gemm(const double *__restrict__ in, 
     }
 }
 
-// The same transforms on the FP64 matrix cores (v_mfma_f64_16x16x4f64):
-//   D[p][q] = sum_k A[p][k] B[k][q]
-// y / z forms: p = output index i, q = column x, A = M, B = the input lines;
-// x form (ROWS): p = grid row r, q = output index i, A = the input rows,
-// B[k][i] = M[i][k].  A workgroup (4 waves) computes a 64 x 64 tile of D,
-// each wave a 32 x 32 block as 2 x 2 MFMA tiles; K runs in chunks of 16
-// staged in LDS.  Lane layout of the instruction: A operand A[l % 16][l / 16],
-// B operand B[l / 16][l % 16], result register j of lane l D[4 j + l / 16][l % 16].
 typedef double lc_double4 __attribute__((ext_vector_type(4)));
 typedef float lc_float4 __attribute__((ext_vector_type(4)));
 
@@ -295,189 +289,300 @@ __device__ inline long long lc_pool_offset(const int *__restrict__ map, int nb, 
   return id > 0 ? (long long)(id - 1) * L::STRIDE + L::in_at(x % NC + 1, y % NC + 1, ck) : -1;
 }
 
-// IO (x form only): 0 grid to grid; 1 the input rows read from the box
-// pool `pin` (the gather, fused); 2 the output rows written to the box pool
-// `pout` (the scatter, fused).  Box map and boxes per axis as k_lc_gather.
-// WAVES wavefronts share a 64 x 64 output tile: two rows of WAVES / 2, each
-// wave 32 x (128 / WAVES) (at 8, two waves per SIMD in every workgroup, for
-// the few workgroups a pass has: (N / 64)^2 N).  Every output element is
-// one wave's sum over K in the same order whatever WAVES is.
+// The transforms on the FP64 matrix cores (v_mfma_f64_16x16x4f64, D = A B on
+// 16 x 16 tiles, K = 4: lane l holds A[l % 16][l / 16], B[l / 16][l % 16] and
+// in register j D[4 j + l / 16][l % 16]).
 //
-// FOLD (N = 128, an axis whose 1-D operator is symmetric under reversal,
-// m -> N - 1 - m): its eigenvectors are even or odd, so a transform needs
-// half the products.  1, forward: M is N x N/2, the even modes' rows first
-// (M[i][m], m < N/2, of the even eigenvectors), then the odd ones'; the
-// even half of the output (the first 64-row tile) takes u_m + u_{N-1-m},
-// the odd half u_m - u_{N-1-m}, over K = N/2.  2, backward: M is N/2 x N,
-// M[m][i] for m < N/2 over the modes in the same order; the sums over the
-// even modes (E) and the odd ones (O) give u_m = E + O and
-// u_{N-1-m} = E - O, one 64-row output tile writing both halves.
-template <int D, int N, bool ROWS, int IO = 0, int NC = 16, typename TS = float, int WAVES = 8, int FOLD = 0>
-__global__ void __launch_bounds__(64 * WAVES) k_lc_mfma(const double *__restrict__ in, double *__restrict__ out,
-                                                        const double *__restrict__ M, int axis, int div,
-                                                        const double *__restrict__ eig, double lambda2,
-                                                        const int *__restrict__ map, int nb,
-                                                        const TS *__restrict__ pin, TS *__restrict__ pout) {
-  static_assert(IO == 0 || ROWS, "box-pool input and output in the x form only");
-  static_assert(N == 64 || N == 128, "matrix-core transform for N = 64, 128");
-  static_assert(WAVES == 4 || WAVES == 8, "4 or 8 wavefronts per 64 x 64 tile");
-  static_assert(FOLD == 0 || N == 128, "the folded form has one 64-row tile per parity");
-  constexpr int BT = 64 * WAVES;
-  constexpr int T = 64, KC = 32, AP = KC + 1, BP = T + 1, NT = N / T;
-  constexpr int NTO = (FOLD == 2) ? 1 : NT;    // output tiles
-  constexpr int KN = (FOLD == 1) ? N / 2 : N;  // K extent
-  constexpr int MS = (FOLD == 1) ? N / 2 : N;  // row stride of M
-  constexpr int NS = (FOLD == 2) ? 2 : 1;      // accumulator sets (E, O)
-  constexpr int PER = T * KC / BT;  // values of each operand tile per thread
-  constexpr int WQ = WAVES / 2, QW = T / WQ, NTB = QW / 16;  // waves along q, their width, 16-wide tiles
-  __shared__ double As[T * AP];   // As[p][kk]
-  __shared__ double Bs[KC * BP];  // Bs[kk][q]
-  // blocks: ROWS: (output tiles) x (row tiles); else (output tiles) x
-  // (column tiles) x (the remaining coordinate)
-  const int t0 = blockIdx.x % NTO, rest = blockIdx.x / NTO;
-  const double sg = (t0 == 0) ? 1.0 : -1.0;  // the fold of the forward form: even, odd half
-  size_t sm = 1, base = 0;
-  int o = 0, x0 = 0, p0 = 0, q0 = 0;
-  if (ROWS) {
-    p0 = rest * T;  // grid rows
-    q0 = t0 * T;    // output index i
-  } else {
-    p0 = t0 * T;  // output index i
-    x0 = (rest % NT) * T;
-    o = rest / NT;
-    q0 = 0;
-    sm = (axis == 1) ? (size_t)N : (size_t)N * N;
-    const size_t so = (D == 2) ? (size_t)N * N : ((axis == 1) ? (size_t)N * N : (size_t)N);
-    base = (size_t)o * so + x0;
+// A workgroup of four or eight wavefronts takes C whole lines along the axis, so that
+// everything it reads (the lines into LDS, its rows of the matrix into
+// registers) is one round of independent loads with one barrier, and the
+// last axis' forward transform, division and backward transform run on the
+// lines while they are in LDS.  The passes are bound by that round and, on a
+// 128^3 level, by the grid's traffic through the caches: 64 x 64 tiles
+// in chunks of 32 along K took six passes and 98 us for 128^3 cells (now
+// five and 71 us), 40 us for 64^3 (21), four passes and 36 us for one run of
+// 128^2 (three, 18), 28 us for 13 runs of 64^2 (12).
+//
+// The matrices are packed in operand order (lc_pack): row tile by row tile,
+// K step by K step, one value per lane.
+//
+// FOLD (an axis whose 1-D operator is symmetric under reversal,
+// m -> N - 1 - m, N = 128): its eigenvectors are even or odd, so a transform
+// needs half the products.  Forward: the even modes (rows 0..N/2 - 1 of the
+// matrix, N x N/2) take u_m + u_{N-1-m}, the odd ones u_m - u_{N-1-m}, over
+// K = N/2.  Backward: the matrix (N/2 x N) gives the sums over the even modes
+// (E) and the odd ones (O), u_m = E + O and u_{N-1-m} = E - O.
+inline std::vector<double> lc_pack(const double *M, int rows, int cols) {
+  std::vector<double> p((size_t)rows * cols);
+  size_t o = 0;
+  for (int rt = 0; rt < rows / 16; rt++)
+    for (int st = 0; st < cols / 4; st++)
+      for (int l = 0; l < 64; l++) p[o++] = M[(size_t)(rt * 16 + l % 16) * cols + 4 * st + l / 16];
+  return p;
+}
+template <int N, bool FOLD>
+struct LcGeo {
+  static constexpr int W = (N == 128 && !FOLD) ? 8 : 4;  // wavefronts of a workgroup
+  static constexpr int NWR = (N / 16 < W) ? N / 16 : W;  // of them along the output index
+  static constexpr int NWC = W / NWR;                    // and along the lines
+  static constexpr int C = 16 * NWC;                     // lines per workgroup
+  static constexpr int RT = N / 16 / NWR;                // 16-row tiles per wavefront
+  static constexpr int BT = 64 * W;
+};
+// A packed 16-row matrix tile over ST steps of K, one value per lane and
+// step in registers: loaded ahead of the barrier that the lines wait for.
+template <int ST>
+struct LcTile {
+  double m[ST];
+  __device__ void load(const double *__restrict__ mp) {
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int st = 0; st < ST; st++) m[st] = mp[st * 64 + lane];
   }
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wp = (w / WQ) * 32, wq = (w % WQ) * QW;
-  // one K chunk of both operands, global -> registers (consecutive threads
-  // take consecutive addresses) and registers -> LDS
-  double pa[PER], pb[PER];
-  auto fetch = [&](int k0) {
-    for (int u = 0; u < PER; u++) {
-      const int q = tid + BT * u;
-      const int pp = q / KC, kk = q % KC;
-      const int k = k0 + kk;
-      if (IO == 1) {
-        const int row = p0 + pp;
-        const long long off = lc_pool_offset<D, NC, TS>(map, nb, k, row % N, row / N);
-        double a = off >= 0 ? (double)pin[off] : 0.0;
-        if (FOLD == 1) {
-          const long long off2 = lc_pool_offset<D, NC, TS>(map, nb, N - 1 - k, row % N, row / N);
-          a = a + sg * (off2 >= 0 ? (double)pin[off2] : 0.0);
-        }
-        pa[u] = a;
-      } else if (ROWS) {
-        const double *r = in + (size_t)(p0 + pp) * N;
-        pa[u] = (FOLD == 1) ? r[k] + sg * r[N - 1 - k] : r[k];
-      } else {
-        pa[u] = M[(size_t)(p0 + pp) * MS + k];
-      }
-      if (ROWS) {
-        pb[u] = M[(size_t)(q0 + pp) * MS + k];
-      } else {
-        const int kb = q / T, qq = q % T;
-        const double *c = in + base + qq;
-        pb[u] = (FOLD == 1) ? c[(size_t)(k0 + kb) * sm] + sg * c[(size_t)(N - 1 - k0 - kb) * sm]
-                            : c[(size_t)(k0 + kb) * sm];
-      }
-    }
-  };
-  auto stash = [&]() {
-    for (int u = 0; u < PER; u++) {
-      const int q = tid + BT * u;
-      As[(q / KC) * AP + q % KC] = pa[u];
-      if (ROWS)
-        Bs[(q % KC) * BP + q / KC] = pb[u];
-      else
-        Bs[(q / T) * BP + q % T] = pb[u];
-    }
-  };
-  lc_double4 acc[NS][2][NTB];
-  for (int e = 0; e < NS; e++)
-    for (int a = 0; a < 2; a++)
-      for (int b = 0; b < NTB; b++) acc[e][a][b] = lc_double4{0.0, 0.0, 0.0, 0.0};
-  fetch(0);
-  for (int k0 = 0; k0 < KN; k0 += KC) {
-    stash();
-    __syncthreads();
-    if (k0 + KC < KN) fetch(k0 + KC);
-    const int e = (NS == 2 && k0 >= N / 2) ? 1 : 0;  // (the backward form: the odd modes' sum)
-    for (int ks = 0; ks < KC; ks += 4) {
-      const int kk = ks + (lane >> 4);
-      double a[2], b[NTB];
-      for (int t = 0; t < 2; t++) a[t] = As[(wp + 16 * t + (lane & 15)) * AP + kk];
-      for (int t = 0; t < NTB; t++) b[t] = Bs[kk * BP + wq + 16 * t + (lane & 15)];
-      for (int ta = 0; ta < 2; ta++)
-        for (int tb = 0; tb < NTB; tb++) {
-          if (NS == 2 && e == 1)
-            acc[NS - 1][ta][tb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ta], b[tb], acc[NS - 1][ta][tb], 0, 0, 0);
-          else
-            acc[0][ta][tb] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[ta], b[tb], acc[0][ta][tb], 0, 0, 0);
-        }
-    }
-    __syncthreads();
+};
+// One product of a wavefront over steps S0 .. S0 + ST - 1 of the tile, the
+// other operand from LDS, at step s at xs[s * step].
+template <int S0, int ST, bool ROWS, int TST>
+__device__ inline lc_double4 lc_product(const LcTile<TST> &mt, const double *xs, int step) {
+  lc_double4 acc = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+  for (int st = 0; st < ST; st++) {
+    const double x = xs[st * step];
+    acc = ROWS ? __builtin_amdgcn_mfma_f64_16x16x4f64(x, mt.m[S0 + st], acc, 0, 0, 0)
+               : __builtin_amdgcn_mfma_f64_16x16x4f64(mt.m[S0 + st], x, acc, 0, 0, 0);
   }
-  for (int ta = 0; ta < 2; ta++)
-    for (int tb = 0; tb < NTB; tb++)
-      for (int j = 0; j < 4; j++) {
-        const int pp = p0 + wp + 16 * ta + 4 * j + (lane >> 4);
-        const int qq = q0 + wq + 16 * tb + (lane & 15);
-        if (FOLD == 2) {
-          // u_m = E + O, u_{N-1-m} = E - O; m is qq (ROWS) or pp (lines)
-          const double vE = acc[0][ta][tb][j], vO = acc[NS - 1][ta][tb][j];
-          const double lo = vE + vO, hi = vE - vO;
-          if (ROWS && IO == 2) {
-            long long off = lc_pool_offset<D, NC, TS>(map, nb, qq, pp % N, pp / N);
-            if (off >= 0) pout[off] = (TS)lo;
-            off = lc_pool_offset<D, NC, TS>(map, nb, N - 1 - qq, pp % N, pp / N);
-            if (off >= 0) pout[off] = (TS)hi;
-          } else if (ROWS) {
-            out[(size_t)pp * N + qq] = lo;
-            out[(size_t)pp * N + N - 1 - qq] = hi;
-          } else {
-            out[base + (size_t)pp * sm + qq] = lo;
-            out[base + (size_t)(N - 1 - pp) * sm + qq] = hi;
-          }
-          continue;
-        }
-        double v = acc[0][ta][tb][j];
-        if (ROWS && IO == 2) {
-          const long long off = lc_pool_offset<D, NC, TS>(map, nb, qq, pp % N, pp / N);
-          if (off >= 0) pout[off] = (TS)v;
-        } else if (ROWS) {
-          out[(size_t)pp * N + qq] = v;
-        } else {
-          if (div) {
-            const int x = x0 + qq;
-            int y, z;
-            if (D == 2) {
-              y = pp;
-              z = 0;
-            } else if (axis == 1) {
-              y = pp;
-              z = o;
-            } else {
-              y = o;
-              z = pp;
-            }
-            double den = eig[x] + eig[N + y];
-            if (D == 3) den = den + eig[2 * N + z];
-            den = den - lambda2;
-            v = v / den;
-          }
-          out[base + (size_t)pp * sm + qq] = v;
-        }
-      }
+  return acc;
 }
 
-// k_lc_mfma in single precision (the mixed form's inner cycle, option
-// AFGPU_OPT_DIRECT_F32): grids, matrices and eigenvalues in FP32, products
-// on the FP32 matrix cores (v_mfma_f32_16x16x4f32: the operands as in the
-// FP64 form, result register j of lane l holding row 4 (l / 16) + j,
-// column l % 16 of the 16 x 16 block).
+// The x transforms: IO 1 forward, the rows read from the box pool `pin`;
+// IO 2 backward, the result written to the box pool `pout`.
+template <int D, int N, int IO, int NC, typename TS, bool FOLD>
+__global__ void __launch_bounds__((LcGeo<N, FOLD>::BT), 4) k_lc_x(const double *__restrict__ in, double *__restrict__ out,
+                                              const double *__restrict__ M, const int *__restrict__ map, int nb,
+                                              const TS *__restrict__ pin, TS *__restrict__ pout) {
+  using LG = LcGeo<N, FOLD>;
+  constexpr int C = LG::C, S = N + 4;  // (row stride: 16 rows and 4 steps of K over all LDS banks)
+  constexpr int H = N / 2, PER = C * N / LG::BT;
+  __shared__ double xs[C * S];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wr = w % LG::NWR, wc = w / LG::NWR;
+  const int r0 = blockIdx.x * C;  // first grid row
+  // a wavefront's row tiles (folded backward: one tile over E and O)
+  constexpr int RT = (IO == 2 && FOLD) ? 1 : LG::RT, KS = (IO == 1 && FOLD ? H : N) / 4;
+  constexpr int EARLY = (KS * RT <= 32) ? RT : 1;  // (tiles held in registers from the start)
+  const double *mw = M + (size_t)wr * RT * KS * 64;
+  LcTile<KS> mt[EARLY];
+  // The rows lie on one plane z (or in one run), in the boxes yb = 0 ..
+  // C / NC - 1 from the first row's on: where column x begins in box yb
+  // (negative: masked out), and cell (x, row) from there on.
+  using L = Lay<D, NC, TS>;
+  const int z = r0 / N, y0 = r0 % N, kz = (D == 3) ? z % NC + 1 : 0;
+  auto box_at = [&](int x, int yb) {
+    const int b = x / NC + nb * (y0 / NC + yb) + ((D == 3) ? nb * nb * (z / NC) : nb * nb * z);
+    const int id = map[b];
+    return id > 0 ? (long long)(id - 1) * L::STRIDE : -1ll;
+  };
+  auto in_box = [&](int x, int r) { return L::in_at(x % NC + 1, r % NC + 1, kz); };
+  if constexpr (IO == 1) {
+    // RU rows per step of the loads: the box of a step's rows is known
+    constexpr int RU = LG::BT / (FOLD ? H : N), YB = C / NC;
+    static_assert(RU <= NC && NC % RU == 0 && C % NC == 0, "a step's rows lie in one box");
+    const int xa = tid % (FOLD ? H : N);
+    long long ba[YB], bb[YB];
+#pragma unroll
+    for (int yb = 0; yb < YB; yb++) {
+      ba[yb] = box_at(xa, yb);
+      if (FOLD) bb[yb] = box_at(N - 1 - xa, yb);
+    }
+    auto val = [&](long long base, int x, int r) { return base >= 0 ? (double)pin[base + in_box(x, r)] : 0.0; };
+    if constexpr (FOLD) {
+      double a[PER / 2], b[PER / 2];
+#pragma unroll
+      for (int u = 0; u < PER / 2; u++) {
+        const int r = (tid + u * LG::BT) / H;
+        a[u] = val(ba[u * RU / NC], xa, r);
+        b[u] = val(bb[u * RU / NC], N - 1 - xa, r);
+      }
+      for (int t = 0; t < EARLY; t++) mt[t].load(mw + (size_t)t * KS * 64);
+#pragma unroll
+      for (int u = 0; u < PER / 2; u++) {
+        const int q = tid + u * LG::BT, x = q % H, r = q / H;
+        xs[r * S + x] = a[u] + b[u];
+        xs[r * S + H + x] = a[u] - b[u];
+      }
+    } else {
+      double a[PER];
+#pragma unroll
+      for (int u = 0; u < PER; u++) {
+        a[u] = val(ba[u * RU / NC], xa, (tid + u * LG::BT) / N);
+      }
+      for (int t = 0; t < EARLY; t++) mt[t].load(mw + (size_t)t * KS * 64);
+#pragma unroll
+      for (int u = 0; u < PER; u++) {
+        const int q = tid + u * LG::BT;
+        xs[(q / N) * S + q % N] = a[u];
+      }
+    }
+  } else {
+    double a[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) a[u] = in[(size_t)r0 * N + tid + u * LG::BT];
+    for (int t = 0; t < EARLY; t++) mt[t].load(mw + (size_t)t * KS * 64);
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+      const int q = tid + u * LG::BT;
+      xs[(q / N) * S + q % N] = a[u];
+    }
+  }
+  __syncthreads();
+  const double *x0 = xs + (16 * wc + (lane & 15)) * S + (lane >> 4);
+  if constexpr (IO == 2 && FOLD) {
+    // output tile m = 16 wr .. of the first half, and its mirror
+    const lc_double4 E = lc_product<0, H / 4, true>(mt[0], x0, 4);
+    const lc_double4 O = lc_product<H / 4, H / 4, true>(mt[0], x0 + H, 4);
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int r = 16 * wc + 4 * j + (lane >> 4), m = 16 * wr + (lane & 15), yb = (16 * wc + 4 * j) / NC;
+      const long long lo = box_at(m, yb), hi = box_at(N - 1 - m, yb);
+      if (lo >= 0) pout[lo + in_box(m, r)] = (TS)(E[j] + O[j]);
+      if (hi >= 0) pout[hi + in_box(N - 1 - m, r)] = (TS)(E[j] - O[j]);
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < RT; t++) {
+      const int rt = wr * RT + t;  // (folded: the first half of the row tiles are the even modes)
+      const double *xt = x0 + (FOLD && rt >= N / 32 ? H : 0);
+      if (t >= EARLY) mt[0].load(mw + (size_t)t * KS * 64);
+      const lc_double4 v = lc_product<0, KS, true>(mt[t < EARLY ? t : 0], xt, 4);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int r = 16 * wc + 4 * j + (lane >> 4), m = 16 * rt + (lane & 15);
+        if constexpr (IO == 2) {
+          const long long base = box_at(m, (16 * wc + 4 * j) / NC);
+          if (base >= 0) pout[base + in_box(m, r)] = (TS)v[j];
+        } else {
+          out[(size_t)(r0 + r) * N + m] = v[j];
+        }
+      }
+    }
+  }
+}
+
+// The transforms along y and z: DIR 1 forward (Mf), 2 backward (Mb), 3 the
+// last axis: forward, division by the eigenvalue sums and backward.  A
+// workgroup takes C neighbouring columns x at one value o of the remaining
+// coordinate (z for the y axis, y for the z axis; the run in 2D).
+template <int D, int N, int DIR, bool FOLD>
+__global__ void __launch_bounds__((LcGeo<N, FOLD>::BT), 4) k_lc_line(const double *__restrict__ in, double *__restrict__ out,
+                                                 const double *__restrict__ Mf, const double *__restrict__ Mb, int axis,
+                                                 const double *__restrict__ eig, double lambda2) {
+  using LG = LcGeo<N, FOLD>;
+  constexpr int C = LG::C, H = N / 2, PER = C * N / LG::BT, NXC = N / C;
+  __shared__ double xs[N * C];
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+  const int wr = w % LG::NWR, wc = w / LG::NWR;
+  const int x0 = (blockIdx.x % NXC) * C, o = blockIdx.x / NXC;
+  const size_t sm = (axis == 1) ? (size_t)N : (size_t)N * N;
+  const size_t so = (D == 2) ? (size_t)N * N : ((axis == 1) ? (size_t)N * N : (size_t)N);
+  const size_t base = (size_t)o * so + x0;
+  // a wavefront's row tiles, forward and (folded: one tile over E and O) backward
+  constexpr int RT = LG::RT, KS = (FOLD ? H : N) / 4, RB = FOLD ? 1 : RT, KB = N / 4;
+  constexpr int EF = (KS * RT <= 32) ? RT : 1, EB = (KB * RB <= 32) ? RB : 1;  // (tiles held from the start)
+  const double *mfw = Mf + (size_t)wr * RT * KS * 64, *mbw = Mb + (size_t)wr * RB * KB * 64;
+  LcTile<KS> mf[EF];
+  LcTile<KB> mb[EB];
+  auto early = [&] {
+    if constexpr (DIR & 1)
+      for (int t = 0; t < EF; t++) mf[t].load(mfw + (size_t)t * KS * 64);
+    else
+      for (int t = 0; t < EB; t++) mb[t].load(mbw + (size_t)t * KB * 64);
+  };
+  if constexpr (FOLD && (DIR & 1)) {
+    double a[PER / 2], b[PER / 2];
+#pragma unroll
+    for (int u = 0; u < PER / 2; u++) {
+      const int q = tid + u * LG::BT, k = q / C, c = q % C;
+      a[u] = in[base + (size_t)k * sm + c];
+      b[u] = in[base + (size_t)(N - 1 - k) * sm + c];
+    }
+    early();
+#pragma unroll
+    for (int u = 0; u < PER / 2; u++) {
+      const int q = tid + u * LG::BT;
+      xs[q] = a[u] + b[u];
+      xs[H * C + q] = a[u] - b[u];
+    }
+  } else {
+    double a[PER];
+#pragma unroll
+    for (int u = 0; u < PER; u++) {
+      const int q = tid + u * LG::BT;
+      a[u] = in[base + (size_t)(q / C) * sm + q % C];
+    }
+    early();
+#pragma unroll
+    for (int u = 0; u < PER; u++) xs[tid + u * LG::BT] = a[u];
+  }
+  __syncthreads();
+  const int col = 16 * wc + (lane & 15);
+  const double *b0 = xs + (lane >> 4) * C + col;
+  if constexpr (DIR & 1) {
+    lc_double4 v[RT];
+#pragma unroll
+    for (int t = 0; t < RT; t++) {
+      if (t >= EF) mf[0].load(mfw + (size_t)t * KS * 64);
+      v[t] = lc_product<0, KS, false>(mf[t < EF ? t : 0], b0 + (FOLD && wr * RT + t >= N / 32 ? H * C : 0), 4 * C);
+    }
+    if constexpr (DIR == 3) {
+      for (int t = 0; t < EB; t++) mb[t].load(mbw + (size_t)t * KB * 64);
+      __syncthreads();  // (every wavefront is done with the lines)
+    }
+#pragma unroll
+    for (int t = 0; t < RT; t++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int p = 16 * (wr * RT + t) + 4 * j + (lane >> 4);
+        if constexpr (DIR == 3) {
+          double den = eig[x0 + col] + eig[N + ((D == 3) ? o : p)];
+          if (D == 3) den = den + eig[2 * N + p];
+          den = den - lambda2;
+          xs[p * C + col] = v[t][j] / den;
+        } else {
+          out[base + (size_t)p * sm + col] = v[t][j];
+        }
+      }
+    if constexpr (DIR == 1) return;
+    __syncthreads();
+  }
+  if constexpr (DIR & 2) {
+    if constexpr (FOLD) {
+      const lc_double4 E = lc_product<0, H / 4, false>(mb[0], b0, 4 * C);
+      const lc_double4 O = lc_product<H / 4, H / 4, false>(mb[0], b0 + H * C, 4 * C);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        const int p = 16 * wr + 4 * j + (lane >> 4);
+        out[base + (size_t)p * sm + col] = E[j] + O[j];
+        out[base + (size_t)(N - 1 - p) * sm + col] = E[j] - O[j];
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < RB; t++) {
+        if (t >= EB) mb[0].load(mbw + (size_t)t * KB * 64);
+        const lc_double4 v = lc_product<0, KB, false>(mb[t < EB ? t : 0], b0, 4 * C);
+#pragma unroll
+        for (int j = 0; j < 4; j++) out[base + (size_t)(16 * (wr * RB + t) + 4 * j + (lane >> 4)) * sm + col] = v[j];
+      }
+    }
+  }
+}
+
+// The transforms in single precision (the mixed form's inner cycle, option
+// AFGPU_OPT_DIRECT_F32), 64 x 64 output tiles in chunks of 32 along K: grids,
+// matrices and eigenvalues in FP32, products on the FP32 matrix cores
+// (v_mfma_f32_16x16x4f32: the operands as in the FP64 form, result register
+// j of lane l holding row 4 (l / 16) + j, column l % 16 of the 16 x 16
+// block).  ROWS: D[p][q], p = grid row, q = output index (IO 1: the rows read
+// from the box pool, 2: written to it); else p = output index, q = column x.
 template <int D, int N, bool ROWS, int IO = 0, int NC = 16>
 __global__ void __launch_bounds__(256) k_lc_mfma32(const float *__restrict__ in, float *__restrict__ out,
                                                    const float *__restrict__ M, int axis, int div,
@@ -594,71 +699,6 @@ __global__ void __launch_bounds__(256) k_lc_mfma32(const float *__restrict__ in,
           }
           out[base + (size_t)pp * sm + qq] = v;
         }
-      }
-}
-
-// The last forward transform (z in 3D, y in 2D), the division by the
-// eigenvalue sums and the first backward transform along the same lines, in
-// one pass: a workgroup (N/16 waves) holds all N points of a 64-column tile
-// of lines in LDS, forms D1 = Mf B on the matrix cores, divides, keeps D1 in
-// LDS and forms D2 = Mb D1 (each product with the K order of k_lc_mfma).
-// One read and one write of the grid instead of two of each.
-template <int D, int N>
-__global__ void __launch_bounds__(4 * N) k_lc_mfma_fused(const double *__restrict__ in, double *__restrict__ out,
-                                                         const double *__restrict__ Mf, const double *__restrict__ Mb,
-                                                         const double *__restrict__ eig, double lambda2) {
-  static_assert(N == 64 || N == 128, "matrix-core transform for N = 64, 128");
-  constexpr int T = 64, KC = 32, AP = KC + 1, BP = T + 1, NT = N / T, NTH = 4 * N;
-  __shared__ double Bs[N * BP];   // the lines Bs[k][q], then D1
-  __shared__ double As[N * AP];   // one K chunk of the matrix, As[p][kk]
-  const int xt = blockIdx.x % NT, o = blockIdx.x / NT;  // o: y in 3D, the run in 2D
-  const int x0 = xt * T;
-  const size_t sm = (D == 3) ? (size_t)N * N : (size_t)N;  // stride along the lines
-  const size_t so = (D == 3) ? (size_t)N : (size_t)N * N;  // stride of o
-  const size_t base = (size_t)o * so + x0;
-  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int wp = (w >> 1) * 32, wq = (w & 1) * 32;
-  for (int q = tid; q < N * T; q += NTH) Bs[(q / T) * BP + q % T] = in[base + (size_t)(q / T) * sm + q % T];
-  lc_double4 acc[2][2];
-  auto product = [&](const double *__restrict__ M) {
-    for (int a = 0; a < 2; a++)
-      for (int b = 0; b < 2; b++) acc[a][b] = lc_double4{0.0, 0.0, 0.0, 0.0};
-    for (int k0 = 0; k0 < N; k0 += KC) {
-      __syncthreads();  // (the chunk and, before the first, the lines in LDS)
-      for (int q = tid; q < N * KC; q += NTH) As[(q / KC) * AP + q % KC] = M[(size_t)(q / KC) * N + k0 + q % KC];
-      __syncthreads();
-      for (int ks = 0; ks < KC; ks += 4) {
-        const int kk = ks + (lane >> 4);
-        double av[2], bv[2];
-        for (int t = 0; t < 2; t++) {
-          av[t] = As[(wp + 16 * t + (lane & 15)) * AP + kk];
-          bv[t] = Bs[(k0 + kk) * BP + wq + 16 * t + (lane & 15)];
-        }
-        for (int ta = 0; ta < 2; ta++)
-          for (int tb = 0; tb < 2; tb++)
-            acc[ta][tb] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[ta], bv[tb], acc[ta][tb], 0, 0, 0);
-      }
-    }
-  };
-  product(Mf);
-  __syncthreads();  // every wave is done with the lines
-  for (int ta = 0; ta < 2; ta++)
-    for (int tb = 0; tb < 2; tb++)
-      for (int j = 0; j < 4; j++) {
-        const int pp = wp + 16 * ta + 4 * j + (lane >> 4);  // position along the lines
-        const int qq = wq + 16 * tb + (lane & 15);
-        double den = eig[x0 + qq] + eig[N + ((D == 3) ? o : pp)];
-        if (D == 3) den = den + eig[2 * N + pp];
-        den = den - lambda2;
-        Bs[pp * BP + qq] = acc[ta][tb][j] / den;
-      }
-  product(Mb);
-  for (int ta = 0; ta < 2; ta++)
-    for (int tb = 0; tb < 2; tb++)
-      for (int j = 0; j < 4; j++) {
-        const int pp = wp + 16 * ta + 4 * j + (lane >> 4);
-        const int qq = wq + 16 * tb + (lane & 15);
-        out[base + (size_t)pp * sm + qq] = acc[ta][tb][j];
       }
 }
 

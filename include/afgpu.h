@@ -411,10 +411,10 @@ int afgpu_kernel_stats(afgpu_t *h, int kind, int reset, double *total_ms,
                                   captured graph with the stopping tests on the device (1), or
                                   one captured graph per cycle with the tests on the host (0);
                                   the results are identical (default 0, measured faster) */
-#define AFGPU_OPT_FUSE_DIRECT 10 /* mixed precision: the uniform-level solve's last forward
-                                    transform, division and first backward transform as one pass
-                                    (1) or two (0); identical results (default 0: the one pass,
-                                    at one 100 KB-LDS workgroup per CU, measured slower) */
+#define AFGPU_OPT_FUSE_DIRECT 10 /* mixed precision: 1 keeps the uniform-level solve in FP64
+                                    whatever AFGPU_OPT_DIRECT_F32 says; its last forward
+                                    transform, division and first backward transform run as one
+                                    pass either way (default 0) */
 #define AFGPU_OPT_DIRECT_F32 11 /* mixed precision: the uniform-level solve of the FP32 inner
                                    cycle on the matrix cores (64 or 128 cells per axis) in FP32
                                    (1) or FP64 (0); the FP64 outer correction sets the accuracy
@@ -429,7 +429,7 @@ int afgpu_kernel_stats(afgpu_t *h, int kind, int reset, double *total_ms,
                                    axes whose 1-D operator is symmetric under reversal (the same
                                    boundary condition at both ends, Cartesian) split the modes by
                                    parity: half the products; results differ in rounding only
-                                   (default 1; AFGPU_OPT_FUSE_DIRECT applies with it off) */
+                                   (default 1) */
 int afgpu_set_option(afgpu_t *h, int option, int value);
 
 /* ---- ensembles of independent runs --------------------------------------
