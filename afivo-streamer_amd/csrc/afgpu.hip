@@ -896,6 +896,13 @@ struct Impl : ImplBase {
           continue;
         }
       }
+      if constexpr (D == 3 && Lay<D, NC, T>::SPLIT && NC == 8) {
+        if (!c.box_lds) {
+          RCHK((items_nt<256, 1>(0, bytes, KC_GSRB, k_gsrb_row3d<NC>, (l.n + 31) / 32 * 8, c.list(l),
+                                 (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, n, v.lambda2, v.m, l.n)));
+          continue;
+        }
+      }
       if constexpr (D == 3 && Lay<D, NC, T>::SPLIT && BS == NC * NC) {
         if (!c.box_lds) {
           RCHK((items_nt<GSRB_SPLIT_NT, 1>(0, bytes, KC_GSRB, k_gsrb_split<D, NC, GSRB_SPLIT_NT>, l.n, c.list(l),

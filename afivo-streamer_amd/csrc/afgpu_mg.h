@@ -1588,6 +1588,131 @@ __global__ void __launch_bounds__(256) k_gsrb_split2d(const int *__restrict__ id
   }
 }
 
+// k_gsrb_lds for 3D boxes of 8^3 cells in the colour-split single-precision
+// layout.  A wavefront takes a box, a lane one row (j, k) of the updated
+// colour (four cells, one 16-byte word): it loads its row's word of the other
+// colour and of the rhs, the row's x ghost (the neighbour's cell across the
+// face on the side of the row's first or last updated cell), and each of half
+// the lanes one word of a y or z face (the neighbour's facing row of the other
+// colour, which is the four ghosts).  On a face without a same-level
+// neighbour the box's own cells next to it take the ghosts' place, and at a
+// refinement boundary the coarse patches are loaded too; those ghosts are
+// formed after the words are in LDS.  The y and z neighbours come from the
+// other lanes' words.  The ghost and stencil expressions and their operands
+// are those of k_gsrb_lds, so the results are identical.
+// Four boxes per workgroup, dealt so that a workgroup's boxes come from the
+// range of the list that its XCD works through (the list is ordered for one
+// box per workgroup).
+// Bound by its chain (record -> words -> LDS) on small levels and by the
+// neighbours' scattered face words on large ones: 4096 boxes take 7.3 us
+// (k_gsrb_lds: 11.9), 1024 boxes 5.2 (5.3).
+template <int NC>
+__global__ void __launch_bounds__(256) k_gsrb_row3d(const int *__restrict__ ids, const DBox *__restrict__ boxes,
+                                                    float *phi, const float *__restrict__ rhs, int redblack,
+                                                    float lambda2, VarBc m, int n_boxes, int nw) {
+  constexpr int D = 3;
+  using L = Lay<D, NC, float>;
+  using P = CoarsePatch<D, NC>;
+  constexpr int HALF = L::HALF, NPT = 2 * D * P::N, NP = (NPT + 63) / 64;
+  static_assert(NC == 8 && HALF == 256 && (L::STRIDE * sizeof(float)) % 16 == 0, "8^3 boxes: a row is one word");
+  __shared__ float4 s_o_all[4][64];  // other colour, row (j, k) at lane (j - 1) + 8 (k - 1)
+  __shared__ float4 s_f_all[4][32];  // ghosts of the faces 2 .. 5, eight rows each
+  __shared__ float s_cp_all[4][NPT];
+  const int wv = lgrp<64, 4>(), lane = threadIdx.x & 63;
+  float4 *s_o = s_o_all[wv], *s_f = s_f_all[wv];
+  float *s_cp = s_cp_all[wv];
+  const int uc = redblack & 1, oc = 1 - uc;  // updated cells: (i + j + k + redblack) even
+  const int j = (lane & 7) + 1, k = (lane >> 3) + 1, i0 = 1 + ((1 + j + k + uc) & 1);
+  const int nbx = (i0 == 1) ? 0 : 1;  // the x face of the row's ghost
+  // the y or z face row of this lane (lanes 0 .. 31): face nbf, row e
+  const int nbf = 2 + ((lane >> 3) & 3), e = lane & 7, pd = (nbf & 1) ? NC : 1;
+  auto row_of = [&](int p) { return nbf < 4 ? (p - 1) + NC * e : e + NC * (p - 1); };
+  for (int w = blockIdx.x; w < nw; w += gridDim.x) {
+    const int q = ((w >> 3) * 4 + wv) * 8 + (w & 7);
+    const int id = q < n_boxes ? __builtin_amdgcn_readfirstlane(ids[q]) : 0;
+    if (id <= 0) continue;  // (past the end, or a run masked out)
+    const DBox &bx = boxes[id - 1];
+    float *u = phi + (size_t)(id - 1) * L::STRIDE;
+    int nbid[2 * D];
+    bool any_rb = false, any_b = false;
+#pragma unroll
+    for (int nb = 0; nb < 2 * D; nb++) {
+      nbid[nb] = __builtin_amdgcn_readfirstlane(bx.nb[nb]);
+      any_b = any_b || nbid[nb] <= 0;
+      any_rb = any_rb || nbid[nb] == 0;
+    }
+    const int nvx = (nbx == 0) ? nbid[0] : nbid[1], nvf = pick<2 * D>(nbid, nbf);
+    const float4 xc = reinterpret_cast<const float4 *>(u + oc * HALF)[lane];
+    const float4 rv = reinterpret_cast<const float4 *>(rhs + (size_t)(id - 1) * L::STRIDE + uc * HALF)[lane];
+    // x ghost: the neighbour's cell, or the box's own one next to the face
+    float gx = (phi + (size_t)((nvx > 0 ? nvx : id) - 1) * L::STRIDE)[L::in_at((nvx > 0) == (nbx == 0) ? NC : 1, j, k)];
+    float4 fw = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (lane < 32) {
+      const float *from = nvf > 0 ? phi + (size_t)(nvf - 1) * L::STRIDE + oc * HALF : u + uc * HALF;
+      fw = reinterpret_cast<const float4 *>(from)[row_of((nvf > 0) == (pd == 1) ? NC : 1)];
+    }
+    float vp[NP];
+    if (any_rb) {
+      int co[3];
+#pragma unroll
+      for (int d = 0; d < D; d++) co[d] = ((bx.ix[d] - 1) & 1) * (NC / 2);
+#pragma unroll
+      for (int t = 0; t < NP; t++) {
+        const int c = min(lane + t * 64, NPT - 1), nb = c / P::N, r = c % P::N, d = nb >> 1;
+        const bool rb = pick<2 * D>(nbid, nb) == 0;
+        int ci, cj, ck;
+        face_cell<D>(nb, ((d == 0) ? co[1] : co[0]) + r % P::PP, ((d == 2) ? co[1] : co[2]) + r / P::PP,
+                     (nb & 1) ? 1 : NC, ci, cj, ck);
+        vp[t] = *(rb ? phi + (size_t)(pick<2 * D>(bx.pnb, nb) - 1) * L::STRIDE + L::at(ci, cj, ck) : u);
+      }
+    }
+    const Sten<D, float> st = lpl_stencil<D, float>(bx, lambda2);
+    const float inv_c1 = 1.0f / st.c[0];
+    s_o[lane] = xc;
+    if (any_rb)
+#pragma unroll
+      for (int t = 0; t < NP; t++)
+        if (lane + t * 64 < NPT) s_cp[lane + t * 64] = vp[t];
+    gsync<64, 4>();
+    if (any_b) {
+      const double run_val = m.run_val ? m.run_val[bx.run] : 0.0;
+      if (nvx <= 0)
+        gx = staged_ghost<D, NC, float>(bx, m, run_val, nvx, nbx, j, k, s_cp + nbx * P::N, gx, nbx == 0 ? xc.x : xc.w);
+      if (lane < 32 && nvf <= 0) {
+        const float4 o = s_o[row_of(pd == 1 ? 2 : NC - 1)];
+        const int a0 = 1 + ((1 + pd + e + 1 + uc) & 1);
+        auto ghost = [&](int c, float x1, float x2) {
+          return staged_ghost<D, NC, float>(bx, m, run_val, nvf, nbf, a0 + 2 * c, e + 1, s_cp + nbf * P::N, x1, x2);
+        };
+        fw = make_float4(ghost(0, fw.x, o.x), ghost(1, fw.y, o.y), ghost(2, fw.z, o.z), ghost(3, fw.w, o.w));
+      }
+    }
+    if (lane < 32) s_f[lane] = fw;
+    gsync<64, 4>();
+    float xw[5];
+    if (i0 == 1) {
+      xw[0] = gx; xw[1] = xc.x; xw[2] = xc.y; xw[3] = xc.z; xw[4] = xc.w;
+    } else {
+      xw[0] = xc.x; xw[1] = xc.y; xw[2] = xc.z; xw[3] = xc.w; xw[4] = gx;
+    }
+    const float4 ym4 = *((j == 1) ? s_f + (k - 1) : s_o + lane - 1);
+    const float4 yp4 = *((j == NC) ? s_f + 8 + (k - 1) : s_o + lane + 1);
+    const float4 zm4 = *((k == 1) ? s_f + 16 + (j - 1) : s_o + lane - 8);
+    const float4 zp4 = *((k == NC) ? s_f + 24 + (j - 1) : s_o + lane + 8);
+    const float ym[4] = {ym4.x, ym4.y, ym4.z, ym4.w}, yp[4] = {yp4.x, yp4.y, yp4.z, yp4.w};
+    const float zm[4] = {zm4.x, zm4.y, zm4.z, zm4.w}, zp[4] = {zp4.x, zp4.y, zp4.z, zp4.w};
+    const float rr[4] = {rv.x, rv.y, rv.z, rv.w};
+    float res[4];
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+      res[c] = (rr[c] - st.c[1] * xw[c] - st.c[2] * xw[c + 1] - st.c[3] * ym[c] - st.c[4] * yp[c] - st.c[5] * zm[c] -
+                st.c[6] * zp[c]) *
+               inv_c1;
+    reinterpret_cast<float4 *>(u + uc * HALF)[lane] = make_float4(res[0], res[1], res[2], res[3]);
+    gsync<64, 4>();  // (the wavefront's LDS is reused by its next box)
+  }
+}
+
 // k_mp_residual with the box staged in LDS.
 template <int D, int NC, int BS, int BB = 1>
 __global__ void __launch_bounds__(BS * BB) k_mp_residual_lds(const int *__restrict__ ids,
