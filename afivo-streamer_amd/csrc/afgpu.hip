@@ -598,12 +598,13 @@ struct Impl : ImplBase {
   }
   // A list kernel (template argument BB) over nw work items, in the shape of
   // its class; the item count is the kernel's last argument.
-  template <int BB, typename K, typename... Args>
+  // (NT: threads per workgroup where they are not BS per box)
+  template <int BB, int NT = BS * BB, typename K, typename... Args>
   int items(int cls, K kernel, int nw, Args... args) {
-    if (c.class_timing && c.timing && !c.capture_pairs) return items_timed<BB>(3 + cls, 0.0, cls, kernel, nw, args...);
+    if (c.class_timing && c.timing && !c.capture_pairs) return items_nt<NT, BB>(3 + cls, 0.0, cls, kernel, nw, args...);
     if (nw <= 0) return AFGPU_OK;
     RCHK(tail_flush());
-    hipLaunchKernelGGL(kernel, dim3(grid_for(cls, nw, BB)), dim3(BS * BB), 0, c.cur, args..., nw);
+    hipLaunchKernelGGL(kernel, dim3(grid_for(cls, nw, BB)), dim3(NT), 0, c.cur, args..., nw);
     HIPCHK(hipGetLastError());
     return AFGPU_OK;
   }
@@ -780,6 +781,17 @@ struct Impl : ImplBase {
     return AFGPU_OK;
   }
 
+  // Threads per box of the staging kernels on levels of up to one 16^3 box
+  // per CU: four times as many as elsewhere, each with a quarter of the loads.
+  static constexpr int MANY_NT = (D == 3 && NC == 16) ? 1024 : BS;
+  // the restriction keeps its cells' residuals in registers: on 16^3 boxes
+  // 8 (FP32) or 4 (FP64) a thread
+  template <typename T>
+  static constexpr int restrict_nt() {
+    return (D == 3 && NC == 16) ? (sizeof(T) == 8 ? 1024 : 512) : BS;
+  }
+  bool many_threads(int n_boxes) const { return MANY_NT != BS && n_boxes <= c.n_cu; }
+
   // Workgroups per box: 1 on large levels; on levels with few boxes the
   // box's work items are spread over several workgroups.
   static int bpb(int n_boxes, int items) {
@@ -910,13 +922,10 @@ struct Impl : ImplBase {
           continue;
         }
       }
-      if constexpr (D == 3 && NC == 16) {
-        // up to one box per CU: four times the threads on each
-        if (l.n <= c.n_cu) {
-          RCHK((items_nt<1024, 1>(0, bytes, KC_GSRB, k_gsrb_lds<D, NC, 1024, T, 1>, l.n, c.list(l),
-                                  (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, n, v.lambda2, cyl, v.m, stored)));
-          continue;
-        }
+      if (many_threads(l.n)) {
+        RCHK((items_nt<MANY_NT, 1>(0, bytes, KC_GSRB, k_gsrb_lds<D, NC, MANY_NT, T, 1>, l.n, c.list(l),
+                                   (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, n, v.lambda2, cyl, v.m, stored)));
+        continue;
       }
       RCHK(with_bb(KC_GSRB, [&](auto B) {
         constexpr int bb = decltype(B)::value;
@@ -928,43 +937,36 @@ struct Impl : ImplBase {
     return final_gc ? gc_var(lvl, v.phi, v.m, !down) : AFGPU_OK;
   }
 
-  // The single-precision inner cycle restricts with the child box staged in
-  // LDS and its face ghosts formed in-kernel, so it needs no ghost fill
-  // after the down-sweep.  (The FP64 form keeps the reference's fills: its
-  // stored ghost layers are part of the state compared with the oracle.)
+  // The single-precision inner cycle restricts with face ghosts formed
+  // in-kernel, so it needs no ghost fill after the down-sweep.  (The FP64
+  // form keeps the reference's fills: its stored ghost layers are part of
+  // the state compared with the oracle.)
   template <typename T>
-  bool restrict_in_lds(int lvl) const {
-    constexpr int NQ = G::NINT / (1 << D);
-    return std::is_same<T, float>::value && bpb(c.l_ids[lvl].n, NQ) == 1;
+  static constexpr bool restrict_forms_ghosts() {
+    return std::is_same<T, float>::value;
   }
 
   template <typename T>
   int update_coarse(const Mg<T> &v, int lvl, bool v_cycle) {
     const int cyl = c.coord == AFGPU_CYL;
     const List &l = c.l_ids[lvl];
-    constexpr int NQ = G::NINT / (1 << D);
-    const int k = bpb(l.n, NQ);
-    if (restrict_in_lds<T>(lvl)) {
-      RCHK(with_bb(KC_RESTRICT, [&](auto B) {
-        constexpr int bb = decltype(B)::value;
-        return items<bb>(KC_RESTRICT, k_restrict_residual_lds<D, NC, BS, T, bb>, l.n, c.list(l),
-                         (const DBox *)c.d_boxes, (const T *)level_buf(v, lvl, v_cycle), v.phi, (const T *)v.rhs, v.tmp,
-                         v.lambda2, cyl, (int)!v_cycle, v.m);
-      }));
-    } else {
-      // (a forest whose runs end on different levels fills every level: a
-      // run's own finest level needs it, and for the other runs the fill
-      // repeats the one the level above has just made, with the same values)
-      if (!v_cycle && (lvl == c.highest_lvl || c.uneven)) RCHK(gc_var(lvl, v.phi, v.m, true));
-      if (in_tail<T>(lvl))
-        RCHK(tail_push(TL_RESTRICT, lvl, !v_cycle));
-      else
-      RCHK(with_bb(KC_RESTRICT, [&](auto B) {
-        constexpr int bb = decltype(B)::value;
-        return items<bb>(KC_RESTRICT, k_restrict_residual<D, NC, BS, T, bb>, l.n * k, c.list(l),
-                         (const DBox *)c.d_boxes, v.phi, (const T *)v.rhs, v.tmp, v.lambda2, cyl, (int)!v_cycle, k);
-      }));
-    }
+    constexpr bool forms = restrict_forms_ghosts<T>();
+    // (a forest whose runs end on different levels fills every level: a
+    // run's own finest level needs it, and for the other runs the fill
+    // repeats the one the level above has just made, with the same values)
+    if (!forms && !v_cycle && (lvl == c.highest_lvl || c.uneven)) RCHK(gc_var(lvl, v.phi, v.m, true));
+    auto restricted = [&](auto NT, auto B) {
+      constexpr int nt = decltype(NT)::value, bb = decltype(B)::value;
+      return items<bb, nt * bb>(KC_RESTRICT, k_restrict_residual<D, NC, nt, T, bb>, l.n, c.list(l),
+                                (const DBox *)c.d_boxes, (const T *)level_buf(v, lvl, v_cycle), v.phi,
+                                (const T *)v.rhs, v.tmp, v.lambda2, cyl, (int)!v_cycle, v.m, (int)!forms);
+    };
+    if (in_tail<T>(lvl))
+      RCHK(tail_push(TL_RESTRICT, lvl, !v_cycle));
+    else if (many_threads(l.n))
+      RCHK(restricted(std::integral_constant<int, MANY_NT>(), std::integral_constant<int, 1>()));
+    else
+      RCHK(with_bb(KC_RESTRICT, [&](auto B) { return restricted(std::integral_constant<int, restrict_nt<T>()>(), B); }));
     RCHK(gc_var(lvl - 1, v.phi, v.m, true));
     if (in_tail<T>(lvl - 1)) return tail_push(TL_RHS, lvl - 1, v_cycle);
     const List &pl = c.l_parents[lvl - 1];
@@ -1053,7 +1055,7 @@ struct Impl : ImplBase {
   template <typename T>
   int vcycle_body(const Mg<T> &v, bool set_residual, int max_lvl, int lc = 1, bool standalone = false) {
     for (int lvl = max_lvl; lvl >= lc + 1; lvl--) {
-      RCHK(gsrb_boxes(v, lvl, true, !restrict_in_lds<T>(lvl), standalone && lvl == max_lvl));
+      RCHK(gsrb_boxes(v, lvl, true, !restrict_forms_ghosts<T>(), standalone && lvl == max_lvl));
       RCHK(update_coarse(v, lvl, true));
     }
     if (lc == 1)

@@ -349,6 +349,13 @@ __host__ __device__ inline void child_pos(int i_f, int jf, int kf, int *pos) {
   }
 }
 
+// Cylindrical weight of a parent cell's restriction.
+template <typename T>
+__device__ inline T restrict_weight(const DBox &bp, int ic) {
+  const T r = (T)bp.r_min[0] + (T(ic) - T(0.5)) * (T)bp.dr[0];
+  return T(0.25) * (T)bp.dr[0] / r;
+}
+
 // Restriction of one parent cell from its 2^D children values
 // (af_restrict_box, afivo/src/m_af_restrict.f90:62-136).
 template <int D, int NC, typename T, typename L = LayStd<D, NC>>
@@ -357,9 +364,8 @@ __device__ inline T restrict_cell(const T *f, int i_f, int jf, int kf, bool cyl_
   child_pos<D, NC, L>(i_f, jf, kf, p);
   if (D == 2) {
     if (cyl_geom) {
-      T r = (T)bp.r_min[0] + (T(ic) - T(0.5)) * (T)bp.dr[0];
-      T tmp = T(0.25) * (T)bp.dr[0] / r;
-      T w1 = T(1) - tmp, w2 = T(1) + tmp;
+      const T t = restrict_weight<T>(bp, ic);
+      T w1 = T(1) - t, w2 = T(1) + t;
       return T(0.25) * (w1 * (f[p[0]] + f[p[2]]) + w2 * (f[p[1]] + f[p[3]]));
     }
     T s = f[p[0]];
@@ -372,24 +378,6 @@ __device__ inline T restrict_cell(const T *f, int i_f, int jf, int kf, bool cyl_
     for (int c = 1; c < 8; c++) s = s + f[p[c]];
     return T(0.125) * s;
   }
-}
-
-// The same from the children's 2^D values (i fastest, then j, then k).
-template <typename T>
-__device__ inline T restrict_weight(const DBox &bp, int ic) {
-  const T r = (T)bp.r_min[0] + (T(ic) - T(0.5)) * (T)bp.dr[0];
-  return T(0.25) * (T)bp.dr[0] / r;
-}
-template <int D, typename T>
-__device__ inline T restrict_children(const T *rs, bool cyl_geom, const DBox &bp, int ic) {
-  if (D == 2 && cyl_geom) {
-    const T t = restrict_weight<T>(bp, ic);
-    T w1 = T(1) - t, w2 = T(1) + t;
-    return T(0.25) * (w1 * (rs[0] + rs[2]) + w2 * (rs[1] + rs[3]));
-  }
-  T sm = rs[0];
-  for (int c = 1; c < (1 << D); c++) sm = sm + rs[c];
-  return T(1.0 / (1 << D)) * sm;
 }
 
 // Restrict variable `src` of child boxes into `dst` of their parents.
@@ -415,53 +403,6 @@ __global__ void __launch_bounds__(BS * BB) k_restrict(const int *__restrict__ id
       const int ic = off[0] + i, jc = off[1] + j, kc = (D == 3) ? off[2] + k : 0;
       u[L::at(ic, jc, kc)] =
           restrict_cell<D, NC, T, L>(f, 2 * i - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0, cyl && use_geom, bp, ic);
-    }
-  }
-}
-
-// update_coarse, first half (m_af_multigrid.f90:703-716): per child box the
-// residual rhs - L phi is restricted (with geometry) into the parent's tmp
-// and phi (without geometry) into the parent's phi.  The residual is formed
-// on the fly, which leaves the child's tmp untouched exactly as the
-// reference's save/restore of tmp does.  With store_residual the residual is
-// also kept in the child's tmp (set_coarse_phi_rhs, :742-776).
-template <int D, int NC, int BS, typename T, int BB = 1>
-__global__ void __launch_bounds__(BS * BB) k_restrict_residual(const int *__restrict__ ids,
-                                                               const DBox *__restrict__ boxes, T *phi,
-                                                               const T *__restrict__ rhs, T *tmp, T lambda2, int cyl,
-                                                               int store_residual, int bpb, int nw) {
-  using L = Lay<D, NC, T>;
-  constexpr int H = NC / 2;
-  constexpr int NQ = (D == 3) ? H * H * H : H * H;
-  for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
-    const Part pt = part_of<BS>(ids, bpb, w);
-    if (pt.id <= 0) continue;  // run masked out
-    const int id = pt.id;
-    const DBox &bc = boxes[id - 1];
-    const DBox &bp = boxes[bc.parent - 1];
-    const Sten<D, T> s = lpl_stencil<D, T>(bc, lambda2);
-    const size_t cb = (size_t)(id - 1) * L::STRIDE, pb = (size_t)(bc.parent - 1) * L::STRIDE;
-    int off[3] = {0, 0, 0};
-    for (int d = 0; d < D; d++) off[d] = ((bc.ix[d] - 1) & 1) * H;
-    for (int q = pt.q0; q < NQ; q += pt.stride) {
-      const int i = q % H + 1, j = (q / H) % H + 1, k = (D == 3) ? q / (H * H) + 1 : 0;
-      const int i_f = 2 * i - 1, jf = 2 * j - 1, kf = (D == 3) ? 2 * k - 1 : 0;
-      // residuals of the 2^D children cells, in the summation order of
-      // af_restrict_box (i fastest, then j, then k)
-      T rs[8];
-      int cp[8];
-      child_pos<D, NC, L>(i_f, jf, kf, cp);
-      const int nch = (D == 3) ? 8 : 4;
-      for (int c = 0; c < nch; c++) {
-        const int ii = i_f + (c & 1), jj = jf + ((c >> 1) & 1), kk = kf + ((c >> 2) & 1);
-        T lp = apply_cell<D, NC, T, L>(phi + cb, s, cyl != 0, bc, ii, jj, kk);
-        rs[c] = rhs[cb + cp[c]] - lp;
-        if (store_residual) tmp[cb + cp[c]] = rs[c];
-      }
-      const int ic = off[0] + i, jc = off[1] + j, kc = (D == 3) ? off[2] + k : 0;
-      const T rv = restrict_children<D, T>(rs, cyl != 0, bp, ic);
-      tmp[pb + L::in_at(ic, jc, kc)] = rv;
-      phi[pb + L::in_at(ic, jc, kc)] = restrict_cell<D, NC, T, L>(phi + cb, i_f, jf, kf, false, bp, ic);
     }
   }
 }
@@ -1763,17 +1704,29 @@ __global__ void __launch_bounds__(BS * BB) k_mp_residual_lds(const int *__restri
   }
 }
 
-// k_restrict_residual with the child box staged in LDS and its face ghosts
-// formed in-kernel, so no ghost fill has to precede it.
+// update_coarse, first half (m_af_multigrid.f90:703-716): per child box the
+// residual rhs - L phi is restricted (with geometry) into the parent's tmp
+// and phi (without geometry) into the parent's phi.  The residual is formed
+// on the fly, which leaves the child's tmp untouched exactly as the
+// reference's save/restore of tmp does.  With store_residual the residual is
+// also kept in the child's tmp (set_coarse_phi_rhs, :742-776).
+// The child box is staged in LDS with its face ghosts: formed in-kernel, or
+// (stored) the stored layer, which the FP64 form fills beforehand as the
+// reference does.  Every thread forms the residuals of its own cells, which
+// then take phi's place in LDS for the restriction, so no thread is idle in
+// the larger part: 21 M cells of 8^2 boxes 66 us (104 with the residuals of
+// one parent cell in one thread), 4096 FP32 8^3 boxes 12.7 (16.6), 64 FP64
+// 16^3 boxes 6.2 (7.9), 768 22.0 (23.9), 1536 FP32 16^3 boxes 20.0 (19.3).
 template <int D, int NC, int BS, typename T, int BB = 1>
-__global__ void __launch_bounds__(BS * BB) k_restrict_residual_lds(const int *__restrict__ ids,
-                                                                   const DBox *__restrict__ boxes, const T *child,
-                                                                   T *phi, const T *__restrict__ rhs, T *tmp, T lambda2,
-                                                                   int cyl, int store_residual, VarBc m, int nw) {
+__global__ void __launch_bounds__(BS * BB, (BS >= 512 ? 4 : 1)) k_restrict_residual(const int *__restrict__ ids,
+                                                               const DBox *__restrict__ boxes, const T *child, T *phi,
+                                                               const T *__restrict__ rhs, T *tmp, T lambda2, int cyl,
+                                                               int store_residual, VarBc m, int stored, int nw) {
   using G = Geo<D, NC>;
   using L = Lay<D, NC, T>;
   constexpr int H = NC / 2;
-  constexpr int NQ = (D == 3) ? H * H * H : H * H;
+  constexpr int NQ = (D == 3) ? H * H * H : H * H, NQT = (NQ + BS - 1) / BS, NI = (G::NINT + BS - 1) / BS;
+  static_assert(G::NINT % BS == 0, "whole strides of cells");
   __shared__ T s_all[BB][G::NCELL];
   __shared__ T cp_all[BB][2 * D * CoarsePatch<D, NC>::N];
   T *s = s_all[lgrp<BS, BB>()], *cp = cp_all[lgrp<BS, BB>()];
@@ -1784,28 +1737,50 @@ __global__ void __launch_bounds__(BS * BB) k_restrict_residual_lds(const int *__
     const DBox &bp = boxes[bc.parent - 1];
     const size_t cb = (size_t)(id - 1) * L::STRIDE, pb = (size_t)(bc.parent - 1) * L::STRIDE;
     Stage<D, NC, BS, T, BB, false> sg;
-    sg.issue(bc, id, child, m, 0, (const T *)phi);
+    sg.issue(bc, id, child, m, 0, (const T *)phi, stored != 0);
+    T rr[NI];
+#pragma unroll
+    for (int t = 0; t < NI; t++) {
+      int i, j, k;
+      rr[t] = rhs[cb + sg.cell(ltid<BS>() + t * BS, i, j, k)];
+    }
     const Sten<D, T> st = lpl_stencil<D, T>(bc, lambda2);
     sg.commit(s, cp, bc, m);
+    // the residuals of the thread's cells and its parent cells' phi
+#pragma unroll
+    for (int t = 0; t < NI; t++) {
+      int i, j, k;
+      const int pos = sg.cell(ltid<BS>() + t * BS, i, j, k);
+      rr[t] = rr[t] - apply_cell<D, NC, T>(s, st, cyl != 0, bc, i, j, k);
+      if (store_residual) tmp[cb + pos] = rr[t];
+    }
+    T ps[NQT];
+#pragma unroll
+    for (int t = 0; t < NQT; t++) {
+      const int q = ltid<BS>() + t * BS;
+      const int i = q % H + 1, j = (q / H) % H + 1, k = (D == 3) ? q / (H * H) + 1 : 0;
+      if (NQ % BS == 0 || q < NQ)
+        ps[t] = restrict_cell<D, NC, T>(s, 2 * i - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0, false, bp, 0);
+    }
+    gsync<BS, BB>();
+#pragma unroll
+    for (int t = 0; t < NI; t++) {
+      int i, j, k;
+      sg.cell(ltid<BS>() + t * BS, i, j, k);
+      s[G::idx(i, j, k)] = rr[t];
+    }
+    gsync<BS, BB>();
     int off[3] = {0, 0, 0};
     for (int d = 0; d < D; d++) off[d] = ((bc.ix[d] - 1) & 1) * H;
-    for (int q = ltid<BS>(); q < NQ; q += BS) {
+#pragma unroll
+    for (int t = 0; t < NQT; t++) {
+      const int q = ltid<BS>() + t * BS;
+      if (NQ % BS && q >= NQ) continue;
       const int i = q % H + 1, j = (q / H) % H + 1, k = (D == 3) ? q / (H * H) + 1 : 0;
-      const int i_f = 2 * i - 1, jf = 2 * j - 1, kf = (D == 3) ? 2 * k - 1 : 0;
-      T rs[8];
-      int cp[8];
-      child_pos<D, NC, L>(i_f, jf, kf, cp);
-      const int nch = (D == 3) ? 8 : 4;
-      for (int c = 0; c < nch; c++) {
-        const int ii = i_f + (c & 1), jj = jf + ((c >> 1) & 1), kk = kf + ((c >> 2) & 1);
-        T lp = apply_cell<D, NC, T>(s, st, cyl != 0, bc, ii, jj, kk);
-        rs[c] = rhs[cb + cp[c]] - lp;
-        if (store_residual) tmp[cb + cp[c]] = rs[c];
-      }
       const int ic = off[0] + i, jc = off[1] + j, kc = (D == 3) ? off[2] + k : 0;
-      const T rv = restrict_children<D, T>(rs, cyl != 0, bp, ic);
-      tmp[pb + L::in_at(ic, jc, kc)] = rv;
-      phi[pb + L::in_at(ic, jc, kc)] = restrict_cell<D, NC, T>(s, i_f, jf, kf, false, bp, ic);
+      tmp[pb + L::in_at(ic, jc, kc)] =
+          restrict_cell<D, NC, T>(s, 2 * i - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0, cyl != 0, bp, ic);
+      phi[pb + L::in_at(ic, jc, kc)] = ps[t];
     }
     gsync<BS, BB>();  // (the group's LDS is reused by its next item)
   }
