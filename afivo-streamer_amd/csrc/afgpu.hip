@@ -287,8 +287,13 @@ struct afgpu_ctx {
     int *d_map = nullptr;
     double *A0 = nullptr, *A1 = nullptr;
     size_t cap = 0;  // doubles in A0 / A1
+    // the factors, and the 1-D operators they were made for: the same for
+    // every operator (lambda enters in the division only), and kept while the
+    // tree changes around the uniform level
     struct F {
       bool ok = false;
+      int N = 0, coord = 0;
+      double r_min[3] = {0, 0, 0}, dr[3] = {0, 0, 0};
       double *vinv = nullptr, *v = nullptr, *vinvT = nullptr, *vT = nullptr, *eig = nullptr;
       float *vinv32 = nullptr, *v32 = nullptr, *eig32 = nullptr;  // (rounded copies)
       // matrix-core operands (lc_pack): V^-1 and V per axis; parity-folded
@@ -297,7 +302,7 @@ struct afgpu_ctx {
       double *vinv_p = nullptr, *v_p = nullptr;
       bool fold[3] = {false, false, false};
       double *mf = nullptr, *bf = nullptr, *eigf = nullptr;
-    } f[1 + AFGPU_MAX_MODES];
+    } f;
   } dir;
   // the coarse levels of the FP64 multigrid in one workgroup per run
   // (k_tail): levels 1..lt, the box id of every slot, and the operations
@@ -1300,7 +1305,6 @@ struct Impl : ImplBase {
           d.cap = cells;
         }
       }
-      for (auto &f : d.f) f.ok = false;
       d.set = true;
     }
     *lc_out = d.lc;
@@ -1308,14 +1312,21 @@ struct Impl : ImplBase {
   }
 
   // 1-D eigen-factors of the level-lc operator (allocation and upload, so
-  // this runs before any capture).
-  int ensure_direct_factors(int op) {
+  // this runs before any capture).  The eigenvalue iterations run on the host,
+  // 0.07 s for an axis of 128 cells, so they run only when the 1-D operators
+  // are not those of the factors at hand (a tree that changes around the
+  // uniform level keeps them).
+  int ensure_direct_factors() {
     afgpu_ctx::Direct &d = c.dir;
-    afgpu_ctx::Direct::F &f = d.f[op];
-    if (f.ok || d.lc <= 1) return AFGPU_OK;
+    afgpu_ctx::Direct::F &f = d.f;
+    if (d.lc <= 1) return AFGPU_OK;
     const int N = d.N;
     const DBox &b1 = c.hboxes[c.h_lists[c.l_ids[1].off] - 1];
     const DBox &bl = c.hboxes[c.h_lists[c.l_ids[d.lc].off] - 1];
+    const bool same = f.N == N && f.coord == c.coord && std::equal(b1.r_min, b1.r_min + D, f.r_min) &&
+                      std::equal(bl.dr, bl.dr + D, f.dr);
+    if (f.ok && same) return AFGPU_OK;
+    f.ok = false;
     int bcd[6] = {0, 0, 0, 0, 0, 0};
     bcd[2 * (D - 1)] = 1;
     bcd[2 * (D - 1) + 1] = 1;
@@ -1414,6 +1425,10 @@ struct Impl : ImplBase {
       HIPCHK(hipMalloc(dst32[q], r.size() * sizeof(float)));
       HIPCHK(hipMemcpy(*dst32[q], r.data(), r.size() * sizeof(float), hipMemcpyHostToDevice));
     }
+    f.N = N;
+    f.coord = c.coord;
+    std::copy(b1.r_min, b1.r_min + D, f.r_min);
+    std::copy(bl.dr, bl.dr + D, f.dr);
     f.ok = true;
     return AFGPU_OK;
   }
@@ -1588,7 +1603,7 @@ struct Impl : ImplBase {
   template <typename T>
   int solve_level(const Mg<T> &v, int lc) {
     afgpu_ctx::Direct &d = c.dir;
-    const afgpu_ctx::Direct::F &f = d.f[v.op];
+    const afgpu_ctx::Direct::F &f = d.f;
     if (d.lc != lc || !f.ok) {
       set_err("uniform-level solve used before its set-up");
       return AFGPU_ERR_STATE;
@@ -1923,7 +1938,7 @@ struct Impl : ImplBase {
     int lc;
     RCHK(ensure_factors(op));
     RCHK(direct_level(&lc));
-    RCHK(ensure_direct_factors(op));
+    RCHK(ensure_direct_factors());
     RCHK(run_graph(c, {G_MP_RES, op, lc, 0}, [&] { return mp_close(op, false, lc); }));
     int n_active = 0;
     for (int r = 0; r < R; r++) n_active += active[r] != 0;
@@ -2163,10 +2178,8 @@ struct Impl : ImplBase {
       // modes take turns, each with its own masks.
       int lc;
       RCHK(direct_level(&lc));
-      for (int n = 0; n < n_modes; n++) {
-        RCHK(ensure_factors(AFGPU_OP_HELMH + n));
-        RCHK(ensure_direct_factors(AFGPU_OP_HELMH + n));
-      }
+      for (int n = 0; n < n_modes; n++) RCHK(ensure_factors(AFGPU_OP_HELMH + n));
+      RCHK(ensure_direct_factors());
       RCHK(ensure_mode_pools());
       const int all = (1 << n_modes) - 1;
       for (int group = 0; group < (R == 1 ? 1 : n_modes); group++) {
@@ -2344,7 +2357,7 @@ struct Impl : ImplBase {
     if (c.precision == AFGPU_PREC_MIXED) {
       int lc;
       RCHK(direct_level(&lc));
-      RCHK(ensure_direct_factors(AFGPU_OP_POISSON));
+      RCHK(ensure_direct_factors());
     }
     return AFGPU_OK;
   }
@@ -2852,7 +2865,8 @@ int afgpu_destroy(afgpu_t *h) {
   for (double *x : h->xsp) (void)hipFree(x);
   (void)hipFree(h->dir.A0);
   (void)hipFree(h->dir.A1);
-  for (auto &f : h->dir.f) {
+  {
+    auto &f = h->dir.f;
     (void)hipFree(f.vinv);
     (void)hipFree(f.v);
     (void)hipFree(f.vinvT);
@@ -3209,7 +3223,6 @@ int afgpu_sync_tree(afgpu_t *h, int n_boxes, const int *lvl, const int *ix, cons
   h->highest_lvl = hl;
   for (auto &o : h->ops) o.ok = false;  // level-1 box may have changed
   h->dir.set = false;
-  for (auto &f : h->dir.f) f.ok = false;
   h->tail.set = false;
   drop_graphs(*h);
   return AFGPU_OK;
@@ -4257,7 +4270,6 @@ int afgpu_set_option(afgpu_t *h, int option, int value) {
       drop_graphs(*h);
       h->direct_max_n = value;
       h->dir.set = false;
-      for (auto &f : h->dir.f) f.ok = false;
       return AFGPU_OK;
     case AFGPU_OPT_FUSE_DIRECT:
       RCHK(sync_stream(h));
