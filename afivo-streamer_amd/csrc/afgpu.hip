@@ -988,7 +988,7 @@ struct Impl : ImplBase {
   int correct_children(const Mg<T> &v, int lvl_p, T *target = nullptr) {
     if (in_tail<T>(lvl_p))
       RCHK(tail_push(TL_SUB, lvl_p));
-    else
+    else if (!Lay<D, NC, T>::SPLIT)
       RCHK(boxop<T>(c.l_parents[lvl_p], v.phi, v.tmp, OP_SUB_FROM));
     if (in_tail<T>(lvl_p + 1)) return tail_push(TL_PROLONG, lvl_p + 1);
     const List &l = c.l_ids[lvl_p + 1];
@@ -997,7 +997,7 @@ struct Impl : ImplBase {
       constexpr int bb = decltype(B)::value;
       if constexpr (Lay<D, NC, T>::SPLIT)
         return items<bb>(KC_PROLONG, k_prolong_add_split<D, NC, BS, bb>, l.n * k, c.list(l), (const DBox *)c.d_boxes,
-                         (const T *)v.tmp, target ? target : v.phi, k);
+                         (const T *)v.phi, (const T *)v.tmp, target ? target : v.phi, k);
       else
         return items<bb>(KC_PROLONG, k_prolong_add<D, NC, BS, T, bb>, l.n * k, c.list(l), (const DBox *)c.d_boxes,
                          (const T *)v.tmp, target ? target : v.phi, k);
