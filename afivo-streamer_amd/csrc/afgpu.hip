@@ -186,7 +186,6 @@ struct afgpu_ctx {
   double *d_run_volt = nullptr;
   std::vector<double> run_min_dr;  // finest cell size per run
   int *d_run_of = nullptr;         // run of every box (index id - 1)
-  int *d_run_active = nullptr;     // runs the list kernels work on
   int *d_run_host = nullptr;       // runs the host has made active
   int *h_run_active = nullptr;     // pinned staging of the above
   int *d_run_maxlvl = nullptr;     // highest level of every run
@@ -725,14 +724,12 @@ struct Impl : ImplBase {
     }
     tl.lt = lt;
     tl.set = true;
-    if (lt > 0 && c.masked) RCHK(mask_tail());
-    return AFGPU_OK;
-  }
-  int mask_tail() {
-    const int n = c.n_runs * TG::SLOTS;
-    hipLaunchKernelGGL(k_mask_ids, dim3((n + 255) / 256), dim3(256), 0, c.cur, c.tail.d_map, n,
-                       (const int *)c.d_run_of, (const int *)c.d_run_active);
-    HIPCHK(hipGetLastError());
+    if (lt > 0 && c.masked) {
+      MaskLists m{};
+      m.ids[0] = tl.d_map;
+      m.n[0] = c.n_runs * TG::SLOTS;
+      RCHK(mask_lists(m, RUNS_IN_LEVELS, 0, std::numeric_limits<int>::max()));
+    }
     return AFGPU_OK;
   }
   // Enqueue an FP64 cycle of operator op (body), its operations on levels
@@ -1151,32 +1148,33 @@ struct Impl : ImplBase {
   // runs made active by the host whose highest level lies in [lo, hi].
   int mask_levels(int lo, int hi) {
     RCHK(tail_flush());
-    hipLaunchKernelGGL(k_runs_in_levels, dim3((c.n_runs + 63) / 64), dim3(64), 0, c.cur, (const int *)c.d_run_host,
-                       (const int *)c.d_run_maxlvl, c.d_run_active, lo, hi, c.n_runs);
-    HIPCHK(hipGetLastError());
-    const int n = (int)c.h_lists.size();
-    hipLaunchKernelGGL(k_mask_ids, dim3((n + 255) / 256), dim3(256), 0, c.cur, c.d_lists, n,
-                       (const int *)c.d_run_of, (const int *)c.d_run_active);
-    HIPCHK(hipGetLastError());
+    MaskLists m{};
+    m.ids[0] = c.d_lists;
+    m.n[0] = (int)c.h_lists.size();
     if (c.dir.set && c.dir.lc > 1) {
-      const int nm = c.l_ids[c.dir.lc].n;
-      hipLaunchKernelGGL(k_mask_ids, dim3((nm + 255) / 256), dim3(256), 0, c.cur, c.dir.d_map, nm,
-                         (const int *)c.d_run_of, (const int *)c.d_run_active);
-      HIPCHK(hipGetLastError());
+      m.ids[1] = c.dir.d_map;
+      m.n[1] = c.l_ids[c.dir.lc].n;
     }
-    return (c.tail.set && c.tail.lt > 0) ? mask_tail() : AFGPU_OK;
+    if (c.tail.set && c.tail.lt > 0) {
+      m.ids[2] = c.tail.d_map;
+      m.n[2] = c.n_runs * TG::SLOTS;
+    }
+    return mask_lists(m, RUNS_IN_LEVELS, lo, hi);
   }
-
   // Device side of the masks of a mode's close in a forest (capturable):
-  // the runs made active by the host that would restrict level lvl (kind
-  // 0) or fill the ghosts of level lvl (kind 1) when solved alone.
+  // the runs made active by the host that would restrict level lvl
+  // (RUNS_RESTRICT) or fill the ghosts of level lvl (RUNS_GHOSTS) when
+  // solved alone.
   int mask_close(int kind, int lvl, int lc) {
-    hipLaunchKernelGGL(k_runs_close, dim3((c.n_runs + 63) / 64), dim3(64), 0, c.cur, (const int *)c.d_run_host,
-                       (const int *)c.d_run_bits, c.d_run_active, kind, lvl, lc, c.n_runs);
-    HIPCHK(hipGetLastError());
-    const int n = (int)c.h_lists.size();
-    hipLaunchKernelGGL(k_mask_ids, dim3((n + 255) / 256), dim3(256), 0, c.cur, c.d_lists, n,
-                       (const int *)c.d_run_of, (const int *)c.d_run_active);
+    MaskLists m{};
+    m.ids[0] = c.d_lists;
+    m.n[0] = (int)c.h_lists.size();
+    return mask_lists(m, kind, lc, lvl);
+  }
+  int mask_lists(const MaskLists &m, int kind, int lo, int hi) {
+    const RunRule u = {c.d_run_host, c.d_run_maxlvl, c.d_run_bits, kind, lo, hi, c.n_runs};
+    const int n = m.n[0] + m.n[1] + m.n[2];
+    hipLaunchKernelGGL(k_mask_ids, dim3((n + 255) / 256), dim3(256), 0, c.cur, m, (const int *)c.d_run_of, u);
     HIPCHK(hipGetLastError());
     return AFGPU_OK;
   }
@@ -1698,12 +1696,12 @@ struct Impl : ImplBase {
       // over all runs, would touch cells a run alone leaves as they are).
       const int top = std::numeric_limits<int>::max();
       for (int lvl = c.highest_lvl; lvl >= mp_restrict_lo(lc); lvl--) {
-        RCHK(mask_close(0, lvl, lc));
+        RCHK(mask_close(RUNS_RESTRICT, lvl, lc));
         RCHK(restrict_levels(iphi, lvl, lvl));
       }
       for (int lvl = lc; lvl < c.highest_lvl; lvl++)
         if (c.lvl_rb[lvl + 1]) {
-          RCHK(mask_close(1, lvl, lc));
+          RCHK(mask_close(RUNS_GHOSTS, lvl, lc));
           RCHK(gc_list(c.l_rbnb[lvl], c.cc[iphi], m, true));
         }
       RCHK(mask_levels(0, top));
@@ -2890,7 +2888,6 @@ int afgpu_destroy(afgpu_t *h) {
   if (h->h_red) (void)hipHostFree(h->h_red);
   (void)hipFree(h->d_run_of);
   (void)hipFree(h->d_run_volt);
-  (void)hipFree(h->d_run_active);
   (void)hipFree(h->d_run_host);
   (void)hipFree(h->d_run_maxlvl);
   (void)hipFree(h->d_run_bits);
@@ -3141,7 +3138,6 @@ int afgpu_sync_tree(afgpu_t *h, int n_boxes, const int *lvl, const int *ix, cons
     (void)hipFree(h->d_red);
     (void)hipFree(h->d_red_out);
     (void)hipFree(h->d_run_volt);
-    (void)hipFree(h->d_run_active);
     (void)hipFree(h->d_run_host);
     (void)hipFree(h->d_run_maxlvl);
     (void)hipFree(h->d_dt_run);
@@ -3157,17 +3153,16 @@ int afgpu_sync_tree(afgpu_t *h, int n_boxes, const int *lvl, const int *ix, cons
     if (h->h_dt_run) (void)hipHostFree(h->h_dt_run);
     h->d_red = h->d_red_out = nullptr;
     h->d_run_volt = h->d_dt_run = nullptr;
-    h->d_run_active = h->d_run_host = h->d_run_maxlvl = h->d_run_bits = nullptr;
     h->h_red = nullptr;
     h->h_run_active = nullptr;
     h->h_dt_run = nullptr;
+    h->d_run_host = h->d_run_maxlvl = h->d_run_bits = nullptr;
     h->red_cap_runs = 0;
     const size_t nr = (size_t)n_runs;
     HIPCHK(hipMalloc(&h->d_red, nr * RED_STRIPES * N_RED_SLOTS * sizeof(unsigned long long)));
     HIPCHK(hipMalloc(&h->d_red_out, nr * N_RED_SLOTS * sizeof(unsigned long long)));
     HIPCHK(hipHostMalloc(&h->h_red, nr * N_RED_SLOTS * sizeof(unsigned long long), hipHostMallocDefault));
     HIPCHK(hipMalloc(&h->d_run_volt, nr * sizeof(double)));
-    HIPCHK(hipMalloc(&h->d_run_active, nr * sizeof(int)));
     HIPCHK(hipMalloc(&h->d_run_host, nr * sizeof(int)));
     HIPCHK(hipMalloc(&h->d_run_maxlvl, nr * sizeof(int)));
     HIPCHK(hipMalloc(&h->d_run_bits, 2 * nr * sizeof(int)));
