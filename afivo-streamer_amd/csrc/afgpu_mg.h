@@ -2091,6 +2091,53 @@ __global__ void __launch_bounds__(BS * BB) k_gc(const int *__restrict__ ids, con
   }
 }
 
+// k_gc with corners on a level, and k_coarse_rhs on its boxes with children:
+// the two that follow the restriction onto a level, in one launch (the
+// second reads only its own box's cells and the ghosts just filled).  Both
+// are bound by their chains on small levels of 2D boxes.
+template <int D, int NC, int BS, typename T, int BB = 1>
+__global__ void __launch_bounds__(BS * BB) k_gc_rhs(const int *__restrict__ ids, const DBox *__restrict__ boxes,
+                                                    T *phi, T *rhs, T *tmp, T lambda2, int cyl, int copy_phi,
+                                                    VarBc m, int nw) {
+  using G = Geo<D, NC>;
+  using L = Lay<D, NC, T>;
+  __shared__ T s_all[BB][GcGeo<D, NC>::NFC];
+  __shared__ T cp_all[BB][2 * D * CoarsePatch<D, NC>::N];
+  T *s = s_all[lgrp<BS, BB>()], *cp = cp_all[lgrp<BS, BB>()];
+  for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
+    const int id = __builtin_amdgcn_readfirstlane(ids[w]);
+    if (id <= 0) continue;  // run masked out
+    const DBox &bx = boxes[id - 1];
+    const size_t base = (size_t)(id - 1) * L::STRIDE;
+    const bool parent = bx.children[0] > 0;
+    gc_box<D, NC, BS, T, BB>(s, cp, boxes, id, phi, m, 1);
+    if (!parent) continue;
+    // (the ghosts were stored by other threads of the group)
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    gsync<BS, BB>();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+    const Sten<D, T> st = lpl_stencil<D, T>(bx, lambda2);
+#pragma unroll 2
+    for (int x = ltid<BS>(); x < G::NCELL; x += BS) {
+      int i, j, k;
+      bool inner;
+      if constexpr (L::SPLIT) {
+        inner = x < G::NINT;
+        if (inner) colour_cell<D, NC>(x >= L::HALF, x >= L::HALF ? x - L::HALF : x, i, j, k);
+      } else {
+        i = x % G::NG, j = (x / G::NG) % G::NG, k = (D == 3) ? x / (G::NG * G::NG) : 0;
+        inner = i >= 1 && i <= NC && j >= 1 && j <= NC && (D == 2 || (k >= 1 && k <= NC));
+      }
+      // (nothing reads the ghost part of a split pool's rhs)
+      if (inner)
+        rhs[base + x] = apply_cell<D, NC, T, L>(phi + base, st, cyl != 0, bx, i, j, k) + tmp[base + x];
+      else if (!L::SPLIT)
+        rhs[base + x] = rhs[base + x] + tmp[base + x];
+      if (copy_phi) tmp[base + x] = phi[base + x];
+    }
+  }
+}
+
 // The same for several FP64 variables in one launch: work item w is box
 // w / vars.n, variable w % vars.n.
 constexpr int GC_MAX_VARS = 8;
