@@ -98,15 +98,32 @@ __global__ void __launch_bounds__(BS * BB)
            unsigned long long *cfl_max, unsigned long long *sig_max, int nw) {
   using G = Geo<D, NC>;
   constexpr int NT = G::NTAN;
-  __shared__ TF halo_all[BB][2 * D][2][NT];
-  TF(&halo)[2 * D][2][NT] = halo_all[lgrp<BS, BB>()];
-  // the mobility and diffusion columns of the transport table (3D, single
-  // precision, up to TABMAX rows), converted as lt_at_t converts them
-  constexpr int TABMAX = (D == 3 && sizeof(TF) < sizeof(double)) ? 1024 : 1;
-  __shared__ TF tab_all[BB][2 * TABMAX];
+  // columns of cells marched through (16^3), or the box's cells in LDS
+  constexpr bool MARCH = D == 3 && BS == NC * NC;
+  constexpr int NP = NC + 4, NE = NC + 2;
+  __shared__ TF halo_all[BB][2 * D][2][MARCH ? NT : 1];
+  TF(&halo)[2 * D][2][MARCH ? NT : 1] = halo_all[lgrp<BS, BB>()];
+  // the mobility and diffusion columns of the transport table (single
+  // precision, up to TABMAX rows), converted as lt_at_t converts them; one
+  // copy for all groups
+  constexpr int TABMAX = (sizeof(TF) < sizeof(double)) ? 1024 : 1;
+  __shared__ TF tab[2 * TABMAX];
   const bool tab_lds = TABMAX > 1 && td.n <= TABMAX;
   if (tab_lds)  // (read after the first item's halo barrier)
-    for (int q = ltid<BS>(); q < 2 * td.n; q += BS) tab_all[lgrp<BS, BB>()][(q / td.n) * TABMAX + q % td.n] = (TF)td.cols[q];
+    for (int q = threadIdx.x; q < 2 * td.n; q += BS * BB) tab[(q / td.n) * TABMAX + q % td.n] = (TF)td.cols[q];
+  if (TABMAX > 1 && BB > 1) __syncthreads();  // (the groups' barriers are their own)
+  // MARCH == false: n_e with its two halo layers, |E| with its ghosts, and
+  // |v| and D of the faces: the lower ones of the cells, then the box's
+  // upper ones
+  constexpr int N_PN = MARCH ? 1 : (D == 3) ? NP * NP * NP : NP * NP;
+  constexpr int N_PE = MARCH ? 1 : (D == 3) ? NE * NE * NE : NE * NE;
+  constexpr int N_FC = MARCH ? 1 : G::NINT + NT;
+  __shared__ TF bn_all[BB][N_PN], be_all[BB][N_PE], bv_all[BB][D][N_FC], bd_all[BB][D][N_FC];
+  TF *bn = bn_all[lgrp<BS, BB>()], *be = be_all[lgrp<BS, BB>()];
+  TF(&bv)[D][N_FC] = bv_all[lgrp<BS, BB>()];
+  TF(&bd)[D][N_FC] = bd_all[lgrp<BS, BB>()];
+  auto pos_n = [](int i, int j, int k) { return i + 1 + NP * (j + 1 + (D == 3 ? NP * (k + 1) : 0)); };
+  auto pos_e = [](int i, int j, int k) { return i + NE * (j + (D == 3 ? NE * k : 0)); };
   __shared__ double sh[BS / 64];
   for (int w = item0<BS, BB>(); w < nw; w += item_stride<BB>()) {
     const int id = ids[w];
@@ -116,6 +133,46 @@ __global__ void __launch_bounds__(BS * BB)
     const size_t fbase = (size_t)(id - 1) * D * G::NFACE;
     const TF N_inv = (TF)N_inv_d;
 
+    // what the box's faces need of its own cells, in flight with the halo
+    constexpr int PER = MARCH ? 1 : G::NINT / BS;               // cells of a thread,
+    constexpr int RPER = MARCH ? 1 : (2 * D * NT + BS - 1) / BS;  // |E| ghosts,
+    constexpr int UPER = MARCH ? 1 : (D * NT + BS - 1) / BS;      // upper faces of the box
+    static_assert(MARCH || G::NINT % BS == 0, "whole strides of cells");
+    auto face_at = [](int d, int r, int pn, int *p) {  // position r of a plane across d, at index pn
+      int t0, t1;
+      tangential(D, d, t0, t1);
+      p[0] = p[1] = p[2] = 0;
+      p[t0] = r % NC + 1;
+      if (D == 3) p[t1] = r / NC + 1;
+      p[d] = pn;
+    };
+    double nv[PER], ev[PER], er[RPER];
+    double ex[PER][D], exu[UPER];
+    if constexpr (!MARCH) {
+#pragma unroll
+      for (int t = 0; t < PER; t++) {
+        int i, j, k;
+        interior_ijk<D, NC>(ltid<BS>() + t * BS, i, j, k);
+        nv[t] = ne[base + G::idx(i, j, k)];
+        ev[t] = efield[base + G::idx(i, j, k)];
+#pragma unroll
+        for (int d = 0; d < D; d++) ex[t][d] = efc[fbase + G::fidx(i, j, (D == 3) ? k : 1, d)];
+      }
+#pragma unroll
+      for (int t = 0; t < RPER; t++) {
+        const int q = min(ltid<BS>() + t * BS, 2 * D * NT - 1), nb = q / NT;
+        int p[3];
+        face_at(nb / 2, q % NT, (nb & 1) ? NC + 1 : 0, p);
+        er[t] = efield[base + G::idx(p[0], p[1], p[2])];
+      }
+#pragma unroll
+      for (int t = 0; t < UPER; t++) {
+        const int q = min(ltid<BS>() + t * BS, D * NT - 1);
+        int p[3];
+        face_at(q / NT, q % NT, NC + 1, p);
+        exu[t] = efc[fbase + G::fidx(p[0], p[1], (D == 3) ? p[2] : 1, q / NT)];
+      }
+    }
     // the halo; its first layer also goes back into the box
     // (m_af_ghostcell.f90:740-742): no thread of any box reads a ghost cell
     // of this level during the launch
@@ -123,34 +180,35 @@ __global__ void __launch_bounds__(BS * BB)
       const int nb = q / (2 * NT), layer = (q / NT) % 2, r = q % NT;
       const int a = r % NC + 1, b = (D == 3) ? r / NC + 1 : 0;
       const double hv = gc2_value<D, NC>(boxes, id, ne, m, nb, layer, a, b);
-      halo[nb][layer][r] = (TF)hv;
-      if (layer == 0) {
-        const int d = nb / 2;
-        int t0, t1;
-        tangential(D, d, t0, t1);
-        int p[3] = {0, 0, 0};
-        p[t0] = a;
-        if (D == 3) p[t1] = b;
-        p[d] = (nb % 2) ? NC + 1 : 0;
-        ne[base + G::idx(p[0], p[1], p[2])] = hv;
+      int p[3];
+      face_at(nb / 2, r, (nb % 2) ? NC + 1 + layer : -layer, p);
+      if constexpr (MARCH)
+        halo[nb][layer][r] = (TF)hv;
+      else
+        bn[pos_n(p[0], p[1], p[2])] = (TF)hv;
+      if (layer == 0) ne[base + G::idx(p[0], p[1], p[2])] = hv;
+    }
+    if constexpr (!MARCH) {
+#pragma unroll
+      for (int t = 0; t < PER; t++) {
+        int i, j, k;
+        interior_ijk<D, NC>(ltid<BS>() + t * BS, i, j, k);
+        bn[pos_n(i, j, k)] = (TF)nv[t];
+        be[pos_e(i, j, k)] = (TF)ev[t];
+      }
+#pragma unroll
+      for (int t = 0; t < RPER; t++) {
+        const int q = min(ltid<BS>() + t * BS, 2 * D * NT - 1), nb = q / NT;
+        int p[3];
+        face_at(nb / 2, q % NT, (nb & 1) ? NC + 1 : 0, p);
+        be[pos_e(p[0], p[1], p[2])] = (TF)er[t];
       }
     }
     gsync<BS, BB>();
 
-    auto line = [&](int d, int r, const int *p, int q) -> TF {
-      if (q >= 1 && q <= NC) {
-        int pp[3] = {p[0], p[1], p[2]};
-        pp[d] = q;
-        return (TF)ne[base + G::idx(pp[0], pp[1], pp[2])];
-      }
-      if (q <= 0) return halo[2 * d][-q][r];
-      return halo[2 * d + 1][q - NC - 1][r];
-    };
-
     TF smax = -std::numeric_limits<TF>::max();
     TF cmax = 0;
-    if constexpr (D == 3) {
-      const TF *tab = tab_lds ? tab_all[lgrp<BS, BB>()] : nullptr;
+    {
       auto coef = [&](int c, int ix, TF w) {
         return tab_lds ? w * tab[c * TABMAX + ix - 1] + (1 - w) * tab[c * TABMAX + ix] : lt_at_t<TF>(td, c, ix, w);
       };
@@ -178,7 +236,7 @@ __global__ void __launch_bounds__(BS * BB)
       auto cfl_term = [](TF av_hi, TF av_lo, TF dc_hi, TF dc_lo, TF inv_dx) -> TF {
         return TF(1) * fmax(av_hi, av_lo) * inv_dx + TF(2) * fmax(dc_hi, dc_lo) * (inv_dx * inv_dx);
       };
-      if constexpr (BS == NC * NC) {
+      if constexpr (MARCH) {
         // Face fluxes (flux_upwind, src/m_fluid.f90:102-209), one thread per
         // grid column (i, j), walking up the box in z.  Plane k is staged in
         // LDS (n_e with its two halo layers in x and y, |E| with its ghost
@@ -192,7 +250,6 @@ __global__ void __launch_bounds__(BS * BB)
         // the next plane.  Global loads and stores are rows of cells or
         // faces in x, the contiguous direction.
         static_assert(BB == 1 && BS >= 12 * NC, "one box of NC x NC columns per workgroup");
-        constexpr int NP = NC + 4, NE = NC + 2;
         __shared__ TF pn[NP * NP];            // n_e of the plane: (i, j) at (j + 1) NP + i + 1, i, j = -1 .. NC + 2
         __shared__ TF pe[NE * NE];            // |E| of the plane: (i, j) at j NE + i, i, j = 0 .. NC + 1
         __shared__ TF fv[2][BS + NC], fd[2][BS + NC];  // |v| and D of the plane's x and y faces (lower, upper boundary)
@@ -294,132 +351,76 @@ __global__ void __launch_bounds__(BS * BB)
             (double)face(n0, n1, n2, n3, (TF)efc[fbase + G::fidx(i, j, NC + 1, 2)], em, e0, inv_dx[2], vz, dz);
         cmax = fmax(cmax, pend + cfl_term(fabs(vz), avz_prev, dz, dz_prev, inv_dx[2]));
       } else {
-        // Boxes with fewer columns than threads (8^3): face fluxes
-        // (flux_upwind, src/m_fluid.f90:102-209) cell by cell, x fastest
-        // over the threads, so that the loads of every direction
-        // are coalesced and a cell's n_e and field are read while still in
-        // cache by all three directions.  For each direction a cell forms its
-        // lower and its upper face: an interior face is formed by both of its
-        // cells, from the same values, and written by the cell above it; the
-        // box's last face by the cell below it.  The two faces' velocities and
-        // diffusion coefficients give the cell's CFL term (m_fluid.f90:194-195,
-        // m_af_flux_schemes.f90:779-848), summed over the directions in the
-        // order x, y, z.
-        for (int q = ltid<BS>(); q < G::NINT; q += BS) {
-          const int p[3] = {q % NC + 1, (q / NC) % NC + 1, q / (NC * NC) + 1};
+        // Face fluxes (flux_upwind, src/m_fluid.f90:102-209) with the box in
+        // LDS, x fastest over the threads: a thread forms the lower faces of
+        // its cells, some threads one of the box's upper faces too, so every
+        // face is formed once; then a cell takes its upper faces' |v| and D
+        // from the threads that formed them for its CFL term
+        // (m_fluid.f90:194-195, m_af_flux_schemes.f90:779-848), summed over
+        // the directions in the order x, y, z.  Bound by the faces' limiters
+        // and table look-ups (in LDS in single precision).  With a face per
+        // thread and the cells' CFL terms from look-ups of their own, 16 M
+        // 2D cells took 290 us (123); with both faces of every cell formed
+        // by it, 4096 8^3 boxes 157 us (87) and 370 FP64 ones 17 (13).
+        constexpr int sn[3] = {1, NP, NP * NP}, se[3] = {1, NE, NE * NE}, sc[3] = {1, NC, NC * NC};
+        TF inv_dx[D], av[PER][D], dl[PER][D];
+#pragma unroll
+        for (int d = 0; d < D; d++) inv_dx[d] = TF(1) / (TF)bx.dr[d];
+        // the face below cell p along d, its position f among bv and bd
+        auto form = [&](int d, const int *p, TF e, int f, TF &v, TF &dc) {
+          const TF *n = bn + pos_n(p[0], p[1], p[2]), *ee = be + pos_e(p[0], p[1], p[2]);
+          flux[fbase + G::fidx(p[0], p[1], (D == 3) ? p[2] : 1, d)] = (double)face(
+              n[-2 * sn[d]], n[-sn[d]], n[0], n[sn[d]], e, ee[-se[d]], ee[0], inv_dx[d], v, dc);
+          v = fabs(v);
+          bv[d][f] = v;
+          bd[d][f] = dc;
+        };
+#pragma unroll
+        for (int t = 0; t < PER; t++) {
+          const int q = ltid<BS>() + t * BS;
+          int p[3];
+          interior_ijk<D, NC>(q, p[0], p[1], p[2]);
+#pragma unroll
+          for (int d = 0; d < D; d++) form(d, p, (TF)ex[t][d], q, av[t][d], dl[t][d]);
+        }
+#pragma unroll
+        for (int t = 0; t < UPER; t++) {
+          const int q = ltid<BS>() + t * BS, d = q / NT, r = q % NT;
+          if (q >= D * NT) break;
+          int p[3];
+          face_at(d, r, NC + 1, p);
+          TF inv = inv_dx[0];
+#pragma unroll
+          for (int dd = 1; dd < D; dd++) inv = (d == dd) ? inv_dx[dd] : inv;
+          const int on = (d == 0) ? sn[0] : (d == 1) ? sn[1] : sn[2], oe = (d == 0) ? se[0] : (d == 1) ? se[1] : se[2];
+          const TF *n = bn + pos_n(p[0], p[1], p[2]), *ee = be + pos_e(p[0], p[1], p[2]);
+          TF v, dc;
+          flux[fbase + G::fidx(p[0], p[1], (D == 3) ? p[2] : 1, d)] =
+              (double)face(n[-2 * on], n[-on], n[0], n[on], (TF)exu[t], ee[-oe], ee[0], inv, v, dc);
+          bv[d][G::NINT + r] = fabs(v);
+          bd[d][G::NINT + r] = dc;
+        }
+        gsync<BS, BB>();
+#pragma unroll
+        for (int t = 0; t < PER; t++) {
+          const int q = ltid<BS>() + t * BS;
+          int p[3];
+          interior_ijk<D, NC>(q, p[0], p[1], p[2]);
           TF cfl = 0;
+#pragma unroll
           for (int d = 0; d < D; d++) {
-            const TF inv_dx = TF(1) / (TF)bx.dr[d];
             int t0, t1;
             tangential(D, d, t0, t1);
-            const int r = (p[t0] - 1) + NC * (p[t1] - 1);  // the cell's position on a face of direction d
-            constexpr int st[3] = {1, G::NG, G::NG * G::NG};
-            const int cd = p[d];
-            const size_t c0 = base + G::idx(p[0], p[1], p[2]);
-            TF nl[5];  // n_e at cd - 2 .. cd + 2 along d
-            for (int s2 = -2; s2 <= 2; s2++) {
-              const int pos = cd + s2;
-              nl[s2 + 2] = (pos >= 1 && pos <= NC) ? (TF)ne[c0 + s2 * st[d]]
-                           : (pos <= 0)              ? halo[2 * d][-pos][r]
-                                                     : halo[2 * d + 1][pos - NC - 1][r];
-            }
-            const TF e_m = (TF)efield[c0 - st[d]], e_0 = (TF)efield[c0], e_p = (TF)efield[c0 + st[d]];
-            int fp[3] = {p[0], p[1], p[2]};
-            const size_t f_lo = fbase + G::fidx(fp[0], fp[1], fp[2], d);
-            fp[d] = cd + 1;
-            const size_t f_hi = fbase + G::fidx(fp[0], fp[1], fp[2], d);
-            TF v_lo, dc_lo, v_hi, dc_hi;
-            const TF fl_lo = face(nl[0], nl[1], nl[2], nl[3], (TF)efc[f_lo], e_m, e_0, inv_dx, v_lo, dc_lo);
-            const TF fl_hi = face(nl[1], nl[2], nl[3], nl[4], (TF)efc[f_hi], e_0, e_p, inv_dx, v_hi, dc_hi);
-            flux[f_lo] = (double)fl_lo;
-            if (cd == NC) flux[f_hi] = (double)fl_hi;
-            cfl = cfl + cfl_term(fabs(v_hi), fabs(v_lo), dc_hi, dc_lo, inv_dx);
+            const int r = (p[t0] - 1) + (D == 3 ? NC * (p[t1] - 1) : 0);
+            const int f = (p[d] < NC) ? q + sc[d] : G::NINT + r;
+            cfl = cfl + cfl_term(bv[d][f], av[t][d], bd[d][f], dl[t][d], inv_dx[d]);
           }
           cmax = fmax(cmax, cfl);
         }
       }
-      double smax_d = group_max<BS, BB>((double)smax, sh);
-      if (ltid<BS>() == 0) atomic_max_nonneg(run_slot(sig_max, bx), fmax(smax_d, 1e-100));
-    } else {
-      // 2D boxes have too few lines per direction for a thread each: one
-      // face per thread (flux_upwind, src/m_fluid.f90:102-209), then the
-      // CFL sum per cell from its faces
-      for (int q = ltid<BS>(); q < D * (NC + 1) * NT; q += BS) {
-        const int d = q / ((NC + 1) * NT);
-        // x faces: consecutive threads take consecutive faces of one grid row
-        // (contiguous in memory); y/z faces: consecutive rows of one face plane
-        const int qd = q % ((NC + 1) * NT);
-        const int f = (d == 0) ? qd % (NC + 1) + 1 : qd / NT + 1;
-        const int r = (d == 0) ? qd / (NC + 1) : qd % NT;
-        int t0, t1;
-        tangential(D, d, t0, t1);
-        int p[3] = {0, 0, 0};
-        p[t0] = r % NC + 1;
-        if (D == 3) p[t1] = r / NC + 1;
-        const TF inv_dx = TF(1) / (TF)bx.dr[d];
-        int fp[3] = {p[0], p[1], (D == 3) ? p[2] : 1};
-        fp[d] = f;
-        const TF ex = (TF)efc[fbase + G::fidx(fp[0], fp[1], fp[2], d)];
-        const TF Lm2 = line(d, r, p, f - 2), Lm1 = line(d, r, p, f - 1), L0 = line(d, r, p, f),
-                 Lp1 = line(d, r, p, f + 1);
-        TF u;
-        if (-1 * ex > 0) {
-          u = Lm1 + TF(0.5) * lim_koren<TF>(L0 - Lm1, Lm1 - Lm2);
-        } else {
-          u = L0 - TF(0.5) * lim_koren<TF>(L0 - Lm1, Lp1 - L0);
-        }
-        int e0[3] = {p[0], p[1], p[2]}, e1[3] = {p[0], p[1], p[2]};
-        e0[d] = f - 1;
-        e1[d] = f;
-        const TF tmp_fc = TF(0.5) * ((TF)efield[base + G::idx(e0[0], e0[1], e0[2])] +
-                                     (TF)efield[base + G::idx(e1[0], e1[1], e1[2])]) *
-                          (TF)SI_to_Townsend * N_inv;
-        int lix;
-        TF lw;
-        lt_loc_t<TF>(td, tmp_fc, lix, lw);
-        const TF mu = lt_at_t<TF>(td, 0, lix, lw) * N_inv;
-        const TF dc = lt_at_t<TF>(td, 1, lix, lw) * N_inv;
-        const TF v = -mu * ex;
-        flux[fbase + G::fidx(fp[0], fp[1], fp[2], d)] = (double)(v * u - dc * inv_dx * (L0 - Lm1));
-        smax = fmax(smax, mu * u);
-      }
-      double smax_d = group_max<BS, BB>((double)smax, sh);
-      if (ltid<BS>() == 0) atomic_max_nonneg(run_slot(sig_max, bx), fmax(smax_d, 1e-100));
-
-      // CFL sum per cell (m_fluid.f90:194-195 summed over dimensions,
-      // m_af_flux_schemes.f90:779-848)
-      for (int q = ltid<BS>(); q < G::NINT; q += BS) {
-        int i, j, k;
-        interior_ijk<D, NC>(q, i, j, k);
-        TF cfl = 0;
-        for (int d = 0; d < D; d++) {
-          const TF inv_dx = TF(1) / (TF)bx.dr[d];
-          TF vv[2], dd[2];
-          for (int s = 0; s < 2; s++) {
-            int c[3] = {i, j, k};
-            int fp[3] = {i, j, (D == 3) ? k : 1};
-            fp[d] += s;  // faces c and c+1
-            const TF ex = (TF)efc[fbase + G::fidx(fp[0], fp[1], fp[2], d)];
-            int e0[3] = {c[0], c[1], c[2]};
-            e0[d] = c[d] - 1 + s;
-            int e1[3] = {c[0], c[1], c[2]};
-            e1[d] = c[d] + s;
-            const TF tmp_fc = TF(0.5) * ((TF)efield[base + G::idx(e0[0], e0[1], e0[2])] +
-                                         (TF)efield[base + G::idx(e1[0], e1[1], e1[2])]) *
-                              (TF)SI_to_Townsend * N_inv;
-            int lix;
-            TF lw;
-            lt_loc_t<TF>(td, tmp_fc, lix, lw);
-            const TF mu = lt_at_t<TF>(td, 0, lix, lw) * N_inv;
-            dd[s] = lt_at_t<TF>(td, 1, lix, lw) * N_inv;
-            vv[s] = -mu * ex;
-          }
-          const TF cl = TF(1) * fmax(fabs(vv[1]), fabs(vv[0])) * inv_dx + TF(2) * fmax(dd[1], dd[0]) * (inv_dx * inv_dx);
-          cfl = cfl + cl;
-        }
-        cmax = fmax(cmax, cfl);
-      }
     }
+    const double smax_d = group_max<BS, BB>((double)smax, sh);
+    if (ltid<BS>() == 0) atomic_max_nonneg(run_slot(sig_max, bx), fmax(smax_d, 1e-100));
     const double cmax_d = group_max<BS, BB>((double)cmax, sh);
     if (ltid<BS>() == 0) atomic_max_nonneg(run_slot(cfl_max, bx), cmax_d);
     gsync<BS, BB>();  // (the group's halo is reused by its next item)

@@ -1,5 +1,6 @@
 """The ghost fill and coarse rhs in one launch (k_gc_rhs, smaller 2D levels)
-against the two launches of large levels: the same bits."""
+against the two launches of large levels, and k_flux's two homes of the
+transport table: the same bits."""
 import numpy as np
 import pytest
 
@@ -32,3 +33,25 @@ def test_copies_of_a_run_in_small_and_large_forests(S, A, mixed):
         for a, b in zip(got[0], info):
             assert list(a) == [b[0]] * n
         assert np.array_equal(got[1], np.broadcast_to(want[0], got[1].shape))
+
+
+@pytest.mark.parametrize("ndim,nc", [(2, 8), (2, 16), (3, 8), (3, 16)])
+def test_flux_with_the_table_in_lds_and_in_memory(S, A, ndim, nc):
+    """A transport table of more rows than LDS holds, its first rows the
+    small one's and its others never reached, gives the same step."""
+    case = S.small_amr(ndim, nc=nc, uniform_lvl=2, max_lvl=3, frac=0.5, seed=31)
+    out = []
+    for rows in (case.tdata["n"], 1024, 1025):
+        tb = dict(case.tdata)
+        for k in ("td", "chem"):
+            cols = np.asarray(tb[k]).reshape(-1, tb["n"])
+            tb[k] = np.ascontiguousarray(np.concatenate([cols, np.repeat(cols[:, -1:], rows - tb["n"], 1)], 1))
+        tb["n"] = rows
+        p = A.Path("gpu", ndim, nc, A.XYZ, A.PREC_MIXED)
+        S.apply(p, case)
+        p.set_tables(tb)
+        out.append([p.field_compute(0, False)] + [p.step() for _ in range(2)] + [p.get_cc(A.CC_ELECTRON)])
+        p.close()
+    for o in out[1:]:
+        assert o[:-1] == out[0][:-1]
+        assert np.array_equal(o[-1], out[0][-1])
