@@ -786,12 +786,6 @@ struct Impl : ImplBase {
   // Threads per box of the staging kernels on levels of up to one 16^3 box
   // per CU: four times as many as elsewhere, each with a quarter of the loads.
   static constexpr int MANY_NT = (D == 3 && NC == 16) ? 1024 : BS;
-  // the restriction keeps its cells' residuals in registers: on 16^3 boxes
-  // 8 (FP32) or 4 (FP64) a thread
-  template <typename T>
-  static constexpr int restrict_nt() {
-    return (D == 3 && NC == 16) ? (sizeof(T) == 8 ? 1024 : 512) : BS;
-  }
   bool many_threads(int n_boxes) const { return MANY_NT != BS && n_boxes <= c.n_cu; }
 
   // Workgroups per box: 1 on large levels; on levels with few boxes the
@@ -957,18 +951,27 @@ struct Impl : ImplBase {
     // run's own finest level needs it, and for the other runs the fill
     // repeats the one the level above has just made, with the same values)
     if (!forms && !v_cycle && (lvl == c.highest_lvl || c.uneven)) RCHK(gc_var(lvl, v.phi, v.m, true));
-    auto restricted = [&](auto NT, auto B) {
+    auto restricted = [&](auto NT, auto B, auto OWN) {
       constexpr int nt = decltype(NT)::value, bb = decltype(B)::value;
-      return items<bb, nt * bb>(KC_RESTRICT, k_restrict_residual<D, NC, nt, T, bb>, l.n, c.list(l),
+      constexpr bool own = decltype(OWN)::value;
+      return items<bb, nt * bb>(KC_RESTRICT, k_restrict_residual<D, NC, nt, T, bb, own>, l.n, c.list(l),
                                 (const DBox *)c.d_boxes, (const T *)level_buf(v, lvl, v_cycle), v.phi,
                                 (const T *)v.rhs, v.tmp, v.lambda2, cyl, (int)!v_cycle, v.m, (int)!forms);
     };
+    // (up to one 16^3 box per CU 1024 threads; FP32 levels of more, from 512
+    // to 2816 boxes, are 4 to 17 % faster a parent cell per thread)
+    constexpr bool parents = D == 3 && NC == 16 && std::is_same<T, float>::value;
+    using std::integral_constant;
     if (in_tail<T>(lvl))
       RCHK(tail_push(TL_RESTRICT, lvl, !v_cycle));
     else if (many_threads(l.n))
-      RCHK(restricted(std::integral_constant<int, MANY_NT>(), std::integral_constant<int, 1>()));
+      RCHK(restricted(integral_constant<int, MANY_NT>(), integral_constant<int, 1>(), std::true_type()));
+    else if constexpr (parents)
+      RCHK(restricted(integral_constant<int, BS>(), integral_constant<int, 1>(), std::false_type()));
     else
-      RCHK(with_bb(KC_RESTRICT, [&](auto B) { return restricted(std::integral_constant<int, restrict_nt<T>()>(), B); }));
+      RCHK(with_bb(KC_RESTRICT, [&](auto B) {
+        return restricted(integral_constant<int, MANY_NT>(), B, std::true_type());
+      }));
     if constexpr (D == 2 && NC == 8) {
       // The ghost fill and the rhs in one launch on levels whose launches
       // are bound by their chains: 832 boxes 4.2 us (apart 3.1 + 3.3), 6144

@@ -1721,12 +1721,17 @@ __global__ void __launch_bounds__(BS * BB) k_mp_residual_lds(const int *__restri
 // also kept in the child's tmp (set_coarse_phi_rhs, :742-776).
 // The child box is staged in LDS with its face ghosts: formed in-kernel, or
 // (stored) the stored layer, which the FP64 form fills beforehand as the
-// reference does.  Every thread forms the residuals of its own cells, which
-// then take phi's place in LDS for the restriction, so no thread is idle in
-// the larger part: 21 M cells of 8^2 boxes 66 us (104 with the residuals of
-// one parent cell in one thread), 4096 FP32 8^3 boxes 12.7 (16.6), 64 FP64
-// 16^3 boxes 6.2 (7.9), 768 22.0 (23.9), 1536 FP32 16^3 boxes 20.0 (19.3).
-template <int D, int NC, int BS, typename T, int BB = 1>
+// reference does.
+// OWN: every thread forms the residuals of its own cells, which then take
+// phi's place in LDS for the restriction, so no thread is idle in the larger
+// part: 21 M cells of 8^2 boxes 66 us (104 without), 4096 FP32 8^3 boxes 12.7
+// (16.6), 64 FP64 16^3 boxes 6.2 (7.9), 768 22.0 (23.9).
+// Without OWN (3D) a thread forms the residuals of the eight children of its
+// parent cells and sums them in registers.  Nothing is held over a barrier,
+// so a box of 16^3 needs 256 threads and a CU runs six at once, where OWN
+// takes 512 threads for its residuals and runs four: FP32 levels of 512 boxes
+// 7.1 us (OWN 7.9), 768 10.0 (12.1), 1536 19.2 (19.9), 2816 29.4 (32.9).
+template <int D, int NC, int BS, typename T, int BB = 1, bool OWN = true>
 __global__ void __launch_bounds__(BS * BB, (BS >= 512 ? 4 : 1)) k_restrict_residual(const int *__restrict__ ids,
                                                                const DBox *__restrict__ boxes, const T *child, T *phi,
                                                                const T *__restrict__ rhs, T *tmp, T lambda2, int cyl,
@@ -1747,49 +1752,71 @@ __global__ void __launch_bounds__(BS * BB, (BS >= 512 ? 4 : 1)) k_restrict_resid
     const size_t cb = (size_t)(id - 1) * L::STRIDE, pb = (size_t)(bc.parent - 1) * L::STRIDE;
     Stage<D, NC, BS, T, BB, false> sg;
     sg.issue(bc, id, child, m, 0, (const T *)phi, stored != 0);
-    T rr[NI];
+    T rr[OWN ? NI : 1];
+    if constexpr (OWN) {
 #pragma unroll
-    for (int t = 0; t < NI; t++) {
-      int i, j, k;
-      rr[t] = rhs[cb + sg.cell(ltid<BS>() + t * BS, i, j, k)];
+      for (int t = 0; t < NI; t++) {
+        int i, j, k;
+        rr[t] = rhs[cb + sg.cell(ltid<BS>() + t * BS, i, j, k)];
+      }
     }
     const Sten<D, T> st = lpl_stencil<D, T>(bc, lambda2);
     sg.commit(s, cp, bc, m);
-    // the residuals of the thread's cells and its parent cells' phi
-#pragma unroll
-    for (int t = 0; t < NI; t++) {
-      int i, j, k;
-      const int pos = sg.cell(ltid<BS>() + t * BS, i, j, k);
-      rr[t] = rr[t] - apply_cell<D, NC, T>(s, st, cyl != 0, bc, i, j, k);
-      if (store_residual) tmp[cb + pos] = rr[t];
-    }
-    T ps[NQT];
-#pragma unroll
-    for (int t = 0; t < NQT; t++) {
-      const int q = ltid<BS>() + t * BS;
-      const int i = q % H + 1, j = (q / H) % H + 1, k = (D == 3) ? q / (H * H) + 1 : 0;
-      if (NQ % BS == 0 || q < NQ)
-        ps[t] = restrict_cell<D, NC, T>(s, 2 * i - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0, false, bp, 0);
-    }
-    gsync<BS, BB>();
-#pragma unroll
-    for (int t = 0; t < NI; t++) {
-      int i, j, k;
-      sg.cell(ltid<BS>() + t * BS, i, j, k);
-      s[G::idx(i, j, k)] = rr[t];
-    }
-    gsync<BS, BB>();
     int off[3] = {0, 0, 0};
     for (int d = 0; d < D; d++) off[d] = ((bc.ix[d] - 1) & 1) * H;
+    if constexpr (OWN) {
+      // the residuals of the thread's cells and its parent cells' phi
 #pragma unroll
-    for (int t = 0; t < NQT; t++) {
-      const int q = ltid<BS>() + t * BS;
-      if (NQ % BS && q >= NQ) continue;
-      const int i = q % H + 1, j = (q / H) % H + 1, k = (D == 3) ? q / (H * H) + 1 : 0;
-      const int ic = off[0] + i, jc = off[1] + j, kc = (D == 3) ? off[2] + k : 0;
-      tmp[pb + L::in_at(ic, jc, kc)] =
-          restrict_cell<D, NC, T>(s, 2 * i - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0, cyl != 0, bp, ic);
-      phi[pb + L::in_at(ic, jc, kc)] = ps[t];
+      for (int t = 0; t < NI; t++) {
+        int i, j, k;
+        const int pos = sg.cell(ltid<BS>() + t * BS, i, j, k);
+        rr[t] = rr[t] - apply_cell<D, NC, T>(s, st, cyl != 0, bc, i, j, k);
+        if (store_residual) tmp[cb + pos] = rr[t];
+      }
+      T ps[NQT];
+#pragma unroll
+      for (int t = 0; t < NQT; t++) {
+        const int q = ltid<BS>() + t * BS;
+        const int i = q % H + 1, j = (q / H) % H + 1, k = (D == 3) ? q / (H * H) + 1 : 0;
+        if (NQ % BS == 0 || q < NQ)
+          ps[t] = restrict_cell<D, NC, T>(s, 2 * i - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0, false, bp, 0);
+      }
+      gsync<BS, BB>();
+#pragma unroll
+      for (int t = 0; t < NI; t++) {
+        int i, j, k;
+        sg.cell(ltid<BS>() + t * BS, i, j, k);
+        s[G::idx(i, j, k)] = rr[t];
+      }
+      gsync<BS, BB>();
+#pragma unroll
+      for (int t = 0; t < NQT; t++) {
+        const int q = ltid<BS>() + t * BS;
+        if (NQ % BS && q >= NQ) continue;
+        const int i = q % H + 1, j = (q / H) % H + 1, k = (D == 3) ? q / (H * H) + 1 : 0;
+        const int ic = off[0] + i, jc = off[1] + j, kc = (D == 3) ? off[2] + k : 0;
+        tmp[pb + L::in_at(ic, jc, kc)] =
+            restrict_cell<D, NC, T>(s, 2 * i - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0, cyl != 0, bp, ic);
+        phi[pb + L::in_at(ic, jc, kc)] = ps[t];
+      }
+    } else {
+      static_assert(D == 3, "restrict_cell's sum without cylindrical weights");
+      for (int q = ltid<BS>(); q < NQ; q += BS) {
+        const int i = q % H + 1, j = (q / H) % H + 1, k = q / (H * H) + 1;
+        int pos[8];
+        child_pos<D, NC, L>(2 * i - 1, 2 * j - 1, 2 * k - 1, pos);
+        T sm = 0;  // in restrict_cell's order
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+          const T rv = rhs[cb + pos[c]] - apply_cell<D, NC, T>(s, st, cyl != 0, bc, 2 * i - 1 + (c & 1),
+                                                               2 * j - 1 + ((c >> 1) & 1), 2 * k - 1 + (c >> 2));
+          if (store_residual) tmp[cb + pos[c]] = rv;
+          sm = c ? sm + rv : rv;
+        }
+        const int to = L::in_at(off[0] + i, off[1] + j, off[2] + k);
+        tmp[pb + to] = T(0.125) * sm;
+        phi[pb + to] = restrict_cell<D, NC, T>(s, 2 * i - 1, 2 * j - 1, 2 * k - 1, false, bp, 0);
+      }
     }
     gsync<BS, BB>();  // (the group's LDS is reused by its next item)
   }

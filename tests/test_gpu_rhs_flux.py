@@ -1,6 +1,7 @@
 """The ghost fill and coarse rhs in one launch (k_gc_rhs, smaller 2D levels)
-against the two launches of large levels, and k_flux's two homes of the
-transport table: the same bits."""
+against the two launches of large levels, the two forms of the residual
+restriction of FP32 16^3 boxes, and k_flux's two homes of the transport table:
+the same bits."""
 import numpy as np
 import pytest
 
@@ -33,6 +34,30 @@ def test_copies_of_a_run_in_small_and_large_forests(S, A, mixed):
         for a, b in zip(got[0], info):
             assert list(a) == [b[0]] * n
         assert np.array_equal(got[1], np.broadcast_to(want[0], got[1].shape))
+
+
+def test_restriction_of_small_and_large_3d_levels(S, A):
+    """FP32 levels of 16^3 boxes are restricted a cell per thread up to one
+    box per CU and a parent cell per thread above: 2, 10 and 11 copies of a
+    run with 24 boxes and refinement boundaries on level 3 lie on either side
+    of that line (256 boxes)."""
+    one = S.small_amr(3, nc=16, uniform_lvl=2, max_lvl=3, frac=0.4, seed=37)
+    one.params.mg_num_vcycles = 12
+    one.params.mg_max_rel_residual = 1e-8
+    assert list(np.bincount(one.extra["export"]["lvl"])) == [0, 1, 8, 24]
+    out = []
+    for n in (2, 10, 11):
+        t, ne0, offs = S.merge_forest([one] * n)
+        p = A.Path("gpu", 3, 16, A.XYZ, A.PREC_MIXED)
+        S.apply_ensemble(p, S.Ensemble([one] * n, t, ne0, offs, np.full(n, one.voltage), name="copies"))
+        info = [list(x) for x in p.field_compute_runs(0, have_guess=False)]
+        out.append((info, p.get_cc(A.CC_PHI).reshape(n, -1)))
+        p.close()
+    want = out[0][1][0]
+    for info, phi in out:
+        for a, b in zip(info, out[0][0]):
+            assert list(a) == [b[0]] * len(phi)
+        assert np.array_equal(phi, np.broadcast_to(want, phi.shape))
 
 
 @pytest.mark.parametrize("ndim,nc", [(2, 8), (2, 16), (3, 8), (3, 16)])
