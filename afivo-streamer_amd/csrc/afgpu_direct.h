@@ -471,9 +471,11 @@ __global__ void __launch_bounds__((LcGeo<N, FOLD>::BT), 4) k_lc_x(const double *
 // The transforms along y and z: DIR 1 forward (Mf), 2 backward (Mb), 3 the
 // last axis: forward, division by the eigenvalue sums and backward.  A
 // workgroup takes C neighbouring columns x at one value o of the remaining
-// coordinate (z for the y axis, y for the z axis; the run in 2D).
+// coordinate (z for the y axis, y for the z axis; the run in 2D).  The last
+// axis is done in place (in == out): a workgroup reads and writes the same
+// lines, all of them into LDS before a barrier and none stored before it.
 template <int D, int N, int DIR, bool FOLD>
-__global__ void __launch_bounds__((LcGeo<N, FOLD>::BT), 4) k_lc_line(const double *__restrict__ in, double *__restrict__ out,
+__global__ void __launch_bounds__((LcGeo<N, FOLD>::BT), 4) k_lc_line(const double *in, double *out,
                                                  const double *__restrict__ Mf, const double *__restrict__ Mb, int axis,
                                                  const double *__restrict__ eig, double lambda2) {
   using LG = LcGeo<N, FOLD>;
