@@ -237,34 +237,35 @@ def test_mixed_direct_solve_128_matrix_cores(A, S):
         assert e < 1e-11
 
 
-def test_mixed_direct_solve_fused_passes_bit_for_bit(A, S):
-    """The uniform-level solve with the gather and scatter folded into the
-    x transforms and the last axis's forward transform, division and
-    backward transform as one pass gives the same bits as the separate
-    passes: 3D with photoionization (level 4 = 128^3), a few full steps.
-    (The fused pass exists in FP64 only: both runs transform in FP64.)"""
+def test_mixed_direct_solve_fuse_option_keeps_fp64(A, S):
+    """AFGPU_OPT_FUSE_DIRECT 1 keeps the uniform-level solve in FP64 whatever
+    AFGPU_OPT_DIRECT_F32 says, and chooses nothing else: the bits of the FP64
+    transforms with it, other bits without it.  3D with photoionization (level
+    4 = 128^3), a few full steps."""
     case = setup(S.small_amr(3, nc=16, uniform_lvl=4, max_lvl=5, frac=0.03, seed=4), photoi=True)
     runs = []
-    for fuse in (1, 0):
+    for fuse, f32 in ((0, 0), (1, 0), (1, 1), (0, 1)):
         m = S.apply(A.Path("gpu", case.D, case.nc, case.coord, A.PREC_MIXED), case)
-        m.set_option(A.OPT_DIRECT_F32, 0)
-        m.set_option(A.OPT_DIRECT_FOLD, 0)  # (the fused pass transforms unsplit)
+        m.set_option(A.OPT_DIRECT_F32, f32)
         m.set_option(A.OPT_FUSE_DIRECT, fuse)
         infos = [m.field_compute(0, False)] + [m.step() for _ in range(3)]
         runs.append((infos, [m.get_cc(iv) for iv in (A.CC_PHI, A.CC_ELECTRON, A.CC_PHOTO)]))
-    assert runs[0][0] == runs[1][0]
-    for a, b in zip(runs[0][1], runs[1][1]):
-        assert np.array_equal(a, b)
+        m.close()
+    for r in runs[1:3]:
+        assert r[0] == runs[0][0]
+        for a, b in zip(r[1], runs[0][1]):
+            assert np.array_equal(a, b)
+    assert not np.array_equal(runs[3][1][0], runs[0][1][0])
 
 
 def test_split_half_sweeps_bit_for_bit(A, S):
     """The inner cycle's half-sweeps staging only the other colour's block
     and the rhs (k_gsrb_split, the default for 3D 16^3 boxes) give the same
-    bits as the half-sweeps staging the whole box in LDS (k_gsrb_lds).
-    They run on levels of at least 256 boxes: the channel tree's level 5
-    (1536 boxes, refinement boundaries and the domain's faces), and a
-    uniform level 4 (512 boxes) smoothed above a 64^3 direct solve; Poisson
-    and the photoionization modes (Helmholtz) over a few steps."""
+    bits as the half-sweeps staging the whole box in LDS (k_gsrb_lds), on
+    every level above the direct solve: the channel tree's level 5 (1536
+    boxes, refinement boundaries and the domain's faces), and a uniform
+    level 4 (512 boxes) smoothed above a 64^3 direct solve; Poisson and the
+    photoionization modes (Helmholtz) over a few steps."""
     cases = ((setup(S.config1(photoi=True), photoi=True), {}),
              (setup(S.small_amr(3, nc=16, uniform_lvl=4, max_lvl=5, frac=0.05, seed=6), photoi=True),
               {A.OPT_DIRECT_N: 64}))
@@ -286,15 +287,17 @@ def test_split_half_sweeps_bit_for_bit(A, S):
 
 def test_split2d_half_sweeps_bit_for_bit(A, S):
     """The 2D half-sweep of 8^2 boxes that stages everything by DMA
-    (k_gsrb_split2d, the default on levels of at least 256 boxes) gives the
+    (k_gsrb_split2d, the default on levels of at least 7168 boxes) gives the
     same bits as the generic box-staging half-sweep (k_gsrb_lds): a
-    cylindrical and a Cartesian tree refined past a uniform level 5 (256
-    boxes), so that refinement boundaries, the axis and the domain's faces
-    all border levels of several hundred boxes; Poisson and the
-    photoionization modes over a few steps; and a forest of runs of
-    different depths (runs masked out as they converge)."""
-    cases = [setup(S.small_amr(2, coord=A.CYL, uniform_lvl=5, max_lvl=7, frac=0.3, seed=17), photoi=True),
-             setup(S.small_amr(2, coord=A.XYZ, uniform_lvl=5, max_lvl=7, frac=0.3, seed=19), photoi=True)]
+    cylindrical and a Cartesian tree refined past a uniform level 7, so that
+    refinement boundaries, the axis and the domain's faces all border levels
+    of that size; Poisson and the photoionization modes over a few steps; and
+    a forest of runs of different depths (runs masked out as they
+    converge)."""
+    cases = [setup(S.small_amr(2, coord=A.CYL, uniform_lvl=7, max_lvl=9, frac=0.5, seed=17), photoi=True),
+             setup(S.small_amr(2, coord=A.XYZ, uniform_lvl=7, max_lvl=9, frac=0.5, seed=19), photoi=True)]
+    for case in cases:
+        assert np.bincount(case.extra["export"]["lvl"])[8:].min() >= 7168
     for case in cases:
         runs = []
         for box_lds in (0, 1):
@@ -307,14 +310,15 @@ def test_split2d_half_sweeps_bit_for_bit(A, S):
         assert runs[0][0] == runs[1][0], case.name
         for a, b in zip(runs[0][1], runs[1][1]):
             assert np.array_equal(a, b), case.name
-    ens = S.ensemble(level_list=[5, 6, 5, 6], num_vcycles=20, rel_residual=1e-8)
+    ens = S.ensemble(level_list=[8, 5, 7, 8], num_vcycles=20, rel_residual=1e-8, photoi=True)
+    assert np.bincount(ens.export["lvl"])[7:].min() >= 7168
     out = []
     for box_lds in (0, 1):
         g = S.apply_ensemble(A.Path("gpu", 2, 8, A.CYL, A.PREC_MIXED), ens)
         g.set_option(A.OPT_BOX_LDS, box_lds)
         g.field_compute_runs(0, have_guess=False)
         infos = [g.step_ensemble() for _ in range(2)]
-        out.append((infos, [g.get_cc(iv) for iv in (A.CC_PHI, A.CC_ELECTRON)]))
+        out.append((infos, [g.get_cc(iv) for iv in (A.CC_PHI, A.CC_ELECTRON, A.CC_PHOTO)]))
         g.close()
     assert out[0][0] == out[1][0]
     for a, b in zip(out[0][1], out[1][1]):
