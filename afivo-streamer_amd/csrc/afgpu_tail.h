@@ -49,9 +49,10 @@ constexpr int TAIL_MAX_OPS = 240;
 constexpr int TAIL_NT = 1024;
 // Levels held: 4096 cells on the finest one (two cells of a colour per
 // thread): 85 boxes of 8^2, 21 of 16^2, 9 of 8^3 or one of 16^3.  phi of all
-// of them and rhs and tmp of the levels below the finest are in LDS (49 to
-// 108 KB); rhs and tmp of the finest, which a cycle touches a few times only,
-// stay in memory.
+// of them and rhs and tmp of the levels below the finest are in LDS (99, 78,
+// 86 and 46 KB, with the tables and the level-1 matrices 120, 100, 111 and
+// 98); rhs and tmp of the finest, which a cycle touches a few times only, stay
+// in memory.
 template <int D, int NC>
 struct TailGeo {
   static constexpr int LT = (D == 2) ? (NC == 8 ? 4 : 3) : (NC == 8 ? 2 : 1);
@@ -69,6 +70,15 @@ struct TailGeo {
   static constexpr int NX = (D == 3 ? 12 * NC : 0) + (1 << D);
   static constexpr int N_GH = SLOTS * 2 * NGB, N_CR = SLOTS * NX;
   static constexpr int COLS = NC * ((1 << LT) - 1);  // cell columns along x of all levels
+  // k_tail's LDS arrays
+  static constexpr int N_PHI = SLOTS * Geo<D, NC>::NCELL;
+  static constexpr int N_LOW = LOW ? LOW * Geo<D, NC>::NCELL : 2;  // (2: a word that nothing reads)
+  static constexpr int N_MAT = 2 * D * NC * (NC + 1);
+  static constexpr int N_CYL = D == 2 ? COLS : 1;
+  static constexpr int N_F64 =
+      N_PHI + 2 * N_LOW + Geo<D, NC>::NINT + N_MAT + D * NC + LT * (8 + 4 * D) + N_CYL * 5;
+  static constexpr int LDS = 8 * N_F64 + 4 * (N_GH + N_CR + 2 * SLOTS);
+  static_assert(LDS <= 160 * 1024, "the LDS of a CU");
 };
 // A face ghost: bits 0-13 its cell, 14-27 the cell it is formed from (the
 // neighbour's, or the box's first one; the second one lies as far again),
@@ -148,20 +158,18 @@ __global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs A) {
   using G = Geo<D, NC>;
   using TG = TailGeo<D, NC>;
   constexpr int HALF = G::NINT / 2, NCELL = G::NCELL;
-  constexpr int H = NC / 2, NQ = G::NINT >> D, NCH = 1 << D, NMAT = 2 * D * NC * (NC + 1);
+  constexpr int H = NC / 2, NQ = G::NINT >> D, NCH = 1 << D, NMAT = TG::N_MAT;
   constexpr int TOP = 1 << (D * (TG::LT - 1));  // boxes of the finest level
   constexpr int PER = (TOP * HALF + TAIL_NT - 1) / TAIL_NT;
   constexpr int NGB = TG::NGB, NX = TG::NX;
   constexpr int GPER = (TOP * NGB + TAIL_NT - 1) / TAIL_NT;
-  __shared__ __align__(16) double s_phi[TG::SLOTS * NCELL];
-  __shared__ __align__(16) double s_rhs[(TG::LOW ? TG::LOW : 1) * NCELL];
-  __shared__ __align__(16) double s_tmp[(TG::LOW ? TG::LOW : 1) * NCELL];
+  __shared__ __align__(16) double s_phi[TG::N_PHI];
+  __shared__ __align__(16) double s_rhs[TG::N_LOW], s_tmp[TG::N_LOW];
   __shared__ double s_buf[G::NINT];            // level-1 solve
   __shared__ double s_mat[NMAT + D * NC];      // its matrices, padded rows, and eigenvalues
-  __shared__ double s_dr[TG::LT][3];           // spacing of the levels
-  __shared__ double s_st[TG::LT][8];           // their stencils, and 1 / the diagonal
+  __shared__ double s_st[TG::LT][8];           // the levels' stencils, and 1 / the diagonal
   __shared__ double s_bc[TG::LT][2 * D][2];    // phys_coeffs of their faces
-  __shared__ double s_cyl[D == 2 ? TG::COLS : 1][5];  // per column: c1, c2, c3, 1 / c1, restriction weight
+  __shared__ double s_cyl[TG::N_CYL][5];       // per column: c1, c2, c3, 1 / c1, restriction weight
   __shared__ unsigned s_gh[TG::N_GH], s_cr[TG::N_CR];
   __shared__ int s_id[TG::SLOTS];
   __shared__ int s_par[TG::SLOTS];
@@ -191,7 +199,6 @@ __global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs A) {
     const Sten<D, double> st = lpl_stencil<D, double>(bx, A.lambda2);
     for (int q = 0; q <= 2 * D; q++) s_st[tid][q] = st.c[q];
     s_st[tid][7] = 1.0 / st.c[0];
-    for (int d = 0; d < D; d++) s_dr[tid][d] = bx.dr[d];
     for (int nb = 0; nb < 2 * D; nb++) phys_coeffs<D, double>(bx.dr, A.m, run_val, nb, s_bc[tid][nb][0], s_bc[tid][nb][1]);
   }
   if (D == 2 && cyl) {
@@ -214,7 +221,7 @@ __global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs A) {
     const int s = q / NV, x = q - s * NV;
     const size_t base = (size_t)(map[s] - 1) * NCELL;
     reinterpret_cast<d2 *>(s_phi)[q] = reinterpret_cast<const d2 *>(A.phi + base)[x];
-    if (s < n_low) {
+    if (TG::LOW && s < n_low) {
       reinterpret_cast<d2 *>(s_rhs)[q] = reinterpret_cast<const d2 *>(A.rhs + base)[x];
       reinterpret_cast<d2 *>(s_tmp)[q] = reinterpret_cast<const d2 *>(A.tmp + base)[x];
     }
@@ -222,8 +229,12 @@ __global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs A) {
   const double lambda2 = A.lambda2;
   // box position p of a level: its coordinate along d
   auto coord = [](int p, int lvl, int d) { return (p >> (d * (lvl - 1))) & ((1 << (lvl - 1)) - 1); };
-  auto rhs_of = [&](int slot) { return slot < TG::LOW ? s_rhs + slot * NCELL : A.rhs + (size_t)(s_id[slot] - 1) * NCELL; };
-  auto tmp_of = [&](int slot) { return slot < TG::LOW ? s_tmp + slot * NCELL : A.tmp + (size_t)(s_id[slot] - 1) * NCELL; };
+  auto rhs_of = [&](int slot) {
+    return TG::LOW && slot < TG::LOW ? s_rhs + slot * NCELL : A.rhs + (size_t)(s_id[slot] - 1) * NCELL;
+  };
+  auto tmp_of = [&](int slot) {
+    return TG::LOW && slot < TG::LOW ? s_tmp + slot * NCELL : A.tmp + (size_t)(s_id[slot] - 1) * NCELL;
+  };
   __syncthreads();
 
   // Edges (3D) and corners of a level's boxes, the faces being filled: the
@@ -372,45 +383,46 @@ __global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs A) {
         if (op.a) corners(o, n_box);
         break;
       }
-      case TL_RESTRICT: {
-        const int po = level_off(lvl - 1);
-        for (int q = tid; q < n_box * NQ; q += TAIL_NT) {
-          const int p = q / NQ, r = q % NQ;
-          int pp = 0, off[3] = {0, 0, 0};
+      case TL_RESTRICT:
+        if constexpr (TG::LT > 1) {
+          const int po = level_off(lvl - 1);
+          for (int q = tid; q < n_box * NQ; q += TAIL_NT) {
+            const int p = q / NQ, r = q % NQ;
+            int pp = 0, off[3] = {0, 0, 0};
 #pragma unroll
-          for (int d = 0; d < D; d++) {
-            const int c = coord(p, lvl, d);
-            pp += (c >> 1) << (d * (lvl - 2));
-            off[d] = (c & 1) * H;
-          }
-          const double *u = s_phi + (o + p) * NCELL, *rc = rhs_of(o + p);
-          double *tc = tmp_of(o + p);
-          const int i = r % H + 1, j = (r / H) % H + 1, k = (D == 3) ? r / (H * H) + 1 : 0;
-          const int x0 = G::idx(2 * i - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0), c0 = col(p) + 2 * i - 2;
-          // the children's residuals and values, in af_restrict_box's order
-          double rs[4], sm = 0, sp = 0;
+            for (int d = 0; d < D; d++) {
+              const int c = coord(p, lvl, d);
+              pp += (c >> 1) << (d * (lvl - 2));
+              off[d] = (c & 1) * H;
+            }
+            const double *u = s_phi + (o + p) * NCELL, *rc = rhs_of(o + p);
+            double *tc = tmp_of(o + p);
+            const int i = r % H + 1, j = (r / H) % H + 1, k = (D == 3) ? r / (H * H) + 1 : 0;
+            const int x0 = G::idx(2 * i - 1, 2 * j - 1, (D == 3) ? 2 * k - 1 : 0), c0 = col(p) + 2 * i - 2;
+            // the children's residuals and values, in af_restrict_box's order
+            double rs[4], sm = 0, sp = 0;
 #pragma unroll
-          for (int c = 0; c < NCH; c++) {
-            const int x = x0 + (c & 1) + ((c >> 1) & 1) * G::NG + ((c >> 2) & 1) * G::NG * G::NG;
-            const double rv = rc[x] - apply(u, x, st, c0 + (c & 1));
-            if (op.a) tc[x] = rv;
-            if (D == 2) rs[c & 3] = rv;
-            sm = c ? sm + rv : rv;
-            sp = c ? sp + u[x] : u[x];
+            for (int c = 0; c < NCH; c++) {
+              const int x = x0 + (c & 1) + ((c >> 1) & 1) * G::NG + ((c >> 2) & 1) * G::NG * G::NG;
+              const double rv = rc[x] - apply(u, x, st, c0 + (c & 1));
+              if (op.a) tc[x] = rv;
+              if (D == 2) rs[c & 3] = rv;
+              sm = c ? sm + rv : rv;
+              sp = c ? sp + u[x] : u[x];
+            }
+            const int ic = off[0] + i, y = G::idx(ic, off[1] + j, (D == 3) ? off[2] + k : 0);
+            if (D == 2 && cyl) {
+              // (the parent's column)
+              const double tw = s_cyl[NC * ((1 << (lvl - 2)) - 1) + NC * coord(pp, lvl - 1, 0) + ic - 1][4];
+              const double w1 = 1.0 - tw, w2 = 1.0 + tw;
+              sm = w1 * (rs[0] + rs[2]) + w2 * (rs[1] + rs[3]);
+            }
+            tmp_of(po + pp)[y] = (1.0 / NCH) * sm;
+            s_phi[(po + pp) * NCELL + y] = (1.0 / NCH) * sp;
           }
-          const int ic = off[0] + i, y = G::idx(ic, off[1] + j, (D == 3) ? off[2] + k : 0);
-          if (D == 2 && cyl) {
-            // (the parent's column)
-            const double tw = s_cyl[NC * ((1 << (lvl - 2)) - 1) + NC * coord(pp, lvl - 1, 0) + ic - 1][4];
-            const double w1 = 1.0 - tw, w2 = 1.0 + tw;
-            sm = w1 * (rs[0] + rs[2]) + w2 * (rs[1] + rs[3]);
-          }
-          tmp_of(po + pp)[y] = (1.0 / NCH) * sm;
-          s_phi[(po + pp) * NCELL + y] = (1.0 / NCH) * sp;
+          __syncthreads();
         }
-        __syncthreads();
         break;
-      }
       case TL_RHS: {
         for (int q = tid; q < n_box * NCELL; q += TAIL_NT) {
           const int p = q / NCELL, x = q % NCELL;
@@ -460,26 +472,27 @@ __global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs A) {
         __syncthreads();
         break;
       }
-      case TL_PROLONG: {
-        const int po = level_off(lvl - 1);
-        for (int q = tid; q < n_box * G::NINT; q += TAIL_NT) {
-          const int p = q / G::NINT;
-          int i, j, k;
-          interior_ijk<D, NC>(q % G::NINT, i, j, k);
-          int pp = 0, off[3] = {0, 0, 0};
+      case TL_PROLONG:
+        if constexpr (TG::LT > 1) {
+          const int po = level_off(lvl - 1);
+          for (int q = tid; q < n_box * G::NINT; q += TAIL_NT) {
+            const int p = q / G::NINT;
+            int i, j, k;
+            interior_ijk<D, NC>(q % G::NINT, i, j, k);
+            int pp = 0, off[3] = {0, 0, 0};
 #pragma unroll
-          for (int d = 0; d < D; d++) {
-            const int c = coord(p, lvl, d);
-            pp += (c >> 1) << (d * (lvl - 2));
-            off[d] = (c & 1) * H;
+            for (int d = 0; d < D; d++) {
+              const int c = coord(p, lvl, d);
+              pp += (c >> 1) << (d * (lvl - 2));
+              off[d] = (c & 1) * H;
+            }
+            double &u = s_phi[(o + p) * NCELL + G::idx(i, j, k)];
+            // (level - 1 is below the finest held: its tmp is in LDS)
+            u = prolong_value<D, NC, double>(u, s_tmp + (po + pp) * NCELL, off, i, j, k);
           }
-          double &u = s_phi[(o + p) * NCELL + G::idx(i, j, k)];
-          // (level - 1 is below the finest held: its tmp is in LDS)
-          u = prolong_value<D, NC, double>(u, s_tmp + (po + pp) * NCELL, off, i, j, k);
+          __syncthreads();
         }
-        __syncthreads();
         break;
-      }
       case TL_RESID: {
         double mx = 0;
         for (int q = tid; q < n_box * G::NINT; q += TAIL_NT) {
@@ -508,7 +521,7 @@ __global__ void __launch_bounds__(TAIL_NT) k_tail(TailArgs A) {
     const int s = q / NV, x = q - s * NV;
     const size_t base = (size_t)(s_id[s] - 1) * NCELL;
     reinterpret_cast<d2 *>(A.phi + base)[x] = reinterpret_cast<const d2 *>(s_phi)[q];
-    if (s < n_low) {
+    if (TG::LOW && s < n_low) {
       reinterpret_cast<d2 *>(A.rhs + base)[x] = reinterpret_cast<const d2 *>(s_rhs)[q];
       reinterpret_cast<d2 *>(A.tmp + base)[x] = reinterpret_cast<const d2 *>(s_tmp)[q];
     }
