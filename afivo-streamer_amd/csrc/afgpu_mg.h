@@ -818,11 +818,10 @@ __global__ void __launch_bounds__(BS * BB) k_mp_residual(const int *__restrict__
 }
 
 // ---- LDS-staged forms (one workgroup per box) ---------------------------------
-// The box interior is loaded once, coalesced, into LDS; the face ghosts that
-// the pass needs are formed by ghost_value() into the LDS ghost layer (all
-// threads of an iteration on the same face, so without divergence); the
-// stencil then reads LDS only.  Same arithmetic, in the same order, as the
-// direct kernels above.
+// The box interior is loaded once, coalesced, into LDS with the face ghosts
+// that the pass needs (Stage: copied from the neighbours, or formed by
+// staged_ghost, ghost_value's operations); the stencil then reads LDS only.
+// k_smooth_block forms its ghosts by ghost_value itself.
 
 template <int D, int NC, int BS, typename T, int BB = 1>
 __device__ inline void lds_load_interior(T *s, const T *u) {

@@ -580,7 +580,7 @@ def main():
     ap.add_argument("--direct-f32", type=int, default=0,
                     help="mixed precision: uniform-level solve of the FP32 inner cycle in FP32 (1) or FP64 (0)")
     ap.add_argument("--fuse-direct", type=int, default=0,
-                    help="mixed precision: uniform-level solve with the fused transform passes (1) or separate (0)")
+                    help="mixed precision: 1 keeps the uniform-level solve in FP64 whatever --direct-f32 says")
     ap.add_argument("--photoi-vcycle", type=int, default=0,
                     help="mixed precision: photoionization inner cycle V-cycle (1) or FMG (0)")
     ap.add_argument("--copy-probe", type=int, default=0, metavar="MIB",

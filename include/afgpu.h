@@ -381,7 +381,10 @@ long long afgpu_num_leaf_cells(afgpu_t *h);
  * (0 = GSRB half-sweep, 1 = flux, 2 = density update) is bracketed by HIP
  * events on the library's stream.  Reports the summed duration (ms), the
  * launch count and the algorithmic bytes (interior words moved) of those
- * launches since the last reset. */
+ * launches since the last reset.  While it is enabled the sequences run
+ * launch by launch, without graphs, and the coarse levels of the FP64 cycles
+ * run as level kernels, which otherwise are one kernel of their own: the
+ * times are those of the kernels counted, not shares of an untimed step. */
 int afgpu_kernel_timing(afgpu_t *h, int enable);
 int afgpu_kernel_stats(afgpu_t *h, int kind, int reset, double *total_ms,
                        long long *launches, double *algo_bytes);
@@ -399,8 +402,8 @@ int afgpu_kernel_stats(afgpu_t *h, int kind, int reset, double *total_ms,
                                     same-level neighbours' values held (default 0) */
 #define AFGPU_OPT_BATCH_MODES 5 /* mixed precision: the photoionization modes' cycles run as
                                    parallel branches of one captured graph (default 1) */
-#define AFGPU_OPT_DIRECT_MFMA 6 /* mixed precision: uniform-level transforms (64 or 128 cells
-                                   per axis) on the FP64 matrix cores (1) or as vector FMA
+#define AFGPU_OPT_DIRECT_MFMA 6 /* mixed precision: uniform-level transforms (32, 64 or 128
+                                   cells per axis) on the FP64 matrix cores (1) or as vector FMA
                                    tiles (0) (default 1) */
 #define AFGPU_OPT_PHOTOI_VCYCLE 7 /* mixed precision: the photoionization modes' inner cycle is
                                      one V-cycle (1) or one FMG cycle (0) per outer iteration
@@ -410,7 +413,12 @@ int afgpu_kernel_stats(afgpu_t *h, int kind, int reset, double *total_ms,
 #define AFGPU_OPT_STEP_GRAPH 9 /* ensembles: each step's first attempt and its field solve as one
                                   captured graph with the stopping tests on the device (1), or
                                   one captured graph per cycle with the tests on the host (0);
-                                  the results are identical (default 0, measured faster) */
+                                  the results are identical (default 0: in FP64 the host's
+                                  cycles run their coarse levels in one kernel and the graph's
+                                  do not, 2.9 ms a step against 3.6 for 13 uneven runs; in mixed
+                                  precision the graph is the faster one, 1.7 ms against 1.8 for
+                                  these, 0.23 against 0.33 for 16 runs of 64^2 cells, 4.2 against
+                                  4.3 for 16 of up to 1024^2) */
 #define AFGPU_OPT_FUSE_DIRECT 10 /* mixed precision: 1 keeps the uniform-level solve in FP64
                                     whatever AFGPU_OPT_DIRECT_F32 says; its last forward
                                     transform, division and first backward transform run as one
